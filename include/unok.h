@@ -45,6 +45,20 @@ int unok_gemm_nt(int in_dtype, int out_dtype, int M, int N, int K,
                  void* C, int64_t ldc, const void* R, int64_t ldr,
                  const uint8_t* gate, float alpha, void* stream);
 
+/* unok_gemm_nt with a workspace (16-byte aligned; null: none) for the fp32 partial sums of products
+ * whose K the library splits into ranges (few rows, too few output tiles for the chip), ranges x M x N
+ * floats; a second kernel adds the partials in range order, so a result does not depend on timing.
+ * plan 0: the library's choice of tile and ranges, as unok_gemm_nt_plan returns it for the sizes:
+ * tile + 16 * ranges with tile 1: 256x256, 2: 128x256, 3: 128x128, 4: 64 rows x all columns, 5: 256x256
+ * with 64-bit addresses (0: the register-staged kernel, no ranges); otherwise that plan. */
+int unok_gemm_nt_plan(int in_dtype, int M, int N, int K, int K2, int nseg, const int* seg_end);
+int unok_gemm_nt_ws(int in_dtype, int out_dtype, int M, int N, int K,
+                    const void* A, int64_t lda, const void* B, int64_t ldb,
+                    const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
+                    int nseg, const int* seg_end, const int* seg_col,
+                    void* C, int64_t ldc, const void* R, int64_t ldr,
+                    const uint8_t* gate, float alpha, int plan, void* workspace, int64_t ws_bytes, void* stream);
+
 /* C[M, N/2] = silu(G) (.) U of the gate/up product A[M,K] B[N,K]^T (+ A2[M,K2] B2[N,K2]^T, the
  * LoRA extension), bf16, for B (and B2) with 64-row interleaved gate/up rows (rows 128 b + [0, 64):
  * gate features 64 b + [0, 64); rows 128 b + [64, 128): the same up features); rounded exactly as
@@ -56,6 +70,10 @@ int unok_gemm_nt(int in_dtype, int out_dtype, int M, int N, int K,
 int unok_gemm_nt_swiglu(int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
                         const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
                         void* C, int64_t ldc, void* gu, int64_t ldgu, void* stream);
+/* The same for any number of rows. */
+int unok_gemm_nt_swiglu_any(int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
+                        const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
+                        void* C, int64_t ldc, void* gu, int64_t ldgu, void* stream);
 
 /* dgu[M, 2F] = SwiGLU backward of dS = A[M,K] B[F,K]^T + A2[M,K2] B2[F,K2]^T against
  * gu[M, 2F] = [gate | up] (dS is never stored); bf16, rounded exactly as unok_gemm_nt followed by
@@ -63,6 +81,10 @@ int unok_gemm_nt_swiglu(int M, int N, int K, const void* A, int64_t lda, const v
  * act_fn(gate_proj(x)) * up_proj(x) through down_proj (modeling_qwen3.py:81-82) with the LoRA
  * data-gradient extension of down_proj (peft 0.15.2 lora.Linear). */
 int unok_gemm_nt_swiglu_bwd(int M, int F, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
+                            const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
+                            const void* gu, int64_t ldgu, void* dgu, int64_t lddgu, void* stream);
+/* The same for any number of rows. */
+int unok_gemm_nt_swiglu_bwd_any(int M, int F, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
                             const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
                             const void* gu, int64_t ldgu, void* dgu, int64_t lddgu, void* stream);
 
@@ -149,6 +171,12 @@ int unok_rope_table(int P, int half, const float* inv_freq, float* cos_tab, floa
  * projections of the remote Qwen3 attention with their gated LoRA (modeling_qwen3.py:237-253,
  * training/lora.py:164-174). M and 128 (nq + 2 nk) multiples of 256, K of 64, K2 of 32. */
 int unok_gemm_nt_qkv_rope(int M, int K, int nq, int nk, const void* A, int64_t lda, const void* B,
+                          int64_t ldb, const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
+                          int nseg, const int* seg_end, const int* seg_col, const void* wq, const void* wk,
+                          const int64_t* pos, const float* cos_tab, const float* sin_tab, int P, float eps,
+                          void* q_out, void* k_out, void* v_out, float* rstd, void* qk_pre, void* stream);
+/* The same for any number of rows. */
+int unok_gemm_nt_qkv_rope_any(int M, int K, int nq, int nk, const void* A, int64_t lda, const void* B,
                           int64_t ldb, const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
                           int nseg, const int* seg_end, const int* seg_col, const void* wq, const void* wk,
                           const int64_t* pos, const float* cos_tab, const float* sin_tab, int P, float eps,

@@ -26,6 +26,9 @@ SIGNATURES: dict[str, tuple] = {
     "unok_last_error": (C.c_char_p, []),
     "unok_gemm_nt": (_i, [_i, _i, _i, _i, _i, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _i,
                           _i, _ip, _ip, _p, _i64, _p, _i64, _p, _f, _p]),
+    "unok_gemm_nt_plan": (_i, [_i, _i, _i, _i, _i, _i, _ip]),
+    "unok_gemm_nt_ws": (_i, [_i, _i, _i, _i, _i, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _i,
+                             _i, _ip, _ip, _p, _i64, _p, _i64, _p, _f, _i, _p, _i64, _p]),
     "unok_gemm_nt_swiglu": (_i, [_i, _i, _i, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _i, _p, _i64, _p, _i64, _p]),
     "unok_gemm_nt_swiglu_bwd": (_i, [_i, _i, _i, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _i, _p, _i64, _p, _i64,
                                      _p]),
@@ -77,6 +80,9 @@ SIGNATURES: dict[str, tuple] = {
     "unok_cast_copy": (_i, [_i, _i64, _i64, _f, _p, _p, _p]),
     "unok_transpose_jobs": (_i, [_i, _p, _i, _i64, _p, _p, _p]),
 }
+
+for _name in ("unok_gemm_nt_swiglu", "unok_gemm_nt_swiglu_bwd", "unok_gemm_nt_qkv_rope"):
+    SIGNATURES[_name + "_any"] = SIGNATURES[_name]
 
 _lock = threading.Lock()
 _lib = None

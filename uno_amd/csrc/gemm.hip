@@ -18,6 +18,7 @@
 #include "common.h"
 #include "lds_tile.h"
 
+#include <math.h>
 #include <stdlib.h>
 #include <type_traits>
 
@@ -30,7 +31,8 @@ struct GemmNT {
   const void* R; int64_t ldr;
   const uint8_t* gate;
   void* C2; int64_t ldc2;          // second output of the SwiGLU forward epilogue (gate | up), or null
-  int group;                       // row tiles per tile group of the 256x256 kernel (0: 8)
+  int group;                       // row tiles per tile group of the direct-to-LDS tile kernel (0: 8)
+  int splits;                      // K ranges (0 or 1: none): the product writes fp32 partials [splits][M][N] to C
   int M, N, K, K2;
   int nseg;
   int seg_end[4];
@@ -242,7 +244,9 @@ __device__ __forceinline__ void wait_tiles(int later) {
   }
 }
 
-template <int BM, int BN, int NW, int BK, int STAGES, typename OutT, bool ROT = false>
+// With SPLIT (no extension, no gate, no residual), range z of p.splits covers the main K tiles
+// [z nk1 / splits, (z + 1) nk1 / splits) and writes its fp32 sums to C + z M ldc.
+template <int BM, int BN, int NW, int BK, int STAGES, typename OutT, bool ROT = false, bool SPLIT = false>
 __global__ __launch_bounds__(NW * 64) void gemm_nt_bf16_dma_kernel(const GemmNT p) {
   constexpr int CPR = BK / 8;                     // 16-byte chunks per tile row
   constexpr int RPI = 64 / CPR;                   // tile rows per wave load instruction
@@ -259,7 +263,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_bf16_dma_kernel(const GemmNT 
 
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int nM = (p.M + BM - 1) / BM, nN = (p.N + BN - 1) / BN;
-  const int lin = xcd_remap(blockIdx.x, nM * nN);
+  int lin = xcd_remap(blockIdx.x, SPLIT ? nM * nN * p.splits : nM * nN);
+  const int split = SPLIT ? lin / (nM * nN) : 0;
+  if (SPLIT) lin %= nM * nN;
   constexpr int GROUP = 8;
   const int group = lin / (GROUP * nN);
   const int first_m = group * GROUP;
@@ -273,7 +279,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_bf16_dma_kernel(const GemmNT 
   const bf16_t* A2 = nullptr;
   if (p.A2 != nullptr && p.K2 > 0) A2 = (const bf16_t*)p.A2 + seg_col_of(p, n0);
   const bf16_t* B2 = (const bf16_t*)p.B2;
-  const int nk1 = p.K / BK;
+  const int kbeg = SPLIT ? (int)((int64_t)split * (p.K / BK) / p.splits) : 0;
+  const int nk1 = (SPLIT ? (int)((int64_t)(split + 1) * (p.K / BK) / p.splits) : p.K / BK) - kbeg;
   const int nk = nk1 + (A2 ? p.K2 / BK : 0);
 
   // Per-lane source rows (clamped) and swizzled chunk, fixed for the whole K loop.
@@ -303,7 +310,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_bf16_dma_kernel(const GemmNT 
     bf16_t* bs = Bs + buf * BN * BK;
     if (kt < nk1) {
       const int kr = kt + rot;
-      const int kk = (kr >= nk1 ? kr - nk1 : kr) * BK;
+      const int kk = (kbeg + (kr >= nk1 ? kr - nk1 : kr)) * BK;
 #pragma unroll
       for (int i = 0; i < A_INS; ++i) lds_dma16(A + a_off[i] + kk, as + (i * NW + wid) * RPI * BK);
 #pragma unroll
@@ -366,7 +373,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_bf16_dma_kernel(const GemmNT 
     compute(kt % STAGES);
   }
 
-  OutT* C = (OutT*)p.C;
+  OutT* C = (OutT*)p.C + (SPLIT ? (int64_t)split * p.M * p.ldc : 0);
   const OutT* R = (const OutT*)p.R;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
@@ -703,20 +710,28 @@ static void launch_nt_bf16(const GemmNT& p, int out_dtype, hipStream_t st) {
 static bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
 
 // ---------------------------------------------------------------------------------------
-// 256x256 bf16 NT kernel with 16x16x32 MFMAs: 4 waves of 128x128 (8 x 8 accumulators of 4 floats,
-// 256 AGPRs), BK 64, A tiles in 3 LDS stages and B tiles in 2 (160 KB), filled by direct-to-LDS
-// loads with the same swizzled layout as the 32x32x16 kernel. A tile is two 32-wide k-steps: step 0
-// reads step 1's fragments and issues the A loads of the tile two ahead, then the barrier, then
-// step 1 reads the next tile's step-0 fragments and issues that tile's B loads (one load per eight
-// MFMAs in both steps: with all 16 in one step the 64 B/clk vector-memory path saturated and
-// stalled the MFMA stream). Per 32 k and wave: 8 A + 8 B fragment reads (16 bytes per lane) and 64
-// MFMAs. With the B fragment as the first operand, lane l holds C[row 16i + l % 16][cols 16j +
-// 4 (l / 16) + 0..3] of accumulator (i, j).
+// BM x BN bf16 NT kernel with 16x16x32 MFMAs: 4 waves of BM/2 x BN/2 (at 256x256 8 x 8 accumulators
+// of 4 floats, 256 AGPRs), BK 64, A tiles in 3 LDS stages and B tiles in 2 (160 KB at 256x256),
+// filled by direct-to-LDS loads with the same swizzled layout as the 32x32x16 kernel. A tile is two
+// 32-wide k-steps: step 0 reads step 1's fragments and issues the A loads of the tile two ahead,
+// then the barrier, then step 1 reads the next tile's step-0 fragments and issues that tile's B
+// loads, spread evenly over the step's MFMAs (with all loads in one step the 64 B/clk
+// vector-memory path saturated and stalled the MFMA stream). Per 32 k and wave: BM/32 A + BN/32 B
+// fragment reads (16 bytes per lane) and BM BN / 1024 MFMAs. With the B fragment as the first
+// operand, lane l holds C[row 16i + l % 16][cols 16j + 4 (l / 16) + 0..3] of accumulator (i, j).
+//
+// 256x256 reads the fewest LDS bytes per MFMA (half the LDS rate) and serves every product with at
+// least about a tile per CU; 128x256 (three quarters) and 128x128 (all of it, two workgroups per CU)
+// serve the products that would leave CUs idle, and split-K ranges those that have too few tiles at
+// any size (nt_plan below holds the rule). With p.splits > 1, EPI 6 writes the range's fp32 sums.
 // ---------------------------------------------------------------------------------------
-template <typename OutT, int EPI = 0>
+template <typename OutT, int EPI = 0, int BM = 256, int BN = 256>
 __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p) {
-  constexpr int BM = 256, BN = 256, BK = 64, NW = 4, TM = 8, TN = 8;
-  constexpr int CPR = BK / 8, RPI = 64 / CPR, INS = BM / (RPI * NW);   // 8 loads per operand and wave
+  constexpr int BK = 64, NW = 4, WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
+  constexpr int CPR = BK / 8, RPI = 64 / CPR;
+  constexpr int AI = BM / (RPI * NW), BI = BN / (RPI * NW);   // loads per wave and tile of A and of B
+  static_assert(EPI == 0 || EPI == 6 || WN == 128, "the fused epilogues take 128 columns per wave");
+  static_assert((EPI != 3 && EPI != 4) || BM == 256, "the loss epilogues take 256-row tiles");
   extern __shared__ __attribute__((aligned(16))) bf16_t smem[];
   bf16_t* As = smem;                            // [3][BM*BK]
   bf16_t* Bs = smem + 3 * BM * BK;              // [2][BN*BK]
@@ -724,7 +739,10 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nM = (p.M + BM - 1) / BM, nN = (p.N + BN - 1) / BN;
-  const int lin = xcd_remap(blockIdx.x, nM * nN);
+  const int ntile = nM * nN;
+  int lin = xcd_remap(blockIdx.x, EPI == 6 ? ntile * p.splits : ntile);
+  const int split = EPI == 6 ? lin / ntile : 0;
+  if (EPI == 6) lin %= ntile;
   const int GROUP = p.group > 0 ? p.group : 8;
   const int group = lin / (GROUP * nN);
   const int first_m = group * GROUP;
@@ -736,8 +754,12 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
   const int nk1 = p.K / BK;
   // The LoRA extension runs in whole 64-deep tiles; K2 = 32 (mod 64) leaves the last one half full,
   // and its second 32-wide k-step then runs on zeroed fragments.
-  const int nk = nk1 + (ext ? (p.K2 + BK - 1) / BK : 0);
-  const bool half_last = ext && (p.K2 % BK) != 0;
+  const int nk_all = nk1 + (ext ? (p.K2 + BK - 1) / BK : 0);
+  // this range's K tiles [kt0, nk): the main tiles are divided among the ranges and the extension
+  // belongs to the last one, so an extension of zeros leaves every sum as it was
+  const int kt0 = EPI == 6 ? (int)((int64_t)split * nk1 / p.splits) : 0;
+  const int nk = EPI == 6 && split + 1 < p.splits ? (int)((int64_t)(split + 1) * nk1 / p.splits) : nk_all;
+  const bool half_last = ext && nk == nk_all && (p.K2 % BK) != 0;
 
   const int lrowi = lane / CPR, slot = lane % CPR;
   // Operand rows are addressed from this tile's first row, so the 32-bit buffer offsets span one
@@ -747,20 +769,23 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
                                         (uint32_t)(((int64_t)(mrows - 1) * p.lda + p.K) * 2));
   __amdgpu_buffer_rsrc_t rb = make_rsrc((const bf16_t*)p.B + (int64_t)n0 * p.ldb,
                                         (uint32_t)(((int64_t)(nrows - 1) * p.ldb + p.K) * 2));
-  uint32_t a_vo[INS], b_vo[INS];
+  uint32_t a_vo[AI], b_vo[BI];
   auto set_offsets = [&](int64_t lda, int64_t ldb) {
 #pragma unroll
-    for (int i = 0; i < INS; ++i) {
+    for (int i = 0; i < AI; ++i) {
       const int r = (i * NW + wid) * RPI + lrowi;
-      const int chunk = slot ^ dma_swz<BK>(r);
-      a_vo[i] = (uint32_t)(((int64_t)min(r, mrows - 1) * lda + chunk * 8) * 2);
-      b_vo[i] = (uint32_t)(((int64_t)min(r, nrows - 1) * ldb + chunk * 8) * 2);
+      a_vo[i] = (uint32_t)(((int64_t)min(r, mrows - 1) * lda + (slot ^ dma_swz<BK>(r)) * 8) * 2);
+    }
+#pragma unroll
+    for (int i = 0; i < BI; ++i) {
+      const int r = (i * NW + wid) * RPI + lrowi;
+      b_vo[i] = (uint32_t)(((int64_t)min(r, nrows - 1) * ldb + (slot ^ dma_swz<BK>(r)) * 8) * 2);
     }
   };
   set_offsets(p.lda, p.ldb);
   int kbase = 0;
   // Sets up the operand pair of tile t (the LoRA pair from tile nk1 on; tiles are set up in
-  // order) and returns its k byte offset.
+  // order, and every range starts before tile nk1) and returns its k byte offset.
   auto dma_tile = [&](int t) -> uint32_t {
     if (t == nk1) {
       ra = make_rsrc((const bf16_t*)p.A2 + seg_col_of(p, n0) + (int64_t)m0 * p.lda2,
@@ -774,16 +799,16 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
   auto dma_one = [&](int n, uint32_t kb, int stage) {
     bf16_t* as = As + stage * BM * BK + wid * RPI * BK;
     bf16_t* bs = Bs + stage * BN * BK + wid * RPI * BK;
-    if (n < INS) buf_lds16(ra, a_vo[n], kb, as + n * NW * RPI * BK);
-    else buf_lds16(rb, b_vo[n - INS], kb, bs + (n - INS) * NW * RPI * BK);
+    if (n < AI) buf_lds16(ra, a_vo[n], kb, as + n * NW * RPI * BK);
+    else buf_lds16(rb, b_vo[n - AI], kb, bs + (n - AI) * NW * RPI * BK);
   };
 
-  // Fragment rows wm*128 + 16i + lane%16 (A) / wn*128 + 16j + lane%16 (B); chunk 4s + lane/16 of
+  // Fragment rows WM wm + 16i + lane%16 (A) / WN wn + 16j + lane%16 (B); chunk 4s + lane/16 of
   // the 8 in a row (k-step s); every such row has the swizzle dma_swz(lane % 16).
   const int wm = wid >> 1, wn = wid & 1;
   const int lr = lane & 15, lk = lane >> 4;
   const int sw = dma_swz<BK>(lr);
-  const int a_row0 = (wm * 128 + lr) * BK, b_row0 = (wn * 128 + lr) * BK;
+  const int a_row0 = (wm * WM + lr) * BK, b_row0 = (wn * WN + lr) * BK;
   bf16x8_t fa0[TM], fb0[TN], fa1[TM], fb1[TN];
 
   f32x4_t acc[TM][TN];
@@ -794,49 +819,57 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
 
-  // One k-step: 64 MFMAs on (fa, fb); after every fourth a fragment read of A stage ra_st / B
-  // stage rb_st, k-step rs, in the order the next step consumes them (fa[0], fb[0..7], fa[1..7]);
-  // between two of those reads, after every eighth MFMA (the third of each eight), one of the 8
-  // direct-to-LDS loads of operand LB (0: A, 1: B) into stage dst.
+  // One k-step: TM TN MFMAs on (fa, fb). Spread evenly between them, a fragment read of A stage ra_st
+  // / B stage rb_st, k-step rs, in the order the next step consumes them (fa[0], fb[0..], fa[1..]),
+  // and one of the direct-to-LDS loads of operand LB (0: A, 1: B) into stage dst, placed between two
+  // of those reads (at 256x256: a read after every fourth MFMA, a load after the third of each eight).
+  constexpr int MF = TM * TN, NR = TM + TN;
   auto step = [&](const bf16x8_t (&fa)[TM], const bf16x8_t (&fb)[TN], bf16x8_t (&na)[TM], bf16x8_t (&nb)[TN],
                   int ra_st, int rb_st, int rs, auto lb, uint32_t kb, int dst) {
-    constexpr int LB = decltype(lb)::value;
+    constexpr int LB = decltype(lb)::value, NL = LB ? BI : AI;
     const bf16_t* as = As + ra_st * BM * BK + a_row0;
     const bf16_t* bs = Bs + rb_st * BN * BK + b_row0;
     const int co = ((4 * rs + lk) ^ sw) << 3;
+    // after MFMA idx: load number load_of(idx) and read number read_of(idx), or none (-1)
+    constexpr int OFF = MF >= 8 * NL ? 2 : 1;
+    auto load_of = [](int idx) {
+      const int n = (idx - OFF + MF) * NL / MF - NL;
+      return idx >= OFF && n * MF / NL + OFF == idx ? n : -1;
+    };
+    auto read_of = [](int idx) {
+      const int r = (idx * NR + MF - 1) / MF;
+      return r < NR && r * MF / NR == idx ? r : -1;
+    };
 #pragma unroll
-    for (int idx = 0; idx < TM * TN; ++idx) {
-      const int i = idx / TN, j = idx % TN;
+    for (int idx = 0; idx < MF; ++idx) {
+      const int i = idx / TN, j = idx % TN, n = load_of(idx), r = read_of(idx);
       acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
-      if (idx % 8 == 2) dma_one(LB * INS + idx / 8, kb, dst);
-      if (idx % 4 == 0) {
-        const int r = idx / 4;   // 0: fa[0]; 1..8: fb[0..7]; 9..15: fa[1..7]
-        if (r == 0) na[0] = *(const bf16x8_t*)&as[co];
-        else if (r <= TN) nb[r - 1] = *(const bf16x8_t*)&bs[(r - 1) * 16 * BK + co];
-        else na[r - TN] = *(const bf16x8_t*)&as[(r - TN) * 16 * BK + co];
-      }
+      if (n >= 0) dma_one(LB * AI + n, kb, dst);
+      if (r == 0) na[0] = *(const bf16x8_t*)&as[co];
+      else if (r > 0 && r <= TN) nb[r - 1] = *(const bf16x8_t*)&bs[(r - 1) * 16 * BK + co];
+      else if (r > TN) na[r - TN] = *(const bf16x8_t*)&as[(r - TN) * 16 * BK + co];
     }
 #pragma unroll
-    for (int idx = 0; idx < TM * TN; ++idx) {
+    for (int idx = 0; idx < MF; ++idx) {
       __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
-      if (idx % 8 == 2) __builtin_amdgcn_sched_group_barrier(SG_VMEM, 1, 0);
-      if (idx % 4 == 0) __builtin_amdgcn_sched_group_barrier(SG_DS_READ, 1, 0);
+      if (load_of(idx) >= 0) __builtin_amdgcn_sched_group_barrier(SG_VMEM, 1, 0);
+      if (read_of(idx) >= 0) __builtin_amdgcn_sched_group_barrier(SG_DS_READ, 1, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
   using LA = std::integral_constant<int, 0>;
   using LBt = std::integral_constant<int, 1>;
 
-  // Prologue: tiles 0 and 1 (clamped) in full; wait for tile 0; its step-0 fragments.
+  // Prologue: the first two tiles (clamped) in full; wait for the first; its step-0 fragments.
   {
-    uint32_t kb = dma_tile(0);
+    uint32_t kb = dma_tile(kt0);
 #pragma unroll
-    for (int n = 0; n < 2 * INS; ++n) dma_one(n, kb, 0);
-    kb = dma_tile(min(1, nk - 1));
+    for (int n = 0; n < AI + BI; ++n) dma_one(n, kb, 0);
+    kb = dma_tile(min(kt0 + 1, nk - 1));
 #pragma unroll
-    for (int n = 0; n < 2 * INS; ++n) dma_one(n, kb, 1);
+    for (int n = 0; n < AI + BI; ++n) dma_one(n, kb, 1);
   }
-  wait_vm<2 * INS>();
+  wait_vm<AI + BI>();
   __builtin_amdgcn_s_waitcnt(0xC07F);
   asm volatile("s_barrier" ::: "memory");
   {
@@ -853,15 +886,15 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
   // loads during the second (into tile kt's B stage, free after this tile's middle barrier), so
   // every step carries 8 loads per wave and the A loads have two to three steps to land.
   int sa = 0;                 // A stage of tile kt
-  for (int kt = 0; kt < nk; ++kt) {
+  for (int kt = kt0; kt < nk; ++kt) {
     const int sa1 = sa == 2 ? 0 : sa + 1, sa2 = sa1 == 2 ? 0 : sa1 + 1;
-    const int sb = kt & 1;
+    const int sb = (kt - kt0) & 1;
     __builtin_amdgcn_sched_barrier(0);
     const uint32_t kb = dma_tile(min(kt + 2, nk - 1));
     step(fa0, fb0, fa1, fb1, sa, sb, 1, LA{}, kb, sa2);
     // Tile kt+1 is complete once every wave is here with its loads landed (only tile kt+2's A
     // loads may still fly); tile kt's B stage is free.
-    wait_vm<INS>();
+    wait_vm<AI>();
     __builtin_amdgcn_s_waitcnt(0xC07F);
     asm volatile("s_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
@@ -881,14 +914,14 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
   auto epilogue = [&](auto has_res, auto checked) {
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      const int row = m0 + wm * 128 + i * 16 + lr;
+      const int row = m0 + wm * WM + i * 16 + lr;
       if (checked && row >= p.M) continue;
       const float sc = (!checked || p.gate == nullptr || p.gate[row] != 0) ? p.alpha : 0.f;
       OutT* crow = C + (int64_t)row * p.ldc;
       const OutT* rrow = has_res ? R + (int64_t)row * p.ldr : nullptr;
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        const int col = n0 + wn * 128 + j * 16 + lk * 4;
+        const int col = n0 + wn * WN + j * 16 + lk * 4;
         if (checked && col >= p.N) continue;
         float v[4];
 #pragma unroll
@@ -901,25 +934,29 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
     // SwiGLU backward of the down-projection data gradient: this product is dS[M, F] (never
     // stored); with R = gu [M, 2F] (ldr) and C = dgu [M, 2F] (ldc), writes dgu[:, f] and
     // dgu[:, F + f] from bf16(dS), g = gu[:, f], u = gu[:, F + f], as the SwiGLU backward kernel
-    // does after a bf16 product. Interior tiles only (checked by the caller). Each wave rounds its
-    // 128 x 128 quadrant of dS into a private 32 KB of the (now idle) LDS stages, 16-byte chunks
+    // does after a bf16 product. F is a multiple of 256; rows past M load the last row and store
+    // nothing. Each wave rounds its WM x 128 quadrant of dS into a private part of the (now idle) LDS stages, 16-byte chunks
     // XOR-swizzled by row so that both the fragment-ordered writes and the row-ordered reads are
     // conflict-free, then walks it four rows per step: every gu load and dgu store is a 256-byte
     // run per row (16 bytes per lane), with the gu loads of the next DEPTH batches of eight rows
     // in flight (the K loop's fragment registers hold them), the first ones issued before the
     // staging so that their latency passes behind it.
-    constexpr int PB = 2, NBATCH = 128 / (4 * PB), DEPTH = 6;
+    constexpr int PB = 2, NBATCH = WM / (4 * PB), DEPTH = 6;
     const int F = p.N;
     const int rsub = lane >> 4, c16 = lane & 15;
-    const int64_t row0 = m0 + wm * 128 + rsub;
-    const int col = n0 + wn * 128 + c16 * 8;
+    const int64_t row0 = m0 + wm * WM + rsub;
+    const int mleft = p.M - (int)row0;            // rows from row0 on that exist (may be <= 0)
+    const int col = n0 + wn * WN + c16 * 8;
     const bf16_t* gsrc = (const bf16_t*)p.R + row0 * p.ldr + col;
     bf16_t* dst = (bf16_t*)p.C + row0 * p.ldc + col;
+    auto body = [&](auto chk) {
+    constexpr bool CHK = decltype(chk)::value;
     uint4 gw[NBATCH][PB], uw[NBATCH][PB];   // fully unrolled: only DEPTH + 1 batches are live
     auto load_batch = [&](int b) {
 #pragma unroll
       for (int t = 0; t < PB; ++t) {
-        const bf16_t* g = gsrc + (int64_t)((b * PB + t) * 4) * p.ldr;
+        const int ro = (b * PB + t) * 4;
+        const bf16_t* g = gsrc + (int64_t)(CHK ? min(ro, mleft - 1) : ro) * p.ldr;
         gw[b][t] = *(const uint4*)g;
         uw[b][t] = *(const uint4*)(g + F);
       }
@@ -927,7 +964,7 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
 #pragma unroll
     for (int b = 0; b < DEPTH; ++b) load_batch(b);
     asm volatile("s_barrier" ::: "memory");   // every wave's fragment reads have completed (waited above)
-    bf16_t* q = smem + wid * 128 * 128;
+    bf16_t* q = smem + wid * WM * 128;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -963,10 +1000,13 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
           pu[e] = (uint32_t)f32_to_bf16(du[2 * e]) | ((uint32_t)f32_to_bf16(du[2 * e + 1]) << 16);
         }
         bf16_t* d = dst + (int64_t)((b * PB + t) * 4) * p.ldc;
+        if (CHK && (b * PB + t) * 4 >= mleft) continue;
         *(uint4*)d = og;
         *(uint4*)(d + F) = ou;
       }
     }
+    };
+    if (m0 + BM <= p.M) body(std::false_type{}); else body(std::true_type{});
     return;
   }
   if constexpr (EPI == 3) {
@@ -981,7 +1021,7 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
       // 4 consecutive columns of each (i, j) block, one 16-byte store each
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
-        const int row = m0 + wm * 128 + i * 16 + lr;
+        const int row = m0 + wm * WM + i * 16 + lr;
         if (row >= p.M) continue;
         float* zrow = p.ce_z + (int64_t)row * p.ce_ldz;
 #pragma unroll
@@ -999,7 +1039,7 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
     }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      const int row = m0 + wm * 128 + i * 16 + lr;
+      const int row = m0 + wm * WM + i * 16 + lr;
       float mx = -INFINITY;
 #pragma unroll
       for (int j = 0; j < TN; ++j)
@@ -1053,7 +1093,7 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
         const int64_t t = p.ce_tgt[row] - p.ce_vocab0;
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-          const int col = n0 + wn * 128 + j * 16 + lk * 4;
+          const int col = n0 + wn * WN + j * 16 + lk * 4;
           float v[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = cf * (fast_expf(acc[i][j][e] - lse) - ((int64_t)(col + e) == t ? 1.f : 0.f));
@@ -1074,14 +1114,14 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
     }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      const int row = m0 + wm * 128 + i * 16 + lr;
+      const int row = m0 + wm * WM + i * 16 + lr;
       if (row >= p.M) continue;
       const float lse = p.ce_lse[row], cf = p.ce_w[row] * gs;
       const int64_t t = p.ce_tgt[row] - p.ce_vocab0;
       bf16_t* crow = (bf16_t*)p.C + (int64_t)row * p.ldc;
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        const int col = n0 + wn * 128 + j * 16 + lk * 4;
+        const int col = n0 + wn * WN + j * 16 + lk * 4;
         if (col >= p.N) continue;
         float v[4];
 #pragma unroll
@@ -1104,17 +1144,20 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
     // C[row][64 b + c] = bf16(silu(g) u) with g, u rounded to bf16 first, as a bf16 GEMM followed
     // by the SwiGLU kernel computes it. With C2, also stores the rounded gate and up
     // values as C2[row][f] and C2[row][N/2 + f] (the [gate | up] layout of the plain product):
-    // then each wave rounds its 128 x (64 gate | 64 up) block into a private 32 KB of the idle
+    // then each wave rounds its WM x (64 gate | 64 up) block into a private part of the idle
     // LDS stages (16-byte chunks XOR-swizzled by row, as in the backward epilogue) and stores
     // both outputs by rows, 16 lanes per row: gate and up as 128-byte runs, C as one.
-    // Interior tiles only (checked by the caller).
+    // N is a multiple of 256 (checked by the caller); rows past M are not stored.
     const int f0 = (n0 + wn * 128) / 2;
+    const int rows = p.M - (m0 + wm * WM);        // this wave's rows that exist (may be <= 0)
+    auto body = [&](auto chk) {
+    constexpr bool CHK = decltype(chk)::value;
     if (p.C2 == nullptr && (p.ldc & 7) == 0) {
-      // Output only: each wave's 128 x 64 block goes through a private 16 KB of the idle LDS
+      // Output only: each wave's WM x 64 block goes through a private part of the idle LDS
       // stages (16-byte chunk c of row r at slot c ^ ((r >> 1) & 7)) and is stored by rows, eight
       // lanes per 128-byte row.
       asm volatile("s_barrier" ::: "memory");   // every wave's fragment reads have completed
-      bf16_t* q = smem + wid * 128 * 64;
+      bf16_t* q = smem + wid * WM * 64;
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         const int r = i * 16 + lr;
@@ -1134,10 +1177,11 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
       __builtin_amdgcn_s_waitcnt(0xC07F);
       __builtin_amdgcn_wave_barrier();
       const int c8 = lane & 7, rs = lane >> 3;
-      OutT* dst = C + (int64_t)(m0 + wm * 128 + rs) * p.ldc + f0 + 8 * c8;
+      OutT* dst = C + (int64_t)(m0 + wm * WM + rs) * p.ldc + f0 + 8 * c8;
 #pragma unroll 4
-      for (int it = 0; it < 16; ++it) {
+      for (int it = 0; it < WM / 8; ++it) {
         const int r = it * 8 + rs;
+        if (CHK && r >= rows) break;
         *(uint4*)(dst + (int64_t)(it * 8) * p.ldc) = *(const uint4*)&q[r * 64 + ((c8 ^ ((r >> 1) & 7)) << 3)];
       }
       return;
@@ -1145,7 +1189,8 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
     if (p.C2 == nullptr) {
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
-        OutT* crow = C + (int64_t)(m0 + wm * 128 + i * 16 + lr) * p.ldc;
+        if (CHK && i * 16 + lr >= rows) continue;
+        OutT* crow = C + (int64_t)(m0 + wm * WM + i * 16 + lr) * p.ldc;
 #pragma unroll
         for (int j = 0; j < TN / 2; ++j) {
           float v[4];
@@ -1161,7 +1206,7 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
       return;
     }
     asm volatile("s_barrier" ::: "memory");   // every wave's fragment reads have completed (waited above)
-    bf16_t* q = smem + wid * 128 * 128;
+    bf16_t* q = smem + wid * WM * 128;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -1176,12 +1221,13 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
     __builtin_amdgcn_wave_barrier();
     const int rsub = lane >> 4, c16 = lane & 15;
     const int F = p.N / 2;
-    const int64_t row0 = m0 + wm * 128 + rsub;
+    const int64_t row0 = m0 + wm * WM + rsub;
     bf16_t* gdst = (bf16_t*)p.C2 + row0 * p.ldc2 + (c16 < 8 ? f0 + 8 * c16 : F + f0 + 8 * (c16 - 8));
     OutT* sdst = C + row0 * p.ldc + f0 + 4 * c16;
 #pragma unroll 8
-    for (int it = 0; it < 32; ++it) {
+    for (int it = 0; it < WM / 4; ++it) {
       const int r = it * 4 + rsub;
+      if (CHK && r >= rows) break;
       const bf16_t* qr = q + r * 128;
       const uint4 vw = *(const uint4*)&qr[(c16 ^ (r & 15)) << 3];
       const uint2 gw = *(const uint2*)&qr[(((c16 >> 1) ^ (r & 15)) << 3) + (c16 & 1) * 4];
@@ -1197,6 +1243,8 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
       }
       store4(sdst + (int64_t)(it * 4) * p.ldc, nullptr, v);
     }
+    };
+    if (m0 + BM <= p.M) body(std::false_type{}); else body(std::true_type{});
     return;
   }
   if constexpr (EPI == 5) {
@@ -1204,10 +1252,10 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
     // in fp32 as for the plain epilogue; each row is then handled by 8 lanes, lane l holding
     // columns [8l, 8l+8) and their RoPE partners [64+8l, 64+8l+8): sum of squares over the head
     // (three lane shuffles), normalisation and weight, rotate_half RoPE within the lane (one
-    // angle-table read serves both halves), one rounding, 16-byte stores. Interior tiles only (the
-    // caller requires M and N to be multiples of 256).
+    // angle-table read serves both halves), one rounding, 16-byte stores. N is a multiple of 256
+    // (checked by the caller); rows past M are not stored.
     const int rsub = lane >> 3, l8 = lane & 7;
-    const int64_t rowb = m0 + wm * 128 + rsub;
+    const int64_t rowb = m0 + wm * WM + rsub;
     const int head = (n0 + wn * 128) >> 7;
     const int nq = p.qk_nq, nqk = p.qk_nq + p.qk_nk;
     const bool isv = head >= nqk, isq = head < nq;
@@ -1236,8 +1284,10 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
     }
     asm volatile("s_barrier" ::: "memory");   // every wave's fragment reads have completed
     float* q = (float*)smem + wid * 64 * 128;
+    auto body = [&](auto chk) {
+    constexpr bool CHK = decltype(chk)::value;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < WM / 64; ++h) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -1262,6 +1312,7 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
           for (int e = 0; e < 4; ++e) x[4 * c + e] = v[e];
         }
         const int64_t row = rowb + 64 * h + it * 8;
+        if (CHK && row >= p.M) break;   // a row's eight lanes leave together; its later rows are past M too
         float out[16];
         if (isv) {
 #pragma unroll
@@ -1306,32 +1357,50 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
       __builtin_amdgcn_s_waitcnt(0xC07F);     // the half's reads are done before the next overwrites
       __builtin_amdgcn_wave_barrier();
     }
+    };
+    if (m0 + BM <= p.M) body(std::false_type{}); else body(std::true_type{});
+    return;
+  }
+  if constexpr (EPI == 6) {
+    // fp32 sums of one K range, [M][N] of range `split` (N a multiple of 4, checked by the caller)
+    float* W = (float*)p.C + (int64_t)split * p.M * p.N;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int row = m0 + wm * WM + i * 16 + lr;
+      if (row >= p.M) continue;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int col = n0 + wn * WN + j * 16 + lk * 4;
+        if (col < p.N) *(f32x4_t*)(W + (int64_t)row * p.N + col) = acc[i][j];
+      }
+    }
     return;
   }
   const bool interior = m0 + BM <= p.M && n0 + BN <= p.N && p.gate == nullptr;
   if constexpr (EPI == 0 && std::is_same<OutT, bf16_t>::value) {
     if (interior && (p.ldc & 7) == 0 && (!R || (p.ldr & 7) == 0)) {
-      // Interior tile with bf16 output: each wave stages its 128 x 128 fp32 quadrant (alpha
-      // applied) through a private 32 KB of the idle LDS stages, 64 rows at a time, and stores by
-      // rows: 16 lanes per row, 8 columns (16 bytes) each, the residual read the same way. 16-byte
+      // Interior tile with bf16 output: each wave stages its WM x WN fp32 quadrant (alpha
+      // applied) through a private part of the idle LDS stages, 64 rows at a time, and stores by
+      // rows: WN / 8 lanes per row, 8 columns (16 bytes) each, the residual read the same way. 16-byte
       // chunk c of staged row r sits at slot c ^ (r & 15). The residual rows of both halves are
       // loaded first, into the registers the K loop's fragments held, so their latency passes
       // once, behind the staging, instead of once per group of rows.
-      const int rsub = lane >> 4, c16 = lane & 15;
-      const int64_t rowb = m0 + wm * 128 + rsub;
-      const int col = n0 + wn * 128 + 8 * c16;
-      uint4 rw[2][16];
+      constexpr int LPR = WN / 8, RS = 64 / LPR, NIT = 64 / RS;
+      const int rsub = lane / LPR, c16 = lane % LPR;
+      const int64_t rowb = m0 + wm * WM + rsub;
+      const int col = n0 + wn * WN + 8 * c16;
+      uint4 rw[WM / 64][NIT];
       if (R) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < WM / 64; ++h)
 #pragma unroll
-          for (int it = 0; it < 16; ++it)
-            rw[h][it] = *(const uint4*)((const bf16_t*)R + (rowb + 64 * h + it * 4) * p.ldr + col);
+          for (int it = 0; it < NIT; ++it)
+            rw[h][it] = *(const uint4*)((const bf16_t*)R + (rowb + 64 * h + it * RS) * p.ldr + col);
       }
       asm volatile("s_barrier" ::: "memory");   // every wave's fragment reads have completed
-      float* q = (float*)smem + wid * 64 * 128;
+      float* q = (float*)smem + wid * 64 * WN;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+      for (int h = 0; h < WM / 64; ++h) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -1340,16 +1409,16 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
             f32x4_t v;
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = acc[4 * h + i][j][e] * p.alpha;
-            *(f32x4_t*)&q[r * 128 + (((4 * j + lk) ^ (r & 15)) << 2)] = v;
+            *(f32x4_t*)&q[r * WN + (((4 * j + lk) ^ (r & 15)) << 2)] = v;
           }
         __builtin_amdgcn_s_waitcnt(0xC07F);
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int it = 0; it < 16; ++it) {
-          const int r = it * 4 + rsub;
-          const f32x4_t v0 = *(const f32x4_t*)&q[r * 128 + (((2 * c16) ^ (r & 15)) << 2)];
-          const f32x4_t v1 = *(const f32x4_t*)&q[r * 128 + (((2 * c16 + 1) ^ (r & 15)) << 2)];
-          const int64_t row = rowb + 64 * h + it * 4;
+        for (int it = 0; it < NIT; ++it) {
+          const int r = it * RS + rsub;
+          const f32x4_t v0 = *(const f32x4_t*)&q[r * WN + (((2 * c16) ^ (r & 15)) << 2)];
+          const f32x4_t v1 = *(const f32x4_t*)&q[r * WN + (((2 * c16 + 1) ^ (r & 15)) << 2)];
+          const int64_t row = rowb + 64 * h + it * RS;
           float a[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
           if (R) {
             const uint32_t* rp = (const uint32_t*)&rw[h][it];
@@ -1381,42 +1450,39 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
 // the others with 8.
 static int w4m16_group(int K) { return K >= 8192 ? 4 : 8; }
 
-template <typename OutT, int EPI = 0>
+template <typename OutT, int EPI = 0, int BM = 256, int BN = 256>
 static void launch_nt_w4m16(const GemmNT& p0, hipStream_t st) {
   GemmNT p = p0;
   p.group = w4m16_group(p.K + p.K2);
-  constexpr size_t lds = (3 * 256 + 2 * 256) * 64 * sizeof(bf16_t);   // 160 KB
-  UNOK_SET_LDS_ONCE((gemm_nt_bf16_w4m16_kernel<OutT, EPI>), lds);
-  const int nb = ((p.M + 255) / 256) * ((p.N + 255) / 256);
-  hipLaunchKernelGGL((gemm_nt_bf16_w4m16_kernel<OutT, EPI>), dim3(nb), dim3(256), lds, st, p);
+  // the K loop's stages (160 KB at 256x256), or what the epilogue stages 64 rows of each wave in
+  constexpr size_t loop = (3 * BM + 2 * BN) * 64 * sizeof(bf16_t), epi = 4 * 64 * (BN / 2) * sizeof(float);
+  constexpr size_t lds = loop > epi ? loop : epi;
+  UNOK_SET_LDS_ONCE((gemm_nt_bf16_w4m16_kernel<OutT, EPI, BM, BN>), lds);
+  const int nb = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN) * (EPI == 6 ? p.splits : 1);
+  hipLaunchKernelGGL((gemm_nt_bf16_w4m16_kernel<OutT, EPI, BM, BN>), dim3(nb), dim3(256), lds, st, p);
 }
 
 // The 4-wave kernel addresses each tile's operand strips (256 rows from the tile's first) through
 // buffer resources with 32-bit byte offsets and stores 4 output columns per vector (C and R rows
 // aligned to 16 bytes, N a multiple of 4).
+static bool out_vec4_ok(const GemmNT& p) {
+  return p.N % 4 == 0 && p.ldc % 4 == 0 && !((uintptr_t)p.C & 15) && (!p.R || (p.ldr % 4 == 0 && !((uintptr_t)p.R & 15)));
+}
 static bool buffer_ranges_ok(const GemmNT& p) {
   const int64_t lim = 0xFFFFFFFFll;
-  if (p.N % 4 || p.ldc % 4 || ((uintptr_t)p.C & 15) || (p.R && (p.ldr % 4 || ((uintptr_t)p.R & 15)))) return false;
+  if (!out_vec4_ok(p)) return false;
   const int64_t mr = (p.M < 256 ? p.M : 256) - 1, nr = (p.N < 256 ? p.N : 256) - 1;
   if ((mr * p.lda + p.K) * 2 > lim || (nr * p.ldb + p.K) * 2 > lim) return false;
   if (p.A2 && ((mr * p.lda2 + p.K2 + 4096) * 2 > lim || (nr * p.ldb2 + p.K2) * 2 > lim)) return false;
   return true;
 }
 
-template <int BM, int BN, int NW, int BK, int STAGES, typename OutT, bool ROT = false>
+template <int BM, int BN, int NW, int BK, int STAGES, typename OutT, bool ROT = false, bool SPLIT = false>
 static void launch_nt_dma_t(const GemmNT& p, hipStream_t st) {
   constexpr size_t lds = (size_t)STAGES * (BM + BN) * BK * sizeof(bf16_t);
-  UNOK_SET_LDS_ONCE((gemm_nt_bf16_dma_kernel<BM, BN, NW, BK, STAGES, OutT, ROT>), lds);
-  const int nb = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
-  hipLaunchKernelGGL((gemm_nt_bf16_dma_kernel<BM, BN, NW, BK, STAGES, OutT, ROT>), dim3(nb), dim3(NW * 64), lds, st, p);
-}
-
-// Large products: the 256x256 16x16x32-MFMA kernel; operands beyond its 32-bit buffer offsets
-// take the 8-wave direct-to-LDS kernel, which addresses them with 64-bit pointers.
-template <typename OutT>
-static void launch_nt_large(const GemmNT& p, hipStream_t st) {
-  if (buffer_ranges_ok(p)) launch_nt_w4m16<OutT>(p, st);
-  else launch_nt_dma_t<256, 256, 8, 64, 2, OutT>(p, st);
+  UNOK_SET_LDS_ONCE((gemm_nt_bf16_dma_kernel<BM, BN, NW, BK, STAGES, OutT, ROT, SPLIT>), lds);
+  const int nb = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN) * (SPLIT ? p.splits : 1);
+  hipLaunchKernelGGL((gemm_nt_bf16_dma_kernel<BM, BN, NW, BK, STAGES, OutT, ROT, SPLIT>), dim3(nb), dim3(NW * 64), lds, st, p);
 }
 
 // Skinny products (N <= 192): one 64 x N tile spans every output column, 4 LDS stages for
@@ -1424,8 +1490,142 @@ static void launch_nt_large(const GemmNT& p, hipStream_t st) {
 // spread over the rows' column offsets instead of all hitting the same one.
 template <int BN, int STAGES>
 static void launch_nt_skinny_t(const GemmNT& p, int out_dtype, hipStream_t st) {
-  if (out_dtype == UNOK_F32) launch_nt_dma_t<64, BN, 4, 64, STAGES, float, true>(p, st);
+  if (p.splits > 1) launch_nt_dma_t<64, BN, 4, 64, STAGES, float, true, true>(p, st);
+  else if (out_dtype == UNOK_F32) launch_nt_dma_t<64, BN, 4, 64, STAGES, float, true>(p, st);
   else launch_nt_dma_t<64, BN, 4, 64, STAGES, bf16_t, true>(p, st);
+}
+
+static void launch_nt_skinny(const GemmNT& p, int out_dtype, hipStream_t st) {
+  const int bn = (p.N + 63) / 64 * 64;
+  if (bn == 64) launch_nt_skinny_t<64, 4>(p, out_dtype, st);
+  else if (bn == 128 && p.splits <= 1 && p.M >= 32768 && p.K >= 8192) {
+    // many rows and a long K (the rank-128 products over the 12288-wide FFN side at 8 x 4096
+    // rows): 128-row tiles of 8 waves read each weight tile from L2 half as often (221 against
+    // 260 us at 32768 x 128 x 12288; at 4096-deep or 16384-row shapes they do not pay)
+    if (out_dtype == UNOK_F32) launch_nt_dma_t<128, 128, 8, 64, 3, float, true>(p, st);
+    else launch_nt_dma_t<128, 128, 8, 64, 3, bf16_t, true>(p, st);
+  } else if (bn == 128) launch_nt_skinny_t<128, 4>(p, out_dtype, st);
+  else launch_nt_skinny_t<192, 3>(p, out_dtype, st);
+}
+
+// C = alpha * gate (.) (sum of the K ranges' fp32 partials, in range order) + R; N a multiple of 4.
+template <typename OutT>
+__global__ __launch_bounds__(256) void nt_splitk_reduce_kernel(const GemmNT p, const float* __restrict__ ws) {
+  const unsigned n4 = (unsigned)p.N / 4, total = n4 * (unsigned)p.M;
+  const unsigned i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= total) return;
+  const int row = (int)(i / n4), col = (int)(i % n4) * 4;
+  const int64_t plane = (int64_t)p.M * p.N;
+  const float* src = ws + (int64_t)row * p.N + col;
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  for (int z0 = 0; z0 < p.splits; z0 += 8) {
+    f32x4_t v[8];
+#pragma unroll
+    for (int z = 0; z < 8; ++z)
+      if (z0 + z < p.splits) v[z] = *(const f32x4_t*)(src + (z0 + z) * plane);
+#pragma unroll
+    for (int z = 0; z < 8; ++z)
+      if (z0 + z < p.splits) acc += v[z];
+  }
+  const bool on = p.gate == nullptr || p.gate[row] != 0;
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = on ? acc[e] * p.alpha : 0.f;
+  OutT* dst = (OutT*)p.C + (int64_t)row * p.ldc + col;
+  const OutT* res = p.R ? (const OutT*)p.R + (int64_t)row * p.ldr + col : nullptr;
+  store4(dst, res, v);
+}
+
+// ---------------------------------------------------------------------------------------
+// Choice of the kernel and the K ranges of a bf16 product: the cheapest by a model of the times
+// measured with weights cold in the caches (microseconds; n = 64-deep K tiles of a range, f = share
+// of the 256 CUs a partial round of tiles covers; fewer workgroups share the L2 and the power
+// budget, so each runs faster):
+//   256x256   one workgroup per CU: 1.41 n + 8 per full round, (0.95 + 0.46 f) n + 8 for the rest
+//   128x256   one per CU:           0.97 n + 6,                (0.77 + 0.20 f) n + 6
+//   128x128   one per CU 0.62 n + 5, two per CU (1.01 n + 4) per 512 tiles, not in lockstep
+//   ranges    a second kernel: 4 us and the fp32 partials written and read once at 6 TB/s
+// and never below the operands' bytes at 4.5 TB/s. It reproduces 2048 x 4096 x 4096 at 83 / 63 / 65
+// us for the three tiles, 4096 x 4096 x 4096 at 100 / 125 / 126, 777 x 4096 x 12288 at 208 / 177 /
+// 139 in one range and 92 in four 256x256 ranges, 1801 x 2048 x 151936 at 2459 in one range and 887
+// in four, and 128 x 4096 x 4096 at 38 in one range of 128x128 tiles and 18 in eight.
+// ---------------------------------------------------------------------------------------
+enum NtTile { NT_REG = 0, NT_256 = 1, NT_128_256 = 2, NT_128 = 3, NT_SKINNY = 4, NT_LARGE64 = 5 };
+struct NtPlan { int tile, splits; };
+
+static bool nt_segs_ok(const GemmNT& p, int bn) {
+  for (int i = 0; p.A2 && i + 1 < p.nseg; ++i)
+    if (p.seg_end[i] % bn) return false;
+  return true;
+}
+
+static double nt_cost(int tile, int64_t M, int64_t N, int nk1, int nk2, int s) {
+  const int64_t bm = tile == NT_256 ? 256 : 128, bn = tile == NT_128 ? 128 : 256;
+  const int64_t wg = (M + bm - 1) / bm * ((N + bn - 1) / bn) * s;
+  const double n = (nk1 + s - 1) / s + nk2;
+  double t;
+  if (tile == NT_128) {
+    t = 0.62 * n + 5;
+    if (wg > 256) t = fmax(t, (double)wg / 512 * (1.01 * n + 4) + 5);
+  } else {
+    const double full = (double)(wg / 256), f = (double)(wg % 256) / 256;
+    t = tile == NT_256 ? full * (1.41 * n + 8) : full * (0.97 * n + 6);
+    if (f > 0) t += tile == NT_256 ? (0.95 + 0.46 * f) * n + 8 : (0.77 + 0.20 * f) * n + 6;
+  }
+  t = fmax(t, (double)(M + N) * (nk1 + nk2) * 128 / 4.5e6);
+  if (s > 1) t += 4 + (double)M * N * (8.0 * s + 2) / 6e6;
+  return t;
+}
+
+static int nt_ext_tiles(const GemmNT& p) { return p.A2 ? (p.K2 + 63) / 64 : 0; }
+
+// Row tile of a product whose epilogue needs 256-wide tiles and whole sums.
+static bool nt_rows128(const GemmNT& p) {
+  const int nk1 = p.K / 64, nk2 = nt_ext_tiles(p);
+  return nt_cost(NT_128_256, p.M, p.N, nk1, nk2, 1) < nt_cost(NT_256, p.M, p.N, nk1, nk2, 1);
+}
+
+static NtPlan nt_plan(const GemmNT& p, bool may_split) {
+  const int nk1 = p.K / 64, nk2 = nt_ext_tiles(p);
+  may_split = may_split && out_vec4_ok(p) && (int64_t)p.M * p.N < (1ll << 32);
+  if (p.N <= 192 && !p.A2 && p.K % 64 == 0 && nk1 > 0) {
+    // Skinny products (LoRA x A^T and dY B, N = r .. 3r): every activation row is read from HBM
+    // once, by 64-row tiles that span all N columns. (N = 256 and 384 run faster on the tiles below.)
+    // Few rows take K ranges, one round of workgroups (two per CU for N <= 64), at least four K tiles
+    // and at most 8 MB of partials: 2048 x 64 x 4096 22.7 -> 11.5 us, 777 x 192 x 12288 107 -> 21 us.
+    const int64_t wg = (p.M + 63) / 64;
+    int64_t s = 1;
+    if (may_split && wg < 256) {
+      s = (p.N <= 64 ? 512 : 256) / wg;
+      s = s < nk1 / 4 ? s : nk1 / 4;
+      s = s < 16 ? s : 16;
+      const int64_t cap = (8ll << 20) / ((int64_t)p.M * p.N * 4);
+      s = s < cap ? s : cap;
+      if (s < 1 || nk1 < 16) s = 1;
+    }
+    return {NT_SKINNY, (int)s};
+  }
+  if (p.K % 64 || nk1 == 0 || (p.A2 && p.K2 % 32) || !nt_segs_ok(p, 128)) return {NT_REG, 1};
+  if (!buffer_ranges_ok(p)) {
+    // operands beyond 32-bit buffer offsets: the kernel with 64-bit addresses
+    const int64_t big = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256);
+    const bool large = p.N > 128 && nt_segs_ok(p, 256) && big >= (p.K >= 8192 ? 192 : 256) && p.K2 % 64 == 0;
+    return {large ? NT_LARGE64 : NT_REG, 1};
+  }
+  const bool wide = p.N > 128 && nt_segs_ok(p, 256);
+  NtPlan best = {NT_128, 1};
+  double best_t = 1e30;
+  for (int tile = wide ? NT_256 : NT_128; tile <= NT_128; ++tile) {
+    for (int s = 1; s <= (may_split ? 16 : 1) && nk1 / s >= 4; ++s) {
+      const double t = nt_cost(tile, p.M, p.N, nk1, nk2, s);
+      if (t < best_t) { best_t = t; best = {tile, s}; }
+    }
+    if (nk1 < 4) {
+      const double t = nt_cost(tile, p.M, p.N, nk1, nk2, 1);
+      if (t < best_t) { best_t = t; best = {tile, 1}; }
+    }
+  }
+  return best;
 }
 
 // C = alpha * gate (.) (A B^T + A2[:, seg_col] B2^T) + R.
@@ -1434,14 +1634,14 @@ static void launch_nt_skinny_t(const GemmNT& p, int out_dtype, hipStream_t st) {
 // C[M, N/2] = silu(G) * U for the gate/up product A[M,K] B[N,K]^T with 64-row interleaved B (rows
 // 128 b + [0, 64) gate, 128 b + [64, 128) up of features 64 b + [0, 64)), bf16, rounded as the
 // unfused product followed by unok_swiglu_fwd. M and N multiples of 256, K of 64.
-UNOK_EXPORT int unok_gemm_nt_swiglu(int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
+static int swiglu_fwd_product(int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
                                     const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
-                                    void* C, int64_t ldc, void* gu, int64_t ldgu, void* stream) {
+                                    void* C, int64_t ldc, void* gu, int64_t ldgu, void* stream, int row_step) {
   UNOK_REQUIRE(M >= 0 && N >= 0 && K >= 0 && K2 >= 0, UNOK_EINVAL, "gemm_nt_swiglu: negative size M=%d N=%d K=%d",
                M, N, K);
   if (M == 0 || N == 0) return 0;
   const bool ext = A2 != nullptr && K2 > 0;
-  UNOK_REQUIRE(M % 256 == 0 && N % 256 == 0 && K % 64 == 0 && K > 0 && (!ext || K2 % 32 == 0), UNOK_EINVAL,
+  UNOK_REQUIRE(M % row_step == 0 && N % 256 == 0 && K % 64 == 0 && K > 0 && (!ext || K2 % 32 == 0), UNOK_EINVAL,
                "gemm_nt_swiglu: M=%d and N=%d must be multiples of 256, K=%d of 64 and K2=%d of 32", M, N, K, K2);
   UNOK_REQUIRE(lda % 8 == 0 && ldb % 8 == 0 && ldc % 8 == 0 && aligned16(A) && aligned16(B) && aligned16(C) &&
                    (!ext || (lda2 % 8 == 0 && ldb2 % 8 == 0 && aligned16(A2) && aligned16(B2))) &&
@@ -1454,8 +1654,22 @@ UNOK_EXPORT int unok_gemm_nt_swiglu(int M, int N, int K, const void* A, int64_t 
   p.M = M; p.N = N; p.K = K; p.K2 = ext ? K2 : 0; p.alpha = 1.f; p.nseg = 1;
   for (int i = 0; i < 4; ++i) { p.seg_end[i] = N; p.seg_col[i] = 0; }
   UNOK_REQUIRE(buffer_ranges_ok(p), UNOK_EINVAL, "gemm_nt_swiglu: operands exceed 32-bit buffer offsets");
-  launch_nt_w4m16<bf16_t, 1>(p, (hipStream_t)stream);
+  if (nt_rows128(p)) launch_nt_w4m16<bf16_t, 1, 128>(p, (hipStream_t)stream);
+  else launch_nt_w4m16<bf16_t, 1>(p, (hipStream_t)stream);
   return unok::check_launch("gemm_nt_swiglu");
+}
+
+UNOK_EXPORT int unok_gemm_nt_swiglu(int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
+                                    const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
+                                    void* C, int64_t ldc, void* gu, int64_t ldgu, void* stream) {
+  return swiglu_fwd_product(M, N, K, A, lda, B, ldb, A2, lda2, B2, ldb2, K2, C, ldc, gu, ldgu, stream, 256);
+}
+
+// unok_gemm_nt_swiglu for any number of rows.
+UNOK_EXPORT int unok_gemm_nt_swiglu_any(int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
+                                        const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
+                                        void* C, int64_t ldc, void* gu, int64_t ldgu, void* stream) {
+  return swiglu_fwd_product(M, N, K, A, lda, B, ldb, A2, lda2, B2, ldb2, K2, C, ldc, gu, ldgu, stream, 1);
 }
 
 // q|k|v projection with the q/k RMSNorm and RoPE in its epilogue (bf16, head dim 128): the product
@@ -1466,17 +1680,18 @@ UNOK_EXPORT int unok_gemm_nt_swiglu(int M, int N, int K, const void* A, int64_t 
 // non-null). cos_tab / sin_tab [P, 64] hold cos / sin of fl32(p * inv_freq[j]) (unok_rope_table);
 // positions are clamped to [0, P). Same values as unok_gemm_nt into fp32 followed by
 // unok_qknorm_rope_fwd. M and N multiples of 256, K of 64, K2 of 32.
-UNOK_EXPORT int unok_gemm_nt_qkv_rope(int M, int K, int nq, int nk, const void* A, int64_t lda, const void* B,
+static int qkv_rope_product(int M, int K, int nq, int nk, const void* A, int64_t lda, const void* B,
                                       int64_t ldb, const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
                                       int nseg, const int* seg_end, const int* seg_col, const void* wq, const void* wk,
                                       const int64_t* pos, const float* cos_tab, const float* sin_tab, int P, float eps,
-                                      void* q_out, void* k_out, void* v_out, float* rstd, void* qk_pre, void* stream) {
+                                      void* q_out, void* k_out, void* v_out, float* rstd, void* qk_pre, void* stream,
+                                      int row_step) {
   UNOK_REQUIRE(M >= 0 && K >= 0 && K2 >= 0 && nq > 0 && nk > 0 && P > 0, UNOK_EINVAL,
                "gemm_nt_qkv_rope: bad sizes M=%d K=%d nq=%d nk=%d P=%d", M, K, nq, nk, P);
   if (M == 0) return 0;
   const int N = 128 * (nq + 2 * nk);
   const bool ext = A2 != nullptr && K2 > 0;
-  UNOK_REQUIRE(M % 256 == 0 && N % 256 == 0 && K % 64 == 0 && K > 0 && (!ext || K2 % 32 == 0) && nseg >= 0 &&
+  UNOK_REQUIRE(M % row_step == 0 && N % 256 == 0 && K % 64 == 0 && K > 0 && (!ext || K2 % 32 == 0) && nseg >= 0 &&
                    nseg <= 4 && (wq == nullptr) == (wk == nullptr),
                UNOK_EINVAL, "gemm_nt_qkv_rope: M=%d and N=%d must be multiples of 256, K=%d of 64, K2=%d of 32", M, N,
                K, K2);
@@ -1503,20 +1718,40 @@ UNOK_EXPORT int unok_gemm_nt_qkv_rope(int M, int K, int nq, int nk, const void* 
   p.qk_wq = wq; p.qk_wk = wk; p.qk_pos = pos; p.qk_cos = cos_tab; p.qk_sin = sin_tab; p.qk_P = P;
   p.qk_nq = nq; p.qk_nk = nk; p.qk_eps = eps;
   UNOK_REQUIRE(buffer_ranges_ok(p), UNOK_EINVAL, "gemm_nt_qkv_rope: operands exceed 32-bit buffer offsets");
-  launch_nt_w4m16<bf16_t, 5>(p, (hipStream_t)stream);
+  if (nt_rows128(p)) launch_nt_w4m16<bf16_t, 5, 128>(p, (hipStream_t)stream);
+  else launch_nt_w4m16<bf16_t, 5>(p, (hipStream_t)stream);
   return unok::check_launch("gemm_nt_qkv_rope");
+}
+
+UNOK_EXPORT int unok_gemm_nt_qkv_rope(int M, int K, int nq, int nk, const void* A, int64_t lda, const void* B,
+                                      int64_t ldb, const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
+                                      int nseg, const int* seg_end, const int* seg_col, const void* wq, const void* wk,
+                                      const int64_t* pos, const float* cos_tab, const float* sin_tab, int P, float eps,
+                                      void* q_out, void* k_out, void* v_out, float* rstd, void* qk_pre, void* stream) {
+  return qkv_rope_product(M, K, nq, nk, A, lda, B, ldb, A2, lda2, B2, ldb2, K2, nseg, seg_end, seg_col, wq, wk, pos, cos_tab, sin_tab, P,
+                          eps, q_out, k_out, v_out, rstd, qk_pre, stream, 256);
+}
+
+// unok_gemm_nt_qkv_rope for any number of rows.
+UNOK_EXPORT int unok_gemm_nt_qkv_rope_any(int M, int K, int nq, int nk, const void* A, int64_t lda, const void* B,
+                                      int64_t ldb, const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
+                                      int nseg, const int* seg_end, const int* seg_col, const void* wq, const void* wk,
+                                      const int64_t* pos, const float* cos_tab, const float* sin_tab, int P, float eps,
+                                      void* q_out, void* k_out, void* v_out, float* rstd, void* qk_pre, void* stream) {
+  return qkv_rope_product(M, K, nq, nk, A, lda, B, ldb, A2, lda2, B2, ldb2, K2, nseg, seg_end, seg_col, wq, wk, pos, cos_tab, sin_tab, P,
+                          eps, q_out, k_out, v_out, rstd, qk_pre, stream, 1);
 }
 
 // dgu[M, 2F] = SwiGLU backward of dS = A[M,K] B[F,K]^T + A2[M,K2] B2[F,K2]^T (bf16, never stored)
 // against gu[M, 2F] = [gate | up]; rounded exactly as unok_gemm_nt followed by unok_swiglu_bwd.
 // M and F multiples of 256, K of 64, K2 of 32.
-UNOK_EXPORT int unok_gemm_nt_swiglu_bwd(int M, int F, int K, const void* A, int64_t lda, const void* B,
+static int swiglu_bwd_product(int M, int F, int K, const void* A, int64_t lda, const void* B,
                                         int64_t ldb, const void* A2, int64_t lda2, const void* B2, int64_t ldb2,
                                         int K2, const void* gu, int64_t ldgu, void* dgu, int64_t lddgu,
-                                        void* stream) {
+                                        void* stream, int row_step) {
   UNOK_REQUIRE(M >= 0 && F >= 0 && K >= 0 && K2 >= 0, UNOK_EINVAL, "gemm_nt_swiglu_bwd: negative size");
   if (M == 0 || F == 0) return 0;
-  UNOK_REQUIRE(M % 256 == 0 && F % 256 == 0 && K % 64 == 0 && K > 0 && K2 % 32 == 0, UNOK_EINVAL,
+  UNOK_REQUIRE(M % row_step == 0 && F % 256 == 0 && K % 64 == 0 && K > 0 && K2 % 32 == 0, UNOK_EINVAL,
                "gemm_nt_swiglu_bwd: M=%d and F=%d must be multiples of 256, K=%d of 64 and K2=%d of 32", M, F, K, K2);
   UNOK_REQUIRE(lda % 8 == 0 && ldb % 8 == 0 && ldgu % 8 == 0 && lddgu % 8 == 0 && aligned16(A) && aligned16(B) &&
                    aligned16(gu) && aligned16(dgu) && (K2 == 0 || (lda2 % 8 == 0 && ldb2 % 8 == 0 && aligned16(A2) &&
@@ -1529,8 +1764,24 @@ UNOK_EXPORT int unok_gemm_nt_swiglu_bwd(int M, int F, int K, const void* A, int6
   p.M = M; p.N = F; p.K = K; p.K2 = p.A2 ? K2 : 0; p.alpha = 1.f; p.nseg = 1;
   for (int i = 0; i < 4; ++i) { p.seg_end[i] = F; p.seg_col[i] = 0; }
   UNOK_REQUIRE(buffer_ranges_ok(p), UNOK_EINVAL, "gemm_nt_swiglu_bwd: operands exceed 32-bit buffer offsets");
-  launch_nt_w4m16<bf16_t, 2>(p, (hipStream_t)stream);
+  if (nt_rows128(p)) launch_nt_w4m16<bf16_t, 2, 128>(p, (hipStream_t)stream);
+  else launch_nt_w4m16<bf16_t, 2>(p, (hipStream_t)stream);
   return unok::check_launch("gemm_nt_swiglu_bwd");
+}
+
+UNOK_EXPORT int unok_gemm_nt_swiglu_bwd(int M, int F, int K, const void* A, int64_t lda, const void* B,
+                                        int64_t ldb, const void* A2, int64_t lda2, const void* B2, int64_t ldb2,
+                                        int K2, const void* gu, int64_t ldgu, void* dgu, int64_t lddgu,
+                                        void* stream) {
+  return swiglu_bwd_product(M, F, K, A, lda, B, ldb, A2, lda2, B2, ldb2, K2, gu, ldgu, dgu, lddgu, stream, 256);
+}
+
+// unok_gemm_nt_swiglu_bwd for any number of rows.
+UNOK_EXPORT int unok_gemm_nt_swiglu_bwd_any(int M, int F, int K, const void* A, int64_t lda, const void* B,
+                                        int64_t ldb, const void* A2, int64_t lda2, const void* B2, int64_t ldb2,
+                                        int K2, const void* gu, int64_t ldgu, void* dgu, int64_t lddgu,
+                                        void* stream) {
+  return swiglu_bwd_product(M, F, K, A, lda, B, ldb, A2, lda2, B2, ldb2, K2, gu, ldgu, dgu, lddgu, stream, 1);
 }
 
 // Operand checks of the LM-head loss products (H[R,K] W[V,K]^T through the 256x256 kernel, which
@@ -1587,12 +1838,12 @@ UNOK_EXPORT int unok_lmhead_ce_grad(int R, int V, int K, const void* H, int64_t 
   return unok::check_launch("lmhead_ce_grad");
 }
 
-UNOK_EXPORT int unok_gemm_nt(int in_dtype, int out_dtype, int M, int N, int K,
-                             const void* A, int64_t lda, const void* B, int64_t ldb,
-                             const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
-                             int nseg, const int* seg_end, const int* seg_col,
-                             void* C, int64_t ldc, const void* R, int64_t ldr,
-                             const uint8_t* gate, float alpha, void* stream) {
+static int gemm_nt_any(int in_dtype, int out_dtype, int M, int N, int K,
+                       const void* A, int64_t lda, const void* B, int64_t ldb,
+                       const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
+                       int nseg, const int* seg_end, const int* seg_col,
+                       void* C, int64_t ldc, const void* R, int64_t ldr,
+                       const uint8_t* gate, float alpha, int plan, void* ws, int64_t ws_bytes, void* stream) {
   UNOK_REQUIRE(M >= 0 && N >= 0 && K >= 0, UNOK_EINVAL, "gemm_nt: negative size M=%d N=%d K=%d", M, N, K);
   if (M == 0 || N == 0) return 0;
   UNOK_REQUIRE(in_dtype == UNOK_F32 || in_dtype == UNOK_BF16, UNOK_EINVAL, "gemm_nt: bad in_dtype %d", in_dtype);
@@ -1632,39 +1883,102 @@ UNOK_EXPORT int unok_gemm_nt(int in_dtype, int out_dtype, int M, int N, int K,
     for (int i = 0; i < p.nseg; ++i)
       UNOK_REQUIRE(p.seg_col[i] % 8 == 0, UNOK_EALIGN, "gemm_nt(bf16): segment column %d not a multiple of 8", p.seg_col[i]);
   }
-  // Tile choice: the largest tile whose N-segment boundaries stay tile-aligned.
-  auto segs_ok = [&](int bn) {
-    for (int i = 0; p.A2 && i + 1 < p.nseg; ++i) if (p.seg_end[i] % bn) return false;
-    return true;
-  };
-  const long long big_tiles = (long long)((M + 255) / 256) * ((N + 255) / 256);
-  if (N <= 192 && !p.A2 && K % 64 == 0 && M >= 4096) {
-    // Skinny products (LoRA x·Aᵀ and dY·B, N = r .. 3r): every activation row is read from HBM once.
-    // (N = 256 and 384 run faster on the 128x128 and 256x256 kernels: 116 / 105 us against 135 /
-    // 208 us for a 64 x N tile at 32768 x 4096.)
-    const int bn = (N + 63) / 64 * 64;
-    if (bn == 64) launch_nt_skinny_t<64, 4>(p, out_dtype, st);
-    else if (bn == 128 && M >= 32768 && K >= 8192) {
-      // many rows and a long K (the rank-128 products over the 12288-wide FFN side at 8 x 4096
-      // rows): 128-row tiles of 8 waves read each weight tile from L2 half as often (221 against
-      // 260 us at 32768 x 128 x 12288; at 4096-deep or 16384-row shapes they do not pay)
-      if (out_dtype == UNOK_F32) launch_nt_dma_t<128, 128, 8, 64, 3, float, true>(p, st);
-      else launch_nt_dma_t<128, 128, 8, 64, 3, bf16_t, true>(p, st);
-    } else if (bn == 128) launch_nt_skinny_t<128, 4>(p, out_dtype, st);
-    else launch_nt_skinny_t<192, 3>(p, out_dtype, st);
-  } else if (N <= 64 || !segs_ok(128)) {
-    UNOK_REQUIRE(segs_ok(64), UNOK_EINVAL, "gemm_nt(bf16): segment ends must be multiples of 64");
-    launch_nt_bf16<128, 64>(p, out_dtype, st);
-  } else if (N <= 128 || !segs_ok(256) || big_tiles < (K >= 8192 ? 192 : 256)) {
-    // (a long-K product keeps the 256x256 kernel down to three quarters of a tile per CU)
-    if ((long long)((M + 127) / 128) * ((N + 127) / 128) < 256) launch_nt_bf16<64, 128>(p, out_dtype, st);
-    else launch_nt_bf16<128, 128>(p, out_dtype, st);
-  } else if (K % 64 == 0 && (!p.A2 || p.K2 % 32 == 0)) {
-    if (out_dtype == UNOK_F32) launch_nt_large<float>(p, st); else launch_nt_large<bf16_t>(p, st);
-  } else {
-    launch_nt_bf16<256, 256>(p, out_dtype, st);
+  NtPlan pl = nt_plan(p, ws != nullptr);
+  if (plan > 0) {
+    const int tile = plan & 15, n = plan >> 4;
+    const bool tiles = tile >= NT_256 && tile <= NT_128 && K > 0 && K % 64 == 0 && (!p.A2 || K2 % 32 == 0) &&
+                       nt_segs_ok(p, tile == NT_128 ? 128 : 256) && buffer_ranges_ok(p);
+    const bool skinny = tile == NT_SKINNY && N <= 192 && !p.A2 && K > 0 && K % 64 == 0;
+    UNOK_REQUIRE((tiles || skinny) && n >= 1 && n <= K / 64 && (n == 1 || (ws && out_vec4_ok(p) && (int64_t)M * N < (1ll << 32))),
+                 UNOK_EINVAL, "gemm_nt: plan %d does not take this product", plan);
+    pl = {tile, n};
+  }
+  p.splits = pl.splits;
+  if (pl.splits > 1) {
+    UNOK_REQUIRE((int64_t)pl.splits * M * N * 4 <= ws_bytes && aligned16(ws), UNOK_EINVAL,
+                 "gemm_nt: workspace of %lld bytes (16-byte aligned) required, got %lld",
+                 (long long)((int64_t)pl.splits * M * N * 4), (long long)ws_bytes);
+    GemmNT q = p;
+    q.C = ws; q.ldc = N; q.R = nullptr; q.gate = nullptr; q.alpha = 1.f;
+    if (pl.tile == NT_SKINNY) launch_nt_skinny(q, UNOK_F32, st);
+    else if (pl.tile == NT_256) launch_nt_w4m16<float, 6, 256, 256>(q, st);
+    else if (pl.tile == NT_128_256) launch_nt_w4m16<float, 6, 128, 256>(q, st);
+    else launch_nt_w4m16<float, 6, 128, 128>(q, st);
+    const int rc = unok::check_launch("gemm_nt_splits");
+    if (rc) return rc;
+    const unsigned nb = (unsigned)(((int64_t)M * N / 4 + 255) / 256);
+    if (out_dtype == UNOK_F32) hipLaunchKernelGGL((nt_splitk_reduce_kernel<float>), dim3(nb), dim3(256), 0, st, p, (const float*)ws);
+    else hipLaunchKernelGGL((nt_splitk_reduce_kernel<bf16_t>), dim3(nb), dim3(256), 0, st, p, (const float*)ws);
+    return unok::check_launch("gemm_nt_reduce");
+  }
+  const bool f32 = out_dtype == UNOK_F32;
+  switch (pl.tile) {
+    case NT_SKINNY: launch_nt_skinny(p, out_dtype, st); break;
+    case NT_256: if (f32) launch_nt_w4m16<float>(p, st); else launch_nt_w4m16<bf16_t>(p, st); break;
+    case NT_128_256:
+      if (f32) launch_nt_w4m16<float, 0, 128, 256>(p, st); else launch_nt_w4m16<bf16_t, 0, 128, 256>(p, st);
+      break;
+    case NT_128:
+      if (f32) launch_nt_w4m16<float, 0, 128, 128>(p, st); else launch_nt_w4m16<bf16_t, 0, 128, 128>(p, st);
+      break;
+    case NT_LARGE64:
+      if (f32) launch_nt_dma_t<256, 256, 8, 64, 2, float>(p, st); else launch_nt_dma_t<256, 256, 8, 64, 2, bf16_t>(p, st);
+      break;
+    default: {
+      // register-staged kernel: the largest tile whose N-segment boundaries stay tile-aligned
+      const long long big_tiles = (long long)((M + 255) / 256) * ((N + 255) / 256);
+      if (N <= 64 || !nt_segs_ok(p, 128)) {
+        UNOK_REQUIRE(nt_segs_ok(p, 64), UNOK_EINVAL, "gemm_nt(bf16): segment ends must be multiples of 64");
+        launch_nt_bf16<128, 64>(p, out_dtype, st);
+      } else if (N <= 128 || !nt_segs_ok(p, 256) || big_tiles < (K >= 8192 ? 192 : 256)) {
+        // (a long-K product keeps the 256x256 tile down to three quarters of a tile per CU)
+        if ((long long)((M + 127) / 128) * ((N + 127) / 128) < 256) launch_nt_bf16<64, 128>(p, out_dtype, st);
+        else launch_nt_bf16<128, 128>(p, out_dtype, st);
+      } else {
+        launch_nt_bf16<256, 256>(p, out_dtype, st);
+      }
+    }
   }
   return unok::check_launch("gemm_nt_bf16");
+}
+
+UNOK_EXPORT int unok_gemm_nt(int in_dtype, int out_dtype, int M, int N, int K,
+                             const void* A, int64_t lda, const void* B, int64_t ldb,
+                             const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
+                             int nseg, const int* seg_end, const int* seg_col,
+                             void* C, int64_t ldc, const void* R, int64_t ldr,
+                             const uint8_t* gate, float alpha, void* stream) {
+  return gemm_nt_any(in_dtype, out_dtype, M, N, K, A, lda, B, ldb, A2, lda2, B2, ldb2, K2, nseg, seg_end, seg_col, C, ldc,
+                     R, ldr, gate, alpha, 0, nullptr, 0, stream);
+}
+
+// The library's choice for a product with a workspace: tile + 16 * ranges (0: fp32, and sizes or
+// segments only the register-staged kernel takes). K2 = 0 without an extension.
+UNOK_EXPORT int unok_gemm_nt_plan(int in_dtype, int M, int N, int K, int K2, int nseg, const int* seg_end) {
+  if (in_dtype != UNOK_BF16 || M <= 0 || N <= 0 || K <= 0) return 0;
+  GemmNT p{};
+  p.M = M; p.N = N; p.K = K; p.K2 = K2; p.lda = p.ldb = K; p.lda2 = p.ldb2 = K2; p.ldc = N;
+  p.nseg = 1;
+  for (int i = 0; i < 4; ++i) p.seg_end[i] = N;
+  if (K2 > 0) {
+    p.A2 = &p;      // only tested against null
+    p.nseg = nseg > 0 && nseg <= 4 ? nseg : 1;
+    for (int i = 0; i < p.nseg && nseg > 0; ++i) p.seg_end[i] = seg_end[i];
+  }
+  const NtPlan pl = nt_plan(p, true);
+  return pl.tile == NT_REG ? 0 : pl.tile + 16 * pl.splits;
+}
+
+// unok_gemm_nt with a workspace of ws_bytes for the partial sums of a product whose K is split.
+// plan 0: the library's choice; otherwise tile + 16 * ranges (for measurements and tests).
+UNOK_EXPORT int unok_gemm_nt_ws(int in_dtype, int out_dtype, int M, int N, int K,
+                                const void* A, int64_t lda, const void* B, int64_t ldb,
+                                const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
+                                int nseg, const int* seg_end, const int* seg_col,
+                                void* C, int64_t ldc, const void* R, int64_t ldr,
+                                const uint8_t* gate, float alpha, int plan, void* ws, int64_t ws_bytes, void* stream) {
+  return gemm_nt_any(in_dtype, out_dtype, M, N, K, A, lda, B, ldb, A2, lda2, B2, ldb2, K2, nseg, seg_end, seg_col, C, ldc,
+                     R, ldr, gate, alpha, plan, ws, ws_bytes, stream);
 }
 
 // Workspace bytes gemm_tn needs for a given problem (partials of the split-K reduction).

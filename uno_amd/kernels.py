@@ -6,6 +6,7 @@ non-HIP code path.
 """
 from __future__ import annotations
 
+from functools import lru_cache
 from typing import Sequence
 
 import torch
@@ -39,13 +40,18 @@ def set_recorder(rec: LaunchRecorder | None) -> None:
     _recorder = rec
 
 
+@lru_cache(maxsize=4096)
+def nt_plan(M: int, N_: int, K: int, K2: int = 0, seg_end: tuple = ()) -> tuple[int, int]:
+    """(tile, K ranges) the library takes for a bf16 product with a workspace (unok_gemm_nt_plan);
+    tile 0 is the register-staged kernel. A function of the sizes alone."""
+    code = N.lib().unok_gemm_nt_plan(N.BF16, M, N_, K, K2, len(seg_end), N.int_array(seg_end))
+    return code & 15, max(1, code >> 4)
+
+
 def nt_uses_256_tiles(M: int, N: int, seg_end, K: int = 0) -> bool:
-    """Mirror of the tile choice in unok_gemm_nt for bf16 (the 256x256 MFMA kernel)."""
-    if N <= 128:
-        return False
-    if any(e % 256 for e in list(seg_end)[:-1]):
-        return False
-    return ((M + 255) // 256) * ((N + 255) // 256) >= (192 if K >= 8192 else 256)
+    """Whether unok_gemm_nt runs a bf16 product on the 256x256 MFMA kernel."""
+    segs = tuple(seg_end)
+    return nt_plan(M, N, K or 4096, 64 if len(segs) > 1 else 0, segs if len(segs) > 1 else ())[0] == 1
 
 
 def _rowmajor(t: torch.Tensor, name: str) -> None:
@@ -115,12 +121,14 @@ def gemm_nt(a: torch.Tensor, b: torch.Tensor, *, a2: torch.Tensor | None = None,
         ev0.record()
     else:
         rec = None
-    N.call("unok_gemm_nt", N.dtype_code(a.dtype), N.dtype_code(out_dtype), M, Nn, K,
+    ranges = nt_plan(M, Nn, K, K2, tuple(seg_end))[1] if a.dtype == torch.bfloat16 and M > 0 and Nn > 0 else 1
+    ws = torch.empty(ranges * M * Nn, device=a.device, dtype=torch.float32) if ranges > 1 else None
+    N.call("unok_gemm_nt_ws", N.dtype_code(a.dtype), N.dtype_code(out_dtype), M, Nn, K,
            N.ptr(a), _ld(a), N.ptr(b), _ld(b),
            N.ptr(a2), _ld(a2) if a2 is not None else 0, N.ptr(b2), _ld(b2) if b2 is not None else 0, K2,
            len(seg_end), N.int_array(seg_end), N.int_array(seg_col),
            N.ptr(out), _ld(out), N.ptr(residual), _ld(residual) if residual is not None else 0,
-           N.ptr(gate), float(alpha), N.stream())
+           N.ptr(gate), float(alpha), 0, N.ptr(ws), ranges * M * Nn * 4 if ws is not None else 0, N.stream())
     if rec is not None:
         ev1.record()
         rec.records.append((ev0, ev1, 2.0 * M * Nn * (K + K2), (M, Nn, K, K2)))
