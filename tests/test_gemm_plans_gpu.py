@@ -111,3 +111,58 @@ def test_plan_rejects_what_a_tile_does_not_take(dev):
         _call(4 + 16, a, b, None, None, [], out, None, None, 1.0, 1)       # 256 columns are not skinny
     with pytest.raises(ValueError, match="plan"):
         _call(1 + 16 * 2, a, b, None, None, [], out, None, None, 1.0, 1)   # ranges without a workspace
+
+
+@pytest.mark.parametrize("M", [1, 100, 129, 300, 511, 2100])
+@pytest.mark.parametrize("F,Kd,r", [(256, 128, 32), (1536, 512, 64)])
+def test_fused_epilogues_on_any_row_count(dev, M, F, Kd, r):
+    """The SwiGLU products on row counts between tiles: bit for bit the first M rows of the product over
+    rows padded to a multiple of 256, and no row past M written."""
+    torch.manual_seed(M + F)
+    P = (M + 255) // 256 * 256
+    bf = torch.bfloat16
+    x, h = (torch.randn(P, Kd, device=dev) * 0.5).to(bf), (torch.randn(P, 2 * r, device=dev) * 0.5).to(bf)
+    w, sb = (torch.randn(2 * F, Kd, device=dev) * 0.1).to(bf), (torch.randn(2 * F, 2 * r, device=dev) * 0.1).to(bf)
+    gu_p = torch.empty(P, 2 * F, device=dev, dtype=bf)
+    for kw, kw_p in (({}, {}), (dict(a2=h[:M], b2_interleaved=sb), dict(a2=h, b2_interleaved=sb))):
+        gu = torch.full((P, 2 * F), 7.0, device=dev, dtype=bf)
+        out = torch.full((P, F), 7.0, device=dev, dtype=bf)
+        ref = K.gemm_nt_swiglu(x, w, gu=gu_p, **kw_p)
+        K.gemm_nt_swiglu(x[:M], w, gu=gu[:M], out=out[:M], any_rows=True, **kw)
+        assert torch.equal(out[:M], ref[:M]) and torch.equal(gu[:M], gu_p[:M])
+        assert bool((out[M:] == 7).all()) and bool((gu[M:] == 7).all())
+        out.fill_(7.0)
+        K.gemm_nt_swiglu(x[:M], w, out=out[:M], any_rows=True, **kw)
+        assert torch.equal(out[:M], ref[:M]) and bool((out[M:] == 7).all())
+    dy, wt = x, (torch.randn(F, Kd, device=dev) * 0.1).to(bf)
+    dgu = torch.full((P, 2 * F), 7.0, device=dev, dtype=bf)
+    K.gemm_nt_swiglu_bwd(dy[:M], wt, h[:M, :r].contiguous(), sb[:F, :r].contiguous(), gu_p[:M], dgu=dgu[:M], any_rows=True)
+    ref = K.gemm_nt_swiglu_bwd(dy, wt, h[:, :r].contiguous(), sb[:F, :r].contiguous(), gu_p)
+    assert torch.equal(dgu[:M], ref[:M]) and bool((dgu[M:] == 7).all())
+    if M % 256:
+        with pytest.raises(ValueError, match="multiples of 256"):
+            K.gemm_nt_swiglu(x[:M], w)
+
+
+@pytest.mark.parametrize("M", [64, 200, 257, 777, 2100])     # the entry point takes M (nq + 2 nk) >= 512
+@pytest.mark.parametrize("nq,nk,norm,lora", [(4, 2, True, True), (32, 8, True, False), (8, 8, False, True)])
+def test_qkv_rope_on_any_row_count(dev, M, nq, nk, norm, lora):
+    """The q|k|v projection with q/k norm + RoPE likewise: the first M rows of the padded product."""
+    torch.manual_seed(M + nq)
+    H, r, d, P = 512, 32, 128, (M + 255) // 256 * 256
+    n = (nq + 2 * nk) * d
+    x = (torch.randn(P, H, device=dev) * 0.5).bfloat16()
+    w = (torch.randn(n, H, device=dev) * 0.05).bfloat16()
+    h, b2 = (torch.randn(P, 3 * r, device=dev) * 0.3).bfloat16(), (torch.randn(n, r, device=dev) * 0.05).bfloat16()
+    segs = [(nq * d, 0), ((nq + nk) * d, r), (n, 2 * r)]
+    wq, wk = ((1 + 0.1 * torch.randn(d, device=dev)).bfloat16() if norm else None for _ in range(2))
+    pos = torch.arange(P, device=dev) % 300
+    inv = (1.0 / (1e6 ** (torch.arange(0, d, 2, dtype=torch.int64).float() / d))).to(dev)
+    cos, sin = K.rope_table(300, inv)
+    ref = K.gemm_nt_qkv_rope(x, w, nq, nk, wq, wk, pos, cos, sin, 1e-6, want_pre=True,
+                             **(dict(a2=h, b2=b2, segments=segs) if lora else {}))
+    got = K.gemm_nt_qkv_rope(x[:M], w, nq, nk, wq, wk, pos[:M], cos, sin, 1e-6, want_pre=True, any_rows=True,
+                             **(dict(a2=h[:M], b2=b2, segments=segs) if lora else {}))
+    for i, (a, b) in enumerate(zip(got, ref)):
+        if i != 3 or norm:      # rstd is written with a norm only
+            assert torch.equal(a, b[:M]), i

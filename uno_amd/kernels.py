@@ -305,16 +305,19 @@ def rope_table(P: int, inv_freq: torch.Tensor):
     return cos, sin
 
 
-def qkv_rope_fused_ok(M: int, K: int, K2: int, nq: int, nk: int, d: int, dtype) -> bool:
-    """Whether gemm_nt_qkv_rope takes this q|k|v projection (the 256 x 256 kernel's shapes)."""
-    return (dtype == torch.bfloat16 and d == 128 and M % 256 == 0 and (128 * (nq + 2 * nk)) % 256 == 0
-            and K % 64 == 0 and K2 % 32 == 0 and M * (nq + 2 * nk) >= 256 * 2)
+def qkv_rope_fused_ok(M: int, K: int, K2: int, nq: int, nk: int, d: int, dtype, any_rows: bool = False) -> bool:
+    """Whether gemm_nt_qkv_rope takes this q|k|v projection; ``any_rows``: row counts that are no
+    multiple of 256 too."""
+    return (dtype == torch.bfloat16 and d == 128 and (any_rows or M % 256 == 0) and (128 * (nq + 2 * nk)) % 256 == 0
+            and K % 64 == 0 and K2 % 32 == 0 and M * (nq + 2 * nk) >= 256 * 2
+            and (not any_rows or K2 == 0 or (nq % 2 == 0 and nk % 2 == 0)))   # the extension's segments on tiles
 
 
 def gemm_nt_qkv_rope(x, w_qkv, nq, nk, wq, wk, pos, cos_tab, sin_tab, eps, *, a2=None, b2=None, segments=None,
-                     want_rstd=True, want_pre=False):
+                     want_rstd=True, want_pre=False, any_rows=False):
     """q|k|v projection (+ LoRA extension) with q/k RMSNorm + RoPE in the GEMM epilogue (bf16, head dim
-    128). Returns (q, k, v, rstd or None, pre or None); ``pre`` = the pre-norm q/k columns in bf16."""
+    128). Returns (q, k, v, rstd or None, pre or None); ``pre`` = the pre-norm q/k columns in bf16.
+    ``any_rows`` takes any number of rows; otherwise M must be a multiple of 256."""
     _rowmajor(x, "x")
     _rowmajor(w_qkv, "w_qkv")
     M, Kd = x.shape
@@ -332,7 +335,7 @@ def gemm_nt_qkv_rope(x, w_qkv, nq, nk, wq, wk, pos, cos_tab, sin_tab, eps, *, a2
                 raise RuntimeError("gemm_nt_qkv_rope: extension segment exceeds a2 columns")
         seg_end = [s[0] for s in segs]
         seg_col = [s[1] for s in segs]
-    if not qkv_rope_fused_ok(M, Kd, K2, nq, nk, 128, x.dtype):
+    if not qkv_rope_fused_ok(M, Kd, K2, nq, nk, 128, x.dtype, any_rows):
         raise RuntimeError("gemm_nt_qkv_rope: shape outside the fused kernel")
     if pos.dtype != torch.int64 or pos.numel() != M:
         raise RuntimeError("gemm_nt_qkv_rope: pos must be int64 [M]")
@@ -349,7 +352,7 @@ def gemm_nt_qkv_rope(x, w_qkv, nq, nk, wq, wk, pos, cos_tab, sin_tab, eps, *, a2
         ev0.record()
     else:
         rec = None
-    N.call("unok_gemm_nt_qkv_rope", M, Kd, nq, nk, N.ptr(x), _ld(x), N.ptr(w_qkv), _ld(w_qkv), N.ptr(a2),
+    N.call("unok_gemm_nt_qkv_rope_any" if any_rows else "unok_gemm_nt_qkv_rope", M, Kd, nq, nk, N.ptr(x), _ld(x), N.ptr(w_qkv), _ld(w_qkv), N.ptr(a2),
            _ld(a2) if a2 is not None else 0, N.ptr(b2), _ld(b2) if b2 is not None else 0, K2, len(seg_end),
            N.int_array(seg_end), N.int_array(seg_col), N.ptr(wq), N.ptr(wk), N.ptr(pos), N.ptr(cos_tab),
            N.ptr(sin_tab), cos_tab.shape[0], float(eps), N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(rstd), N.ptr(pre),
@@ -362,10 +365,10 @@ def gemm_nt_qkv_rope(x, w_qkv, nq, nk, wq, wk, pos, cos_tab, sin_tab, eps, *, a2
 
 def gemm_nt_swiglu(a: torch.Tensor, b_interleaved: torch.Tensor, *, a2: torch.Tensor | None = None,
                    b2_interleaved: torch.Tensor | None = None, gu: torch.Tensor | None = None,
-                   out: torch.Tensor | None = None) -> torch.Tensor:
+                   out: torch.Tensor | None = None, any_rows: bool = False) -> torch.Tensor:
     """silu(gate) * up of a @ b.T (+ a2 @ b2.T) for gate/up weight rows interleaved in blocks of 64
     (``interleave_gate_up``; b2 likewise); bf16, M and the row count of b multiples of 256, K and
-    K2 = b2.shape[1] of 32. With ``gu`` ([M, rows]), also stores the product as [gate | up]."""
+    K2 = b2.shape[1] of 32 (with ``any_rows`` any M). With ``gu`` ([M, rows]), also stores the product as [gate | up]."""
     _rowmajor(a, "a")
     _rowmajor(b_interleaved, "b")
     M, K = a.shape
@@ -391,7 +394,7 @@ def gemm_nt_swiglu(a: torch.Tensor, b_interleaved: torch.Tensor, *, a2: torch.Te
         ev0.record()
     else:
         rec = None
-    N.call("unok_gemm_nt_swiglu", M, rows, K, N.ptr(a), _ld(a), N.ptr(b_interleaved), _ld(b_interleaved),
+    N.call("unok_gemm_nt_swiglu_any" if any_rows else "unok_gemm_nt_swiglu", M, rows, K, N.ptr(a), _ld(a), N.ptr(b_interleaved), _ld(b_interleaved),
            N.ptr(a2), _ld(a2) if a2 is not None else 0, N.ptr(b2_interleaved),
            _ld(b2_interleaved) if b2_interleaved is not None else 0, K2,
            N.ptr(out), _ld(out), N.ptr(gu), _ld(gu) if gu is not None else 0, N.stream())
@@ -402,9 +405,9 @@ def gemm_nt_swiglu(a: torch.Tensor, b_interleaved: torch.Tensor, *, a2: torch.Te
 
 
 def gemm_nt_swiglu_bwd(a: torch.Tensor, b: torch.Tensor, a2: torch.Tensor | None, b2: torch.Tensor | None,
-                       gu: torch.Tensor, dgu: torch.Tensor | None = None) -> torch.Tensor:
+                       gu: torch.Tensor, dgu: torch.Tensor | None = None, any_rows: bool = False) -> torch.Tensor:
     """dgu = SwiGLU backward of dS = a @ b.T (+ a2 @ b2.T) against gu = [gate | up]; dS is never
-    stored. bf16; M and F = b.shape[0] multiples of 256."""
+    stored. bf16; M (unless ``any_rows``) and F = b.shape[0] multiples of 256."""
     for t, n in ((a, "a"), (b, "b"), (gu, "gu")):
         _rowmajor(t, n)
     M, K = a.shape
@@ -426,7 +429,7 @@ def gemm_nt_swiglu_bwd(a: torch.Tensor, b: torch.Tensor, a2: torch.Tensor | None
         ev0.record()
     else:
         rec = None
-    N.call("unok_gemm_nt_swiglu_bwd", M, F, K, N.ptr(a), _ld(a), N.ptr(b), _ld(b), N.ptr(a2),
+    N.call("unok_gemm_nt_swiglu_bwd_any" if any_rows else "unok_gemm_nt_swiglu_bwd", M, F, K, N.ptr(a), _ld(a), N.ptr(b), _ld(b), N.ptr(a2),
            _ld(a2) if a2 is not None else 0, N.ptr(b2), _ld(b2) if b2 is not None else 0, K2, N.ptr(gu), _ld(gu),
            N.ptr(dgu), _ld(dgu), N.stream())
     if rec is not None:
@@ -435,9 +438,9 @@ def gemm_nt_swiglu_bwd(a: torch.Tensor, b: torch.Tensor, a2: torch.Tensor | None
     return dgu
 
 
-def swiglu_fused_ok(M: int, F: int, K: int) -> bool:
+def swiglu_fused_ok(M: int, F: int, K: int, any_rows: bool = False) -> bool:
     """Shapes the fused gate/up + SwiGLU product accepts."""
-    return M % 256 == 0 and (2 * F) % 256 == 0 and K % 64 == 0 and K > 0
+    return (any_rows or M % 256 == 0) and (2 * F) % 256 == 0 and K % 64 == 0 and K > 0
 
 
 def interleave_gate_up(w_gu: torch.Tensor, F: int) -> torch.Tensor:

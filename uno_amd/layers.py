@@ -88,10 +88,11 @@ def project_qk_v(x1, lw: LayerWeights, g: Geometry, sc: StreamContext, a2=None, 
     output, or, when the GEMM applies the norm and RoPE in its epilogue, their bf16 copy (only with
     ``for_backward``; None otherwise)."""
     K2 = b2.shape[1] if b2 is not None else 0
-    if sc.rope_cos is not None and K.qkv_rope_fused_ok(x1.shape[0], x1.shape[1], K2, g.nq, g.nk, g.d, x1.dtype):
+    if sc.rope_cos is not None and K.qkv_rope_fused_ok(x1.shape[0], x1.shape[1], K2, g.nq, g.nk, g.d, x1.dtype,
+                                                       any_rows=True):
         q, k, v, rstd, pre = K.gemm_nt_qkv_rope(x1, lw.w_qkv, g.nq, g.nk, lw.q_norm, lw.k_norm, sc.pos, sc.rope_cos,
                                                 sc.rope_sin, g.eps, a2=a2, b2=b2, segments=segments,
-                                                want_rstd=for_backward, want_pre=for_backward)
+                                                want_rstd=for_backward, want_pre=for_backward, any_rows=True)
         return pre, q, k, v, rstd
     qkv = K.gemm_nt(x1, lw.w_qkv, a2=a2, b2=b2, segments=segments, out_dtype=_qkv_dtype(x1))
     if qkv.dtype == x1.dtype:
@@ -111,8 +112,8 @@ def clean_layer(h: torch.Tensor, lw: LayerWeights, g: Geometry, sc: StreamContex
     o, _ = K.attn_fwd(q, k, v, sc.iv_clean, g.nq, g.nk, g.d)
     h1 = K.gemm_nt(o, lw.w_o, residual=h)
     x2, _ = K.rmsnorm_fwd(h1, lw.ln_post, g.eps)
-    if lw.w_gu_i is not None and x2.dtype == torch.bfloat16 and K.swiglu_fused_ok(M, g.F, g.H):
-        s = K.gemm_nt_swiglu(x2, lw.w_gu_i)      # gate/up product with SwiGLU in its epilogue
+    if lw.w_gu_i is not None and x2.dtype == torch.bfloat16 and K.swiglu_fused_ok(M, g.F, g.H, any_rows=True):
+        s = K.gemm_nt_swiglu(x2, lw.w_gu_i, any_rows=True)      # gate/up product with SwiGLU in its epilogue
     else:
         s = K.swiglu_fwd(K.gemm_nt(x2, lw.w_gu), g.F)
     h2 = K.gemm_nt(s, lw.w_d, residual=h1)
@@ -144,12 +145,13 @@ def noisy_layer_forward(h0, lw: LayerWeights, lora, li: int, g: Geometry, sc: St
     h1 = K.gemm_nt(o, lw.w_o, a2=h_o, b2=lora.sb_c(li, "o") if on("o") else None, residual=h0)
     x2, rstd2 = K.rmsnorm_fwd(h1, lw.ln_post, g.eps)
     h_gu = K.gemm_nt(x2, lora.a_c(li, "gu")) if on("gu") else None
-    fused = lw.w_gu_i is not None and x2.dtype == torch.bfloat16 and K.swiglu_fused_ok(x2.shape[0], g.F, x2.shape[1])
+    fused = (lw.w_gu_i is not None and x2.dtype == torch.bfloat16
+             and K.swiglu_fused_ok(x2.shape[0], g.F, x2.shape[1], any_rows=True))
     sb_gu_i = lora.sb_gu_i(li) if fused and on("gu") else None
     if fused and (not on("gu") or (sb_gu_i is not None and (2 * r) % 32 == 0)):
         # gate/up product with its LoRA terms, SwiGLU in the epilogue; [gate | up] kept for backward
         gu = torch.empty((x2.shape[0], 2 * g.F), device=x2.device, dtype=x2.dtype)
-        s = K.gemm_nt_swiglu(x2, lw.w_gu_i, a2=h_gu, b2_interleaved=sb_gu_i, gu=gu)
+        s = K.gemm_nt_swiglu(x2, lw.w_gu_i, a2=h_gu, b2_interleaved=sb_gu_i, gu=gu, any_rows=True)
     else:
         gu = K.gemm_nt(x2, lw.w_gu, a2=h_gu, b2=lora.sb_c(li, "gu") if on("gu") else None,
                        segments=[(g.F, 0), (2 * g.F, r)] if on("gu") else None)
@@ -228,9 +230,9 @@ class NoisyLayer(torch.autograd.Function):
         if on("d"):
             K.gemm_tn(dh2, h_d, out=gb(li, "d"), alpha=sc_l, beta=1.0)                # dB_d
         a_t_d = lora.a_t(li, "d") if on("d") else None
-        if dh2.dtype == torch.bfloat16 and M % 256 == 0 and g.F % 256 == 0 and g.H % 64 == 0 and r % 32 == 0:
+        if dh2.dtype == torch.bfloat16 and g.F % 256 == 0 and g.H % 64 == 0 and r % 32 == 0:
             # dS = dh2 W_d + g_d A_d never leaves the GEMM: its epilogue applies the SwiGLU backward
-            dgu = K.gemm_nt_swiglu_bwd(dh2, lw.w_d_t, g_d, a_t_d, gu)
+            dgu = K.gemm_nt_swiglu_bwd(dh2, lw.w_d_t, g_d, a_t_d, gu, any_rows=True)
         else:
             ds = K.gemm_nt(dh2, lw.w_d_t, a2=g_d, b2=a_t_d)                            # [M, F]
             dgu = K.swiglu_bwd(ds, gu, g.F)
