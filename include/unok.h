@@ -95,8 +95,8 @@ int unok_gemm_nt_swiglu_bwd_any(int M, int F, int K, const void* A, int64_t lda,
  * (alpha/r)-scaled LoRA B; segment i covers output columns [seg_end[i-1], seg_end[i]) and reads
  * H columns [seg_col[i], seg_col[i] + r). LA null: no LoRA (R, LB, r and the segments ignored).
  * epilogue 0: C[M,N] = y;  epilogue 1: C[M,N/2] = silu(G) (.) U of y = [G | U] (no Res), rounded as
- * y in bf16 followed by unok_swiglu_fwd. The product runs on 128 x 128 output tiles (the LA rows are
- * extra columns), each split into `splits` ranges of the K tiles (splits <= 0: chosen from the
+ * y in bf16 followed by unok_swiglu_fwd. The product runs on output tiles of 16 to 128 rows (the LA rows
+ * are extra columns), each split into `splits` ranges of the K tiles (splits <= 0: chosen from the
  * shape) so the grid fills the chip; the ranges' fp32 partial sums go through `workspace` (at
  * least unok_gemm_nt_rows_workspace() bytes, 16-byte aligned) and a second kernel adds them in
  * range order (the result does not depend on timing), forms H and applies the rank-r update and

@@ -215,3 +215,28 @@ def test_attn_split_matches_unsplit(dev):
     valid = (dst >= 0).to(dev)
     assert _rel(out[valid], ref[valid]) < 1e-2
     assert not out[~valid].any()
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64, 65, 129])
+@pytest.mark.parametrize("N,Kd,r,splits", [(68, 128, 8, 1), (132, 640, 24, 2), (196, 1152, 64, 0), (8200, 4096, 40, 0)])
+def test_rows_tiles_and_short_ranges(dev, M, N, Kd, r, splits):
+    """Every row tile (16 to 128 rows) at its edges, both column tiles (the last shape's weight takes the
+    128-column one above 32 rows), column remainders, and ranges of one K tile up, which are shorter than
+    the kernel's pipeline. One bf16 rounding of an fp32 sum is 2^-9 relative; the hidden's own rounding
+    adds as much again on the update's part."""
+    print(f"[rows tiles] M={M} N={N} K={Kd} r={r} splits={splits}", flush=True)
+    torch.manual_seed(M + N + r)
+    a = torch.randn(M, Kd, device=dev).bfloat16()
+    w = (torch.randn(N, Kd, device=dev) * 0.05).bfloat16()
+    la = (torch.randn(2 * r, Kd, device=dev) * 0.05).bfloat16()
+    lb = (torch.randn(N, r, device=dev) * 0.05).bfloat16()
+    segs = [(48, r), (N, 0)]
+    gate = torch.rand(M, device=dev) > 0.3
+    res = torch.randn(M, N, device=dev).bfloat16()
+    out = K.gemm_nt_rows(a, w, lora_a=la, lora_b=lb, segments=segs, residual=res, gate=gate, splits=splits)
+    for _ in range(3):
+        assert torch.equal(out, K.gemm_nt_rows(a, w, lora_a=la, lora_b=lb, segments=segs, residual=res, gate=gate,
+                                               splits=splits))
+    assert _rel(out, _ref(a, w, la, lb, segs, res, gate)) < 4e-3
+    plain = K.gemm_nt_rows(a, w, splits=splits)
+    assert _rel(plain, _ref(a, w)) < 4e-3

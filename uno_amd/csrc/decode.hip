@@ -4,7 +4,7 @@
 // of 16 rows): the product is a stream of the weight matrix past a small activation tile. The
 // training GEMMs tile M and N and give each workgroup the whole K walk; at 128 rows that leaves
 // a few dozen workgroups for a 4096-wide output and most of the chip idle. Here every workgroup
-// owns one 128 x 128 output tile and a contiguous range of the K tiles, so the grid is
+// owns one output tile of up to 128 rows and a contiguous range of the K tiles, so the grid is
 // (output tiles) x (K ranges) and fills all CUs while each weight element is still read once.
 //
 // The gated LoRA update y += (m (.) x A^T) (s B)^T rides along: the rows of A are extra output
@@ -14,11 +14,13 @@
 // update and the epilogue. With one K range and no LoRA the product kernel writes C itself.
 #include "common.h"
 
+#include <type_traits>
+
 namespace {
 
-// Output tile 128 x 128, K tile 128; the weight streams through RB_D + 1 register sets (RB_D tiles
-// in flight), the activation tiles through RB_D + 1 LDS stages.
-constexpr int RB_M = 128, RB_N = 128, RB_K = 128, RB_W = 4, RB_D = 3;
+// RB_K is the unit K ranges are made of, RB_W the waves of a workgroup; RB_D tiles are in flight and
+// RB_P activation fragments are read ahead.
+constexpr int RB_K = 128, RB_W = 4, RB_D = 3, RB_P = 6;
 
 struct RowsGemm {
   const bf16_t* A; int64_t lda;      // [M, K] activations
@@ -45,22 +47,31 @@ template <int N> __device__ __forceinline__ void rows_wait_vm() {
 
 // Grid: one workgroup per (K range, output column tile, output row tile), row tiles fastest so
 // that the row tiles of one weight tile run on the same XCD. Column tiles past N cover the LoRA A
-// rows. Wave w owns output columns 32 w + [0, 32) of the tile for all 128 rows: four 32x32x16 MFMA
-// accumulators, whose second operand (32 weight rows x 16 k) it loads straight from global memory
-// into registers, RB_D K tiles ahead (8 x 16 bytes per lane and tile); the 128 x 128 activation
-// tile, which all four waves read, goes to LDS by direct-to-LDS loads. A lane's eight weight
-// loads cover 128 contiguous bytes of its row (lane groups 0 / 1 take k 0-63 / 64-127), so MFMA
-// step j multiplies k = 64 g + 8 j + [0, 8) of lane group g; the activation fragments use the same
-// order. Rows beyond M and columns beyond N (R) are clamped to the last valid row and never
-// stored. The activation row r's 16-byte chunk c sits in LDS slot c ^ (r % 16).
-template <bool DIRECT>
-__global__ __launch_bounds__(RB_W * 64) void gemm_nt_rows_kernel(const RowsGemm p) {
-  constexpr int BM = RB_M, BN = RB_N, BK = RB_K, D = RB_D, AS = RB_D + 1;
+// rows. Wave w owns output columns 16 CW w + [0, 16 CW) of the tile for all 16 TM rows, as CW x TM
+// accumulators of 16x16x32 MFMAs whose first operand (16 weight rows x 32 k) it loads straight from
+// global memory into registers, RB_D K tiles ahead; consecutive loads take the two 64-byte halves
+// of the rows' 128-byte lines, so a load touches 16 lines for 64 bytes each (a 32x32x16 operand
+// touches 64 lines for 16 bytes). The 16 TM x BK activation tile, which all waves read, goes to LDS
+// by direct-to-LDS loads. Rows beyond M and columns beyond N (R) are clamped to the last valid row
+// and never stored. At most 64 KB of LDS and 256 registers leave room for two workgroups per CU, so
+// one multiplies while the other waits.
+//
+// Bound by HBM: each weight is read once. TM follows the row count, so a block of one sequence (16
+// rows) multiplies one row tile, and CW the weight (rows_narrow). Measured with cold weights, with
+// the reduction below, against 128 x 128 tiles of 32x32x16 MFMAs for every row count: 16 rows, 4096
+// -> 6144 30 -> 18.7 us, 4096 -> 24576 68 -> 49 us, 12288 -> 4096 40 -> 31 us, 4096 -> 151936 282 ->
+// 231 us (5.4 TB/s); 128 rows 37 -> 29, 84 -> 83, 47 -> 44 and 319 -> 302 us, where LDS reads and the
+// activation tiles' own traffic take their share (deeper K tiles and 8-wave workgroups gain nothing).
+template <int TM, int CW, bool DIRECT>
+__global__ __launch_bounds__(RB_W * 64, 2) void gemm_nt_rows_kernel(const RowsGemm p) {
+  constexpr int BM = 16 * TM, NW = RB_W, BN = 16 * CW * NW, BK = TM == 8 ? 64 : 128, D = RB_D, AS = RB_D + 1;
+  constexpr int KS = BK / 32;                       // MFMA k-steps per tile
   constexpr int ACH = BK / 8;                       // 16-byte chunks per activation row
-  constexpr int A_INS = BM * ACH / (RB_W * 64);     // direct-to-LDS loads per wave and tile (4 rows each)
-  constexpr int W_INS = 8;                          // weight loads per lane and tile
+  constexpr int A_RPI = 64 / ACH;                   // activation rows per direct-to-LDS load
+  constexpr int A_INS = BM / (A_RPI * NW);        // direct-to-LDS loads per wave and tile
+  constexpr int W_INS = CW * KS;                    // weight loads per lane and tile
   constexpr int LPT = A_INS + W_INS;
-  static_assert(A_INS == 8 && (D - 1) * LPT < 64, "tile shape");
+  static_assert(A_INS >= 1 && (D - 1) * LPT < 64, "tile shape");
   extern __shared__ __attribute__((aligned(16))) bf16_t smem[];
 
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -74,62 +85,93 @@ __global__ __launch_bounds__(RB_W * 64) void gemm_nt_rows_kernel(const RowsGemm 
   const int n0 = (lora_tile ? tn - nNm : tn) * BN;
   const int ncols = lora_tile ? p.R : p.N;
 
-  const int nk = p.K / BK;
-  const int kb = (int)((int64_t)split * nk / p.splits), ke = (int)((int64_t)(split + 1) * nk / p.splits);
+  const int nku = p.K / RB_K;
+  const int kb = (int)((int64_t)split * nku / p.splits) * (RB_K / BK);
+  const int ke = (int)((int64_t)(split + 1) * nku / p.splits) * (RB_K / BK);
 
-  const int arow_in = lane >> 4, aslot = lane & 15;   // direct-to-LDS lane: tile row 4 (4 i + w) + lane / 16
-  const int lg = lane >> 5;
-  const int wn = min(n0 + wid * 32 + (lane & 31), ncols - 1);
-  const bf16_t* wrow = (lora_tile ? p.LA + (int64_t)wn * p.ldla : p.B + (int64_t)wn * p.ldb) + lg * 64;
+  const int lr = lane & 15, lg = lane >> 4;
+  const int64_t ldw = lora_tile ? p.ldla : p.ldb;
+  const bf16_t* wbase = (lora_tile ? p.LA : p.B) + lg * 8;
+  const bf16_t* wrow[CW];
+#pragma unroll
+  for (int j = 0; j < CW; ++j) wrow[j] = wbase + (int64_t)min(n0 + (wid * CW + j) * 16 + lr, ncols - 1) * ldw;
 
+  // the activation row r's 16-byte chunk c sits in slot c ^ swz(r): the 16 rows one fragment read
+  // covers hit 16 different 16-byte groups of the 256-byte bank row
+  auto swz = [](int r) { return BK == 64 ? (r >> 1) & 7 : r & 15; };
+  const int arow_in = lane / ACH, aslot = lane % ACH;
   auto issue_a = [&](int t, int stage) {
     bf16_t* as = smem + stage * BM * BK;
     const int kk = t * BK;
 #pragma unroll
     for (int i = 0; i < A_INS; ++i) {
-      const int r = (i * RB_W + wid) * 4 + arow_in;
+      const int r = (i * NW + wid) * A_RPI + arow_in;
       const int gm = min(m0 + r, p.M - 1);
-      dma16(p.A + (int64_t)gm * p.lda + kk + ((aslot ^ (r & 15)) << 3), as + (i * RB_W + wid) * 4 * BK);
+      dma16(p.A + (int64_t)gm * p.lda + kk + ((aslot ^ swz(r)) << 3), as + (i * NW + wid) * A_RPI * BK);
     }
   };
   auto issue_w = [&](int t, bf16x8_t (&w)[W_INS]) {
     const int kk = t * BK;
 #pragma unroll
-    for (int j = 0; j < W_INS; ++j) w[j] = *(const bf16x8_t*)(wrow + kk + j * 8);
+    for (int j = 0; j < CW; ++j)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) w[j * KS + s] = *(const bf16x8_t*)(wrow[j] + kk + s * 32);
   };
 
-  f32x16_t acc[4];
+  f32x4_t acc[CW][TM];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int j = 0; j < CW; ++j)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
-
-  auto mfma_step = [&](const bf16_t* as, int chunk, const bf16x8_t& w) {
-    bf16x8_t a[4];
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int mi = 0; mi < 4; ++mi) {
-      const int r = mi * 32 + (lane & 31);
-      a[mi] = *(const bf16x8_t*)&as[r * BK + ((chunk ^ (r & 15)) << 3)];
-    }
-#pragma unroll
-    for (int mi = 0; mi < 4; ++mi) acc[mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[mi], w, acc[mi], 0, 0, 0);
-  };
+      for (int e = 0; e < 4; ++e) acc[j][i][e] = 0.f;
 
   // A uniform pipeline over RB_D + 1 weight register sets. Step t waits for tile t, passes the
   // barrier, issues the weight loads of tile t + RB_D, multiplies tile t and then issues the
   // activation loads of tile t + RB_D (past the end: the range's last tile again, into a free
   // stage and set). RB_D weight tiles stay in flight during the multiply, and each wait leaves
   // exactly the RB_D - 1 younger tile groups outstanding. (Activation loads issued before the
-  // multiply would make the compiler wait for them before its LDS reads.)
+  // multiply would make the compiler wait for them before its LDS reads.) The loop runs whole groups
+  // of four steps; the last n % 4 tiles, in flight already, are waited for in full: the counted wait
+  // would not hold there, because loads that no later step reads are not emitted.
   const int n = ke - kb;
   if (n > 0) {
     bf16x8_t w0[W_INS], w1[W_INS], w2[W_INS], w3[W_INS];
+    // (the empty statements keep the three tiles' loads in order, as the counted waits need)
     issue_w(kb, w0);
     issue_a(kb, 0);
+    asm volatile("" ::: "memory");
     issue_w(kb + min(1, n - 1), w1);
     issue_a(kb + min(1, n - 1), 1);
+    asm volatile("" ::: "memory");
     issue_w(kb + min(2, n - 1), w2);
     issue_a(kb + min(2, n - 1), 2);
+    auto multiply = [&](int t, const bf16x8_t (&w)[W_INS]) {
+      const bf16_t* as = smem + (t % AS) * BM * BK;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        bf16x8_t a[TM];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const int r = i * 16 + lr;
+          a[i] = *(const bf16x8_t*)&as[r * BK + (((s * 4 + lg) ^ swz(r)) << 3)];
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < CW; ++j)
+            acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j * KS + s], a[i], acc[j][i], 0, 0, 0);
+      }
+      // fragment reads run RB_P ahead of the multiplies that use them
+      constexpr int NR = KS * TM, P = NR < RB_P ? NR : RB_P;
+      __builtin_amdgcn_sched_group_barrier(SG_DS_READ, P, 0);
+#pragma unroll
+      for (int i = 0; i < NR - P; ++i) {
+        __builtin_amdgcn_sched_group_barrier(SG_MFMA, CW, 0);
+        __builtin_amdgcn_sched_group_barrier(SG_DS_READ, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(SG_MFMA, CW * P, 0);
+    };
     auto step = [&](int t, bf16x8_t (&w)[W_INS], bf16x8_t (&wnext)[W_INS]) {
       rows_wait_vm<(D - 1) * LPT>();
       // each wave waited for its own loads of tile t; after the barrier the tile is in LDS and
@@ -137,13 +179,11 @@ __global__ __launch_bounds__(RB_W * 64) void gemm_nt_rows_kernel(const RowsGemm 
       asm volatile("s_barrier" ::: "memory");
       const int tnext = kb + min(t + D, n - 1);
       issue_w(tnext, wnext);
-      const bf16_t* as = smem + (t % AS) * BM * BK;
-#pragma unroll
-      for (int j = 0; j < W_INS; ++j) mfma_step(as, lg * 8 + j, w[j]);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(t, w);
+      __builtin_amdgcn_sched_barrier(0);
       issue_a(tnext, (t + D) % AS);
     };
-    // whole groups of four steps in the loop (no conditional step before its back edge, so the
-    // compiler's own wait before each multiply counts the younger groups), the rest after it
     int t = 0;
     for (; t + 4 <= n; t += 4) {
       step(t, w0, w3);
@@ -151,49 +191,56 @@ __global__ __launch_bounds__(RB_W * 64) void gemm_nt_rows_kernel(const RowsGemm 
       step(t + 2, w2, w1);
       step(t + 3, w3, w2);
     }
-    if (t < n) step(t, w0, w3);
-    if (t + 1 < n) step(t + 1, w1, w0);
-    if (t + 2 < n) step(t + 2, w2, w1);
     rows_wait_vm<0>();
+    asm volatile("s_barrier" ::: "memory");
+    if (t < n) multiply(t, w0);
+    if (t + 1 < n) multiply(t + 1, w1);
+    if (t + 2 < n) multiply(t + 2, w2);
   }
 
-  // acc[mi][r] holds C[row 32 mi + 8 (r >> 2) + 4 lg + (r & 3)][col 32 w + lane % 32].
-  const int col = n0 + wid * 32 + (lane & 31);
-  if (col >= ncols) return;
-  const int64_t wcol = lora_tile ? (int64_t)p.N + col : col;
+  // acc[j][i] of lane l: C[row 16 i + l % 16][cols 32 w + 16 j + 4 (l / 16) + 0..3]; N and R are
+  // multiples of 4, so the four columns exist together.
 #pragma unroll
-  for (int mi = 0; mi < 4; ++mi) {
+  for (int j = 0; j < CW; ++j) {
+    const int col = n0 + (wid * CW + j) * 16 + lg * 4;
+    if (col >= ncols) continue;
+    const int64_t wcol = lora_tile ? (int64_t)p.N + col : col;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = m0 + mi * 32 + (r >> 2) * 8 + lg * 4 + (r & 3);
+    for (int i = 0; i < TM; ++i) {
+      const int row = m0 + i * 16 + lr;
       if (row >= p.M) continue;
       if constexpr (DIRECT) {
-        float v = acc[mi][r];
-        if (p.Res) v += bf16_to_f32(p.Res[(int64_t)row * p.ldres + col]);
-        p.C[(int64_t)row * p.ldc + col] = f32_to_bf16(v);
+        f32x4_t v = acc[j][i];
+        if (p.Res) {
+          const uint2 u = *(const uint2*)(p.Res + (int64_t)row * p.ldres + col);
+          v[0] += __uint_as_float(u.x << 16); v[1] += __uint_as_float(u.x & 0xffff0000u);
+          v[2] += __uint_as_float(u.y << 16); v[3] += __uint_as_float(u.y & 0xffff0000u);
+        }
+        *(uint2*)(p.C + (int64_t)row * p.ldc + col) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
       } else {
-        p.ws[((int64_t)split * p.M + row) * p.ldw + wcol] = acc[mi][r];
+        *(f32x4_t*)(p.ws + ((int64_t)split * p.M + row) * p.ldw + wcol) = acc[j][i];
       }
     }
   }
 }
 
 // ---------------------------------------------------------------------------------------
-// Reduction with the rank-r LoRA update and the epilogue. Workgroup tile: 16 rows x 128 product
-// columns ("slots"; EPI 0) or 16 rows x 64 SwiGLU features, i.e. the 64 gate and the 64 matching up
-// columns (EPI 1).
-//   1. h = bf16(m (.) sum of the LoRA-column partials) for the tile's rows (all R columns) into
-//      LDS, and the slots' (s B) rows into LDS;
-//   2. the rank-r update u[row, slot] = h[row, seg(slot) + :r] . (s B)[slot, :r] with 16x16x32
-//      MFMAs (each wave two 16-slot tiles), fp32 into LDS;
-//   3. every thread adds the partials of 4 columns (and 4 up columns) of its rows in range order,
-//      then u, the residual, and rounds:
+// Reduction with the rank-r LoRA update and the epilogue. Workgroup tile: 16 rows x 64 columns
+// (EPI 0) or 16 rows x 64 SwiGLU features, i.e. 64 gate and the 64 matching up columns (EPI 1);
+// wave w takes columns 16 w + [0, 16) of them.
+//   1. every lane starts the loads of its own partials (row l % 16, columns 4 (l / 16) + 0..3 of the
+//      wave's) and of its (s B) fragments, so that their latency passes behind step 2;
+//   2. h = bf16(m (.) sum of the LoRA-column partials, in range order) of the tile's rows, the hidden
+//      columns that its segments read, into LDS;
+//   3. the rank-r update h (s B)^T with 16x16x32 MFMAs, whose result lies in exactly the lanes of
+//      step 1, then the partials in range order, the update and the residual, rounded once:
 // EPI 0: C[M, N]   = bf16(sum + u + Res);
 // EPI 1: C[M, N/2] = bf16(silu(g) * u), g = bf16(gate column value), u = bf16(up column value)
 //        (the [gate | up] product rounded to bf16 and then the SwiGLU of unok_swiglu_fwd).
-// Segment boundaries are multiples of 16, so each 16-slot tile reads one segment of h.
+// Segment boundaries are multiples of 16, so each wave's 16 columns read one segment of h.
+// Bound by latency: one pass of loads, one barrier.
 // ---------------------------------------------------------------------------------------
-constexpr int RR_ROWS = 16, RR_SLOTS = 128, RR_ULD = RR_SLOTS + 4;
+constexpr int RR_ROWS = 16, RR_COLS = 64, RR_HMAX = 512;
 
 struct RowsReduce {
   const float* ws; int64_t ldw; int splits;
@@ -213,160 +260,165 @@ __device__ __forceinline__ int red_seg_col(const RowsReduce& p, int n) {
   return c;
 }
 
-__device__ __forceinline__ int round32(int x) { return (x + 31) & ~31; }
+// Sum of the ranges' partials at src (range stride `plane` floats), in range order; the first eight
+// ranges' values are in v already.
+__device__ __forceinline__ f32x4_t sum_ranges(const float* src, int64_t plane, int splits, const f32x4_t (&v)[8]) {
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    if (q < splits) acc += v[q];
+  for (int k0 = 8; k0 < splits; k0 += 8) {
+    f32x4_t w[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (k0 + q < splits) w[q] = *(const f32x4_t*)(src + (k0 + q) * plane);
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (k0 + q < splits) acc += w[q];
+  }
+  return acc;
+}
 
 template <int EPI>
 __global__ __launch_bounds__(256) void rows_reduce_kernel(const RowsReduce p) {
-  constexpr int NH = EPI == 1 ? 2 : 1;             // column groups per thread: (gate, up) or one
-  constexpr int NG = RR_SLOTS / (4 * NH);          // column groups of 4 per workgroup row: 32 / 16
-  constexpr int RPT = RR_ROWS * NG / 256;          // rows per thread: 2 (EPI 0) or 1 (EPI 1)
-  extern __shared__ __attribute__((aligned(16))) float rsm[];
+  constexpr int NH = EPI == 1 ? 2 : 1;             // column groups per lane: (gate, up) or one
+  __shared__ __attribute__((aligned(16))) bf16_t Hs[RR_ROWS * (RR_HMAX + 40)];
   const bool lora = p.LB != nullptr;
-  const int rp = round32(p.r);
-  const int hld = p.R + 32;                        // bf16 row stride of h (zero tail read by the last steps)
-  const int rld = rp + 8;                          // bf16 row stride of the staged (s B) rows
-  float* Us = rsm;                                                   // [RR_ROWS][RR_ULD] fp32
-  bf16_t* Hs = (bf16_t*)(rsm + RR_ROWS * RR_ULD);                    // [RR_ROWS][hld]
-  bf16_t* Ls = Hs + RR_ROWS * hld;                                   // [RR_SLOTS][rld]
-
   const int nout = EPI == 1 ? p.N / 2 : p.N;
-  const int ctiles = (nout + NG * 4 - 1) / (NG * 4);
+  const int ctiles = (nout + RR_COLS - 1) / RR_COLS;
   const int r0 = (blockIdx.x / ctiles) * RR_ROWS;
-  const int c0 = (blockIdx.x % ctiles) * NG * 4;
+  const int c0 = (blockIdx.x % ctiles) * RR_COLS;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int lr = lane & 15, lg = lane >> 4;
   const int64_t plane = (int64_t)p.M * p.ldw;
 
-  // product column of slot q of this tile: EPI 0: c0 + q; EPI 1: gate c0 + q for q < 64, up
-  // N/2 + c0 + q - 64 above
-  auto slot_col = [&](int q) {
-    if constexpr (EPI == 1) return q < NG * 4 ? c0 + q : nout + c0 + (q - NG * 4);
-    else return c0 + q;
-  };
-  if (lora) {
-    // h: four (row, column) items per thread at a time, each with up to eight ranges' loads in flight
-    const int items = RR_ROWS * p.R;
-    for (int i0 = tid; i0 < items; i0 += 4 * 256) {
-      float acc[4] = {0.f, 0.f, 0.f, 0.f};
-      const float* src[4];
+  // 1. own partials (clamped to existing rows and columns)
+  const int cbase = c0 + wid * 16 + lg * 4;
+  const int row = r0 + lr, lrow = min(row, p.M - 1);
+  const float* src[NH];
+  f32x4_t v[NH][8];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int i = min(i0 + u * 256, items - 1);
-        const int row = min(r0 + i / p.R, p.M - 1);
-        src[u] = p.ws + (int64_t)row * p.ldw + p.N + i % p.R;
-      }
-      for (int k0 = 0; k0 < p.splits; k0 += 8) {
-        float v[4][8];
+  for (int h = 0; h < NH; ++h) {
+    src[h] = p.ws + (int64_t)lrow * p.ldw + min(cbase, nout - 4) + h * nout;
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int q = 0; q < 8; ++q) v[u][q] = k0 + q < p.splits ? src[u][(k0 + q) * plane] : 0.f;
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int q = 0; q < 8; ++q)
-            if (k0 + q < p.splits) acc[u] += v[u][q];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int i = i0 + u * 256;
-        if (i >= items) break;
-        const int rr = i / p.R, j = i % p.R;
-        const int row = min(r0 + rr, p.M - 1);
-        const bool on = p.gate == nullptr || p.gate[row] != 0;
-        Hs[rr * hld + j] = on ? f32_to_bf16(acc[u]) : (bf16_t)0;
-      }
-    }
-    for (int i = tid; i < RR_ROWS * 32; i += 256) Hs[(i / 32) * hld + p.R + i % 32] = 0;
-    const int vec = p.r / 8;
-    for (int i = tid; i < RR_SLOTS * vec; i += 256) {
-      const int q = i / vec, v = i % vec;
-      const int colq = min(slot_col(q), p.N - 1);
-      *(uint4*)(Ls + q * rld + v * 8) = *(const uint4*)(p.LB + (int64_t)colq * p.ldlb + v * 8);
-    }
-    __syncthreads();
-    // rank-r update on MFMA: wave w takes slot tiles 2 w and 2 w + 1; lane l supplies (s B) of slot
-    // l % 16 and h of row l % 16 at k = 32 kk + 8 (l / 16) + [0, 8); the result of slot
-    // 4 (l / 16) + e, row l % 16 is D element e of lane l
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-      const int s0 = (wid * 2 + tt) * 16;
-      const int hc = red_seg_col(p, slot_col(s0));
-      f32x4_t d = {0.f, 0.f, 0.f, 0.f};
-      for (int kk = 0; kk < rp; kk += 32) {
-        const int k = kk + 8 * (lane >> 4);
-        bf16x8_t lb = *(const bf16x8_t*)(Ls + (s0 + (lane & 15)) * rld + k);
-        if (k >= p.r) lb = __builtin_bit_cast(bf16x8_t, make_uint4(0, 0, 0, 0));
-        const bf16x8_t hv = *(const bf16x8_t*)(Hs + (lane & 15) * hld + hc + k);
-        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lb, hv, d, 0, 0, 0);
-      }
-      *(f32x4_t*)(Us + (lane & 15) * RR_ULD + s0 + 4 * (lane >> 4)) = d;
-    }
-    __syncthreads();
+    for (int q = 0; q < 8; ++q)
+      if (q < p.splits) v[h][q] = *(const f32x4_t*)(src[h] + q * plane);
   }
-
-  const int cg = tid % NG, rg = tid / NG;
-  const int cbase = c0 + cg * 4;
-  if (cbase >= nout) return;
-  // partial sums: all rows and column groups of this thread, up to eight ranges in flight each,
-  // added in range order
-  float4 acc[RPT][NH];
-  const float4* src[RPT][NH];
+  uint2 rv = make_uint2(0, 0);
+  if (EPI == 0 && p.Res) rv = *(const uint2*)(p.Res + (int64_t)lrow * p.ldres + min(cbase, nout - 4));
+  f32x4_t u[NH];
 #pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-    const int row = min(r0 + rg * RPT + i, p.M - 1);
+  for (int h = 0; h < NH; ++h) u[h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if (lora) {
+    const int wcol = min(c0 + wid * 16, nout - 1);   // first column of the wave's 16
+    uint4 lb[NH][4];
 #pragma unroll
     for (int h = 0; h < NH; ++h) {
-      acc[i][h] = make_float4(0.f, 0.f, 0.f, 0.f);
-      src[i][h] = (const float4*)(p.ws + (int64_t)row * p.ldw + cbase + h * nout);
-    }
-  }
-  const int64_t plane4 = plane / 4;
-  for (int k0 = 0; k0 < p.splits; k0 += 8) {
-    float4 v[RPT][NH][8];
+      const bf16_t* lrow_b = p.LB + (int64_t)(min(c0 + wid * 16 + lr, nout - 1) + h * nout) * p.ldlb;
 #pragma unroll
-    for (int i = 0; i < RPT; ++i)
-#pragma unroll
-      for (int h = 0; h < NH; ++h)
-#pragma unroll
-        for (int q = 0; q < 8; ++q)
-          v[i][h][q] = k0 + q < p.splits ? src[i][h][(k0 + q) * plane4] : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-    for (int i = 0; i < RPT; ++i)
-#pragma unroll
-      for (int h = 0; h < NH; ++h)
-#pragma unroll
-        for (int q = 0; q < 8; ++q)
-          if (k0 + q < p.splits) acc[i][h] += v[i][h][q];
-  }
-  if (lora) {
-#pragma unroll
-    for (int i = 0; i < RPT; ++i)
-#pragma unroll
-      for (int h = 0; h < NH; ++h) acc[i][h] += *(const float4*)(Us + (rg * RPT + i) * RR_ULD + h * NG * 4 + cg * 4);
-  }
-#pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-    const int row = r0 + rg * RPT + i;
-    if (row >= p.M) continue;
-    const float a[4] = {acc[i][0].x, acc[i][0].y, acc[i][0].z, acc[i][0].w};
-    float o[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      if constexpr (EPI == 0) {
-        float v = a[c];
-        if (p.Res) v += bf16_to_f32(p.Res[(int64_t)row * p.ldres + cbase + c]);
-        o[c] = v;
-      } else {
-        const float b[4] = {acc[i][NH - 1].x, acc[i][NH - 1].y, acc[i][NH - 1].z, acc[i][NH - 1].w};
-        const float g = Elem<bf16_t>::round(a[c]);
-        const float u = Elem<bf16_t>::round(b[c]);
-        o[c] = g * sigmoidf_(g) * u;
+      for (int kk = 0; kk < 4; ++kk) {
+        const int k = kk * 32 + 8 * lg;
+        lb[h][kk] = k < p.r ? *(const uint4*)(lrow_b + k) : make_uint4(0, 0, 0, 0);
       }
     }
-    uint2 packed;
-    packed.x = pack2_bf16(o[0], o[1]);
-    packed.y = pack2_bf16(o[2], o[3]);
-    *(uint2*)(p.C + (int64_t)row * p.ldc + cbase) = packed;
+    // 2. the hidden columns [h0, h1) that this tile's segments read
+    int h0 = p.R, h1 = 0;
+#pragma unroll
+    for (int t = 0; t < RR_COLS / 16; ++t)
+#pragma unroll
+      for (int h = 0; h < NH; ++h) {
+        const int c = red_seg_col(p, min(c0 + t * 16, nout - 1) + h * nout);
+        h0 = min(h0, c);
+        h1 = max(h1, c + p.r);
+      }
+    h0 &= ~7;
+    const int hw4 = (h1 - h0 + 3) / 4;             // columns in fours (R is a multiple of 8)
+    const int hld = ((h1 - h0 + 31) & ~31) + 40;   // bf16 row stride: a zero tail of 32 or more, rows spread over banks
+    for (int i = tid; i < RR_ROWS * hw4; i += 256) {
+      const int rr = i / hw4, j = (i % hw4) * 4;
+      const int hrow = min(r0 + rr, p.M - 1);
+      const float* hs = p.ws + (int64_t)hrow * p.ldw + p.N + h0 + j;
+      f32x4_t x[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (q < p.splits) x[q] = *(const f32x4_t*)(hs + q * plane);
+      const f32x4_t a = sum_ranges(hs, plane, p.splits, x);
+      const bool on = p.gate == nullptr || p.gate[hrow] != 0;
+      *(uint2*)(Hs + rr * hld + j) = on ? make_uint2(pack2_bf16(a[0], a[1]), pack2_bf16(a[2], a[3])) : make_uint2(0, 0);
+    }
+    for (int i = tid; i < RR_ROWS * 16; i += 256) *(uint32_t*)(Hs + (i / 16) * hld + hw4 * 4 + (i % 16) * 2) = 0;
+    __syncthreads();
+    // 3. lane l supplies (s B) of column l % 16 and h of row l % 16 at k = 32 kk + 8 (l / 16) + [0, 8);
+    // D element e of lane l is row l % 16, column 4 (l / 16) + e
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+      const bf16_t* hrow = Hs + lr * hld + red_seg_col(p, wcol + h * nout) - h0;
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        if (kk * 32 >= p.r) break;
+        const bf16x8_t hv = *(const bf16x8_t*)(hrow + kk * 32 + 8 * lg);
+        u[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, lb[h][kk]), hv, u[h], 0, 0, 0);
+      }
+    }
+  }
+
+  if (cbase >= nout || row >= p.M) return;
+  float o[4];
+  if constexpr (EPI == 0) {
+    f32x4_t a = sum_ranges(src[0], plane, p.splits, v[0]) + u[0];
+    if (p.Res) {
+      a[0] += __uint_as_float(rv.x << 16); a[1] += __uint_as_float(rv.x & 0xffff0000u);
+      a[2] += __uint_as_float(rv.y << 16); a[3] += __uint_as_float(rv.y & 0xffff0000u);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o[c] = a[c];
+  } else {
+    const f32x4_t a = sum_ranges(src[0], plane, p.splits, v[0]) + u[0];
+    const f32x4_t b = sum_ranges(src[NH - 1], plane, p.splits, v[NH - 1]) + u[NH - 1];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float g = Elem<bf16_t>::round(a[c]);
+      const float w = Elem<bf16_t>::round(b[c]);
+      o[c] = g * sigmoidf_(g) * w;
+    }
+  }
+  *(uint2*)(p.C + (int64_t)row * p.ldc + cbase) = make_uint2(pack2_bf16(o[0], o[1]), pack2_bf16(o[2], o[3]));
+}
+
+// Row tile of the product in 16-row units.
+int rows_tm(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : 8; }
+
+// Column tile: 64 columns (one MFMA column per wave) put twice the workgroups in flight, 128 read the
+// activation tile half as often. With few rows the activations are small next to the weights; with
+// more, 64 columns pay only while the weight is small enough for the launch, not the traffic, to
+// bound it (64 against 128 columns: 16 rows 4096 -> 24576 49 / 58 us; 32 rows 53 / 57, and 4096 ->
+// 151936 245 / 240; 128 rows 4096 -> 4096 21 / 23 us, 12288 -> 4096 47 / 44 us).
+bool rows_narrow(int M, int N, int K) {
+  return M <= 16 || (int64_t)N * K <= (M <= 32 ? 1ll << 27 : 1ll << 25);
+}
+
+int64_t rows_tiles(int M, int N, int K, int R) {
+  const int bm = rows_tm(M) * 16, bn = rows_narrow(M, N, K) ? 16 * RB_W : 32 * RB_W;
+  return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn + (R + bn - 1) / bn);
+}
+
+template <bool DIRECT>
+void launch_rows(const RowsGemm& p, unsigned nb, hipStream_t st) {
+  auto go = [&](auto tm, auto cw) {
+    constexpr int TM = decltype(tm)::value, CW = decltype(cw)::value;
+    constexpr size_t lds = (size_t)(RB_D + 1) * 16 * TM * (TM == 8 ? 64 : 128) * sizeof(bf16_t);
+    UNOK_SET_LDS_ONCE((gemm_nt_rows_kernel<TM, CW, DIRECT>), lds);
+    hipLaunchKernelGGL((gemm_nt_rows_kernel<TM, CW, DIRECT>), dim3(nb), dim3(RB_W * 64), lds, st, p);
+  };
+  auto by_width = [&](auto tm) {
+    if (rows_narrow(p.M, p.N, p.K)) go(tm, std::integral_constant<int, 1>{});
+    else if constexpr (decltype(tm)::value > 1) go(tm, std::integral_constant<int, 2>{});
+  };
+  switch (rows_tm(p.M)) {
+    case 1: by_width(std::integral_constant<int, 1>{}); break;
+    case 2: by_width(std::integral_constant<int, 2>{}); break;
+    case 4: by_width(std::integral_constant<int, 4>{}); break;
+    default: by_width(std::integral_constant<int, 8>{});
   }
 }
 
@@ -375,8 +427,9 @@ __global__ __launch_bounds__(256) void rows_reduce_kernel(const RowsReduce p) {
 // longest range plus two for the pipeline fill), the partial-sum traffic (written and read once,
 // priced at half a weight tile step per 32 KB per CU because it stays in the on-chip caches for
 // these sizes) and the reduction's serial loads (a quarter step per range).
-int rows_auto_splits(int M, int N, int R, int nk, bool need_ws) {
-  const int64_t tiles = (int64_t)((M + RB_M - 1) / RB_M) * ((N + RB_N - 1) / RB_N + (R + RB_N - 1) / RB_N);
+int rows_auto_splits(int M, int N, int K, int R, bool need_ws) {
+  const int64_t tiles = rows_tiles(M, N, K, R);
+  const int nk = K >= RB_K ? K / RB_K : 1;
   int best = 1;
   double best_t = 1e30;
   const int smax = nk < 64 ? nk : 64;
@@ -392,13 +445,6 @@ int rows_auto_splits(int M, int N, int R, int nk, bool need_ws) {
 }
 
 bool rows_needs_ws(int epilogue, int R, int splits) { return splits > 1 || epilogue != 0 || R > 0; }
-
-size_t rows_reduce_lds(int R, int r) {
-  if (R == 0) return 0;
-  const int rp = (r + 31) & ~31;
-  return (size_t)RR_ROWS * RR_ULD * sizeof(float) + (size_t)RR_ROWS * (R + 32) * sizeof(bf16_t) +
-         (size_t)RR_SLOTS * (rp + 8) * sizeof(bf16_t);
-}
 
 // ---------------------------------------------------------------------------------------
 // Attention of a draft block over the KV cache, in three kernels per layer:
@@ -537,8 +583,7 @@ __global__ __launch_bounds__(256) void attn_split_combine_kernel(const bf16_t* _
 // automatic count).
 UNOK_EXPORT int64_t unok_gemm_nt_rows_workspace(int M, int N, int K, int R, int epilogue, int splits) {
   if (M <= 0 || N <= 0 || K <= 0 || R < 0) return 0;
-  const int nk = K / RB_K;
-  const int s = splits > 0 ? splits : rows_auto_splits(M, N, R, nk > 0 ? nk : 1, epilogue != 0 || R > 0);
+  const int s = splits > 0 ? splits : rows_auto_splits(M, N, K, R, epilogue != 0 || R > 0);
   if (!rows_needs_ws(epilogue, R, s)) return 0;
   return (int64_t)s * M * (N + R) * (int64_t)sizeof(float);
 }
@@ -593,7 +638,7 @@ UNOK_EXPORT int unok_gemm_nt_rows(int M, int N, int K, const void* A, int64_t ld
     R = 0;
   }
   const int nk = K / RB_K;
-  const int s = splits > 0 ? splits : rows_auto_splits(M, N, R, nk, epilogue != 0 || lora);
+  const int s = splits > 0 ? splits : rows_auto_splits(M, N, K, R, epilogue != 0 || lora);
   UNOK_REQUIRE(s <= nk, UNOK_EINVAL, "gemm_nt_rows: %d K ranges for %d K tiles", s, nk);
 
   RowsGemm p{};
@@ -602,15 +647,12 @@ UNOK_EXPORT int unok_gemm_nt_rows(int M, int N, int K, const void* A, int64_t ld
   p.LA = lora ? (const bf16_t*)LA : nullptr; p.ldla = ldla;
   p.M = M; p.N = N; p.K = K; p.R = R;
   p.splits = s;
-  const int64_t ntiles = (int64_t)((N + RB_N - 1) / RB_N) + (lora ? (R + RB_N - 1) / RB_N : 0);
-  const int64_t nb = (int64_t)((M + RB_M - 1) / RB_M) * ntiles * s;
+  const int64_t nb = rows_tiles(M, N, K, R) * s;
   UNOK_REQUIRE(nb < (1ll << 31), UNOK_EINVAL, "gemm_nt_rows: grid too large");
-  constexpr size_t lds = (size_t)(RB_D + 1) * RB_M * RB_K * sizeof(bf16_t);
   hipStream_t st = (hipStream_t)stream;
   if (!rows_needs_ws(epilogue, R, s)) {
     p.C = (bf16_t*)C; p.ldc = ldc; p.Res = (const bf16_t*)Res; p.ldres = ldres;
-    UNOK_SET_LDS_ONCE((gemm_nt_rows_kernel<true>), lds);
-    hipLaunchKernelGGL((gemm_nt_rows_kernel<true>), dim3((unsigned)nb), dim3(RB_W * 64), lds, st, p);
+    launch_rows<true>(p, (unsigned)nb, st);
     return unok::check_launch("gemm_nt_rows");
   }
   const int64_t need = (int64_t)s * M * (N + R) * (int64_t)sizeof(float);
@@ -618,8 +660,7 @@ UNOK_EXPORT int unok_gemm_nt_rows(int M, int N, int K, const void* A, int64_t ld
                "gemm_nt_rows: workspace of %lld bytes (16-byte aligned) required, got %lld", (long long)need,
                (long long)ws_bytes);
   p.ws = (float*)workspace; p.ldw = N + R;
-  UNOK_SET_LDS_ONCE((gemm_nt_rows_kernel<false>), lds);
-  hipLaunchKernelGGL((gemm_nt_rows_kernel<false>), dim3((unsigned)nb), dim3(RB_W * 64), lds, st, p);
+  launch_rows<false>(p, (unsigned)nb, st);
   int rc = unok::check_launch("gemm_nt_rows");
   if (rc) return rc;
 
@@ -630,16 +671,11 @@ UNOK_EXPORT int unok_gemm_nt_rows(int M, int N, int K, const void* A, int64_t ld
   q.Res = (const bf16_t*)Res; q.ldres = ldres;
   q.C = (bf16_t*)C; q.ldc = ldc;
   const int nout = epilogue == 1 ? N / 2 : N;
-  const int cw = epilogue == 1 ? RR_SLOTS / 2 : RR_SLOTS;
-  const int64_t blocks = (int64_t)((M + RR_ROWS - 1) / RR_ROWS) * ((nout + cw - 1) / cw);
-  const size_t rlds = rows_reduce_lds(R, q.r);
-  if (epilogue == 0) {
-    UNOK_SET_LDS_ONCE((rows_reduce_kernel<0>), 96 * 1024);
-    hipLaunchKernelGGL((rows_reduce_kernel<0>), dim3((unsigned)blocks), dim3(256), rlds, st, q);
-  } else {
-    UNOK_SET_LDS_ONCE((rows_reduce_kernel<1>), 96 * 1024);
-    hipLaunchKernelGGL((rows_reduce_kernel<1>), dim3((unsigned)blocks), dim3(256), rlds, st, q);
-  }
+  const int64_t blocks = (int64_t)((M + RR_ROWS - 1) / RR_ROWS) * ((nout + RR_COLS - 1) / RR_COLS);
+  if (epilogue == 0)
+    hipLaunchKernelGGL((rows_reduce_kernel<0>), dim3((unsigned)blocks), dim3(256), 0, st, q);
+  else
+    hipLaunchKernelGGL((rows_reduce_kernel<1>), dim3((unsigned)blocks), dim3(256), 0, st, q);
   return unok::check_launch("gemm_nt_rows_reduce");
 }
 
