@@ -259,6 +259,36 @@ int unok_attn_fwd_split(int QR, int S, int D, const void* Q, int64_t ldq, const 
 int unok_attn_split_combine(int QR, int S, int D, const void* opart, int64_t ldp, const float* lse,
                             const int32_t* dst, void* out, int64_t ldo, void* stream);
 
+/* Key intervals ivs [S * QR, 8] and output rows dst [QR] of a draft block's split-key attention from
+ * the committed lengths (QR = 128 B nk): range s of decode row i holds keys [s c, (s + 1) c) of its
+ * causal prefix over cache and block, c = lengths[b] / S, the last range the rest; rows past rep * L
+ * of each 128 are empty with dst -1, the others go to row (b L + t) nq + head. The cached lengths
+ * and block tables of nano_vllm_uno/layers/attention.py:628-668. */
+int unok_decode_maps(int B, int L, int nq, int nk, int max_len, int S, const int64_t* lengths, int32_t* ivs,
+                     int32_t* dst, void* stream);
+/* One decoder layer of a draft block [B, L] (bf16) over its KV cache: norm, q|k|v, unok_decode_prep,
+ * unok_attn_fwd_split over S ranges, unok_attn_split_combine, o, norm, gate|up with SwiGLU, down, the
+ * linears as unok_gemm_nt_rows with the gated LoRA and the residuals. h and h_out [B L, H] may not
+ * overlap. a_* / b_*: LoRA A rows and scaled B of the fused groups, rank r. scratch: at least
+ * unok_draft_layer_scratch() bytes, 256-byte aligned. Replaces: Qwen3DecoderLayer.forward of a draft
+ * block (nano_vllm_uno/models/qwen3.py:81-132, engine/two_pass_decoding.py:273-283). */
+typedef struct unok_draft_layer_args {
+  int B, L, nq, nk, D, H, F, r, S, max_len;
+  float eps, scale;
+  const void *ln_in, *ln_post, *q_norm, *k_norm;
+  const void *w_qkv, *a_qkv, *b_qkv, *w_o, *a_o, *b_o, *w_gu, *a_gu, *b_gu, *w_d, *a_d, *b_d;
+  void *kc, *vc;
+  const int64_t* lengths;
+  const float* inv_freq;
+  const uint8_t* gate;
+  const int32_t *ivs, *dst;
+  const void* h;
+  void *h_out, *scratch;
+  int64_t scratch_bytes;
+} unok_draft_layer_args;
+int64_t unok_draft_layer_scratch(const unok_draft_layer_args* args);
+int unok_draft_layer(const unok_draft_layer_args* args, void* stream);
+
 /* ---- Block-diffusion batch preparation ----------------------------------------------------- */
 
 /* Noising, [noisy | clean] concatenation, stream maps and interval tables of one batch.

@@ -88,6 +88,8 @@ BAD_CALLS = [
     ("unok_attn_fwd", dict(a0=7, a1=128, a2=1, a3=1, a4=128), -1, "dtype"),
     ("unok_attn_fwd_split", dict(a0=128, a1=0), -1, "S=0"),
     ("unok_decode_prep", dict(a0=1, a1=1, a2=3, a3=2), -1, "nq=3 nk=2"),
+    ("unok_decode_maps", dict(a0=1, a1=1, a2=2, a3=2, a5=0), -1, "S=0"),
+    ("unok_draft_layer", {}, -1, "bad sizes"),
     ("unok_bd_prepare", dict(a0=-1), -1, "negative shape"),
     ("unok_lmhead_ce_stats", dict(a0=1, a1=256, a2=64, a4=64, a6=64, a11=1), -1, "blocks"),
     ("unok_ce_parts_reduce", dict(a0=1, a1=0), -1, "bad sizes"),

@@ -240,3 +240,48 @@ def test_rows_tiles_and_short_ranges(dev, M, N, Kd, r, splits):
     assert _rel(out, _ref(a, w, la, lb, segs, res, gate)) < 4e-3
     plain = K.gemm_nt_rows(a, w, splits=splits)
     assert _rel(plain, _ref(a, w)) < 4e-3
+
+
+@pytest.mark.parametrize("B,L,nq,nk,max_len,S", [(1, 1, 4, 4, 33, 1), (3, 5, 16, 8, 70, 8), (2, 32, 4, 1, 4096, 3)])
+def test_decode_maps(dev, B, L, nq, nk, max_len, S):
+    """Every key of a query's causal prefix lies in exactly one range, ranges follow each other, padding
+    rows are empty, and the output rows are a permutation of the block's (row, head) pairs."""
+    torch.manual_seed(B + L)
+    lengths = torch.randint(0, max_len - L + 1, (B,), device=dev)
+    lengths[0] = 0
+    ivs, dst = K.decode_maps(lengths, B, L, nq, nk, max_len, S)
+    QR, rep = B * nk * 128, nq // nk
+    iv = ivs.view(S, QR, 8).cpu()
+    d = dst.cpu()
+    assert sorted(d[d >= 0].tolist()) == list(range(B * L * nq))
+    for q in range(QR):
+        pair, slot = q // 128, q % 128
+        if slot >= rep * L:
+            assert d[q] == -1 and bool((iv[:, q, 0] == iv[:, q, 1]).all())
+            continue
+        b, kv, t, r = pair // nk, pair % nk, slot % L, slot // L
+        assert d[q] == (b * L + t) * nq + kv * rep + r
+        at = pair * max_len
+        for s in range(S):
+            lo, hi = int(iv[s, q, 0]), int(iv[s, q, 1])
+            if hi > lo:
+                assert lo == at
+                at = hi
+        assert at == pair * max_len + int(lengths[b]) + t + 1
+    assert bool((iv[..., 2:] == 0).all())
+
+
+@pytest.mark.parametrize("S", [1, 3, 8, 11])
+def test_split_combine_range_counts(dev, S):
+    """Merges of one range up to past the eight that are in flight together, with empty ranges."""
+    torch.manual_seed(S)
+    QR, D = 256, 128
+    o = torch.randn(S * QR, D, device=dev).bfloat16()
+    lse = torch.randn(S, QR, device=dev) * 4
+    lse[torch.rand(S, QR, device=dev) < 0.3] = float("-inf")
+    dst = torch.randperm(QR, device=dev).to(torch.int32)
+    out = torch.zeros(QR, D, device=dev, dtype=torch.bfloat16)
+    K.attn_split_combine(o, lse.reshape(-1).contiguous(), dst, QR, S, D, out)
+    w = torch.exp2(lse.double() - lse.double().amax(0).clamp_min(-1e30))
+    ref = (w[..., None] * o.view(S, QR, D).double()).sum(0) / w.sum(0).clamp_min(1e-30)[:, None]
+    assert _rel(out[dst.long()], ref) < 2.0 ** -8      # one bf16 rounding

@@ -20,6 +20,17 @@ _i, _i64, _p, _f = C.c_int, C.c_int64, C.c_void_p, C.c_float
 _u64 = C.c_uint64
 _ip = C.POINTER(C.c_int)
 
+
+class DraftLayerArgs(C.Structure):
+    """unok_draft_layer_args of include/unok.h."""
+    _fields_ = ([(n, _i) for n in ("B", "L", "nq", "nk", "D", "H", "F", "r", "S", "max_len")]
+                + [(n, _f) for n in ("eps", "scale")]
+                + [(n, _p) for n in ("ln_in", "ln_post", "q_norm", "k_norm", "w_qkv", "a_qkv", "b_qkv", "w_o", "a_o", "b_o",
+                                     "w_gu", "a_gu", "b_gu", "w_d", "a_d", "b_d", "kc", "vc", "lengths", "inv_freq", "gate",
+                                     "ivs", "dst", "h", "h_out", "scratch")]
+                + [("scratch_bytes", _i64)])
+
+
 # name -> (restype, argtypes); must match include/unok.h exactly.
 SIGNATURES: dict[str, tuple] = {
     "unok_abi_version": (_i, []),
@@ -53,6 +64,9 @@ SIGNATURES: dict[str, tuple] = {
                            _p, _p, _i64, _p, _f, _p]),
     "unok_attn_fwd_split": (_i, [_i, _i, _i, _p, _i64, _p, _i64, _p, _i64, _p, _p, _i64, _p, _f, _p]),
     "unok_attn_split_combine": (_i, [_i, _i, _i, _p, _i64, _p, _p, _p, _i64, _p]),
+    "unok_decode_maps": (_i, [_i, _i, _i, _i, _i, _i, _p, _p, _p, _p]),
+    "unok_draft_layer_scratch": (_i64, [C.POINTER(DraftLayerArgs)]),
+    "unok_draft_layer": (_i, [C.POINTER(DraftLayerArgs), _p]),
     "unok_decode_prep": (_i, [_i, _i, _i, _i, _i, _p, _i64, _p, _p, _p, _p, _f, _p, _p, _i, _p, _p]),
     "unok_attn_bwd": (_i, [_i, _i, _i, _i, _i, _i, _i, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64,
                            _p, _p, _p, _i64, _p, _p, _i64, _p, _p, _i64, _p, _i64, _p, _i64, _f, _p]),

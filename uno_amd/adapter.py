@@ -190,6 +190,11 @@ class LoraState:
     def sb_c(self, layer: int, group: str) -> torch.Tensor:
         return self.group_b(self.copy, layer, group)
 
+    def group_ptrs(self, layer: int, group: str) -> tuple[int, int]:
+        """Device addresses of ``a_c`` and ``sb_c`` (both contiguous)."""
+        first, base, size = self.slots[layer][GROUPS[group][0]], self.copy.data_ptr(), self.copy.element_size()
+        return base + first.a_off * size, base + first.b_off * size
+
     def grad_a(self, layer: int, group: str) -> torch.Tensor:
         return self.group_a(self.grad, layer, group)
 

@@ -13,6 +13,7 @@
 // finished first) also forms the hidden h = bf16(m (.) x A^T) of its rows and applies the rank-r
 // update and the epilogue. With one K range and no LoRA the product kernel writes C itself.
 #include "common.h"
+#include "../../include/unok.h"
 
 #include <type_traits>
 
@@ -538,6 +539,25 @@ __global__ __launch_bounds__(256) void decode_prep_kernel(const bf16_t* __restri
                                    pack2_bf16(x[6], x[7]));
 }
 
+// Row maps of a draft block's attention from the committed lengths, one thread per (range, decode
+// row): range s of the S key ranges of a query row holds keys [s c, (s + 1) c) of its causal prefix
+// (c = committed length / S), the last range the rest; padding rows have empty ranges and dst -1.
+__global__ __launch_bounds__(256) void decode_maps_kernel(const int64_t* __restrict__ lengths, int L, int nq, int nk,
+                                                          int max_len, int S, int QR, int4* __restrict__ ivs,
+                                                          int32_t* __restrict__ dst) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= S * QR) return;
+  const int s = i / QR, q = i % QR, pair = q / 128, slot = q % 128, rep = nq / nk;
+  const bool valid = slot < rep * L;
+  const int t = slot % L;
+  const int64_t len = lengths[pair / nk], seen = len + t + 1, c = len / S;
+  const int64_t start = (int64_t)pair * max_len;
+  const int64_t lo = s * c, hi = s == S - 1 ? seen : min((s + 1) * c, seen);
+  ivs[2 * i] = make_int4((int)(start + (valid ? lo : 0)), (int)(start + (valid ? max(hi, lo) : 0)), 0, 0);
+  ivs[2 * i + 1] = make_int4(0, 0, 0, 0);
+  if (s == 0) dst[q] = valid ? ((pair / nk) * L + t) * nq + (pair % nk) * rep + slot / L : -1;
+}
+
 // O[dst[i]] = sum_s 2^(lse_s - m) O_s[i] / sum_s 2^(lse_s - m) over the S partial rows s * QR + i
 // (lse in log2 units, m their maximum; a range without keys has lse = -inf and weight 0); rows
 // with dst[i] < 0 are skipped.
@@ -552,22 +572,38 @@ __global__ __launch_bounds__(256) void attn_split_combine_kernel(const bf16_t* _
   const int i = (int)item, c0 = (threadIdx.x % LPR) * 8;
   const int d = dst[i];
   if (d < 0) return;
+  // eight ranges' rows in flight at a time; the ranges are few, so their weights are read twice
   float m = -INFINITY;
-  for (int s = 0; s < S; ++s) m = fmaxf(m, lse[(int64_t)s * QR + i]);
+  for (int s0 = 0; s0 < S; s0 += 8) {
+    float l[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) l[q] = s0 + q < S ? lse[(int64_t)(s0 + q) * QR + i] : -INFINITY;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) m = fmaxf(m, l[q]);
+  }
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   float wsum = 0.f;
   if (m != -INFINITY) {
-    for (int s = 0; s < S; ++s) {
-      const float l = lse[(int64_t)s * QR + i];
-      if (l == -INFINITY) continue;
-      const float w = exp2f(l - m);
-      wsum += w;
-      const uint4 u = *(const uint4*)(op + ((int64_t)s * QR + i) * ldp + c0);
-      const uint32_t v[4] = {u.x, u.y, u.z, u.w};
+    for (int s0 = 0; s0 < S; s0 += 8) {
+      float l[8];
+      uint4 u[8];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        acc[2 * k] += w * __uint_as_float(v[k] << 16);
-        acc[2 * k + 1] += w * __uint_as_float(v[k] & 0xffff0000u);
+      for (int q = 0; q < 8; ++q) {
+        const int64_t r = (int64_t)min(s0 + q, S - 1) * QR + i;
+        l[q] = s0 + q < S ? lse[r] : -INFINITY;
+        u[q] = *(const uint4*)(op + r * ldp + c0);
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        if (l[q] == -INFINITY) continue;
+        const float w = exp2f(l[q] - m);
+        wsum += w;
+        const uint32_t v[4] = {u[q].x, u[q].y, u[q].z, u[q].w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          acc[2 * k] += w * __uint_as_float(v[k] << 16);
+          acc[2 * k + 1] += w * __uint_as_float(v[k] & 0xffff0000u);
+        }
       }
     }
   }
@@ -727,4 +763,105 @@ UNOK_EXPORT int unok_attn_split_combine(int QR, int S, int D, const void* opart,
     hipLaunchKernelGGL((attn_split_combine_kernel<64>), dim3((unsigned)blocks), dim3(256), 0, st,
                        (const bf16_t*)opart, ldp, lse, dst, QR, S, (bf16_t*)out, ldo);
   return unok::check_launch("attn_split_combine");
+}
+
+// Key intervals (ivs, [S * QR, 8] int32) and output rows (dst, [QR] int32) of a draft block's split-key
+// attention, QR = 128 B nk decode rows (see decode_maps_kernel).
+UNOK_EXPORT int unok_decode_maps(int B, int L, int nq, int nk, int max_len, int S, const int64_t* lengths, int32_t* ivs,
+                                 int32_t* dst, void* stream) {
+  UNOK_REQUIRE(B >= 0 && L >= 0 && nq > 0 && nk > 0 && nq % nk == 0 && S >= 1 && max_len >= 0, UNOK_EINVAL,
+               "decode_maps: B=%d L=%d nq=%d nk=%d S=%d max_len=%d", B, L, nq, nk, S, max_len);
+  if (B == 0 || L == 0) return 0;
+  const int64_t rows = (int64_t)B * nk * 128 * S;
+  UNOK_REQUIRE((nq / nk) * L <= 128 && rows < (1ll << 30) && (int64_t)B * nk * max_len < (1ll << 31) &&
+                   (int64_t)B * L * nq < (1ll << 31),
+               UNOK_EINVAL, "decode_maps: B=%d L=%d max_len=%d S=%d exceed the row layout", B, L, max_len, S);
+  UNOK_REQUIRE(((uintptr_t)ivs & 15) == 0, UNOK_EALIGN, "decode_maps: ivs must be 16-byte aligned");
+  hipLaunchKernelGGL(decode_maps_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, (hipStream_t)stream, lengths,
+                     L, nq, nk, max_len, S, B * nk * 128, (int4*)ivs, dst);
+  return unok::check_launch("decode_maps");
+}
+
+// ---------------------------------------------------------------------------------------
+// One decoder layer of a draft block: the kernels above in order, launched from here. A layer of a
+// small model runs for less time than eleven calls take to make one by one from Python.
+// ---------------------------------------------------------------------------------------
+namespace {
+
+struct DraftBuffers {
+  int64_t x, qkv, qd, op, lse, o, h1, s, ws, bytes;
+};
+
+DraftBuffers draft_buffers(const unok_draft_layer_args& a) {
+  const int64_t M = (int64_t)a.B * a.L, q = (int64_t)a.nq * a.D, kv = (int64_t)a.nk * a.D;
+  const int64_t QR = (int64_t)a.B * a.nk * 128;
+  DraftBuffers b;
+  int64_t at = 0;
+  auto take = [&](int64_t n) { const int64_t p = at; at += (n + 255) / 256 * 256; return p; };
+  b.x = take(M * a.H * 2);
+  b.qkv = take(M * (q + 2 * kv) * 2);
+  b.qd = take(QR * a.D * 2);
+  b.op = take(QR * a.S * a.D * 2);
+  b.lse = take(QR * a.S * 4);
+  b.o = take(M * q * 2);
+  b.h1 = take(M * a.H * 2);
+  b.s = take(M * a.F * 2);
+  const int64_t need[4] = {unok_gemm_nt_rows_workspace((int)M, (int)(q + 2 * kv), a.H, 3 * a.r, 0, 0),
+                           unok_gemm_nt_rows_workspace((int)M, a.H, (int)q, a.r, 0, 0),
+                           unok_gemm_nt_rows_workspace((int)M, 2 * a.F, a.H, 2 * a.r, 1, 0),
+                           unok_gemm_nt_rows_workspace((int)M, a.H, a.F, a.r, 0, 0)};
+  int64_t most = 0;
+  for (int64_t n : need) most = n > most ? n : most;
+  b.ws = take(most);
+  b.bytes = at;
+  return b;
+}
+
+int draft_sizes_ok(const unok_draft_layer_args* a) {
+  UNOK_REQUIRE(a != nullptr && a->B >= 0 && a->L >= 0 && a->nq > 0 && a->nk > 0 && a->nq % a->nk == 0 && a->H > 0 &&
+                   a->F > 0 && a->r > 0 && a->S >= 1 && (a->D == 64 || a->D == 128) &&
+                   (int64_t)a->B * a->L < (1 << 24) && (int64_t)a->nq * a->D < (1 << 24) && a->F < (1 << 24),
+               UNOK_EINVAL, "draft_layer: bad sizes");
+  return 0;
+}
+
+}  // namespace
+
+UNOK_EXPORT int64_t unok_draft_layer_scratch(const unok_draft_layer_args* a) {
+  if (draft_sizes_ok(a)) return -1;
+  return draft_buffers(*a).bytes;
+}
+
+UNOK_EXPORT int unok_draft_layer(const unok_draft_layer_args* a, void* stream) {
+  int rc = draft_sizes_ok(a);
+  if (rc || a->B == 0 || a->L == 0) return rc;
+  const DraftBuffers b = draft_buffers(*a);
+  UNOK_REQUIRE(a->scratch != nullptr && a->scratch_bytes >= b.bytes && ((uintptr_t)a->scratch & 255) == 0, UNOK_EINVAL,
+               "draft_layer: scratch of %lld bytes (256-byte aligned) required, got %lld", (long long)b.bytes,
+               (long long)a->scratch_bytes);
+  const int M = a->B * a->L, q = a->nq * a->D, kv = a->nk * a->D, H = a->H, F = a->F, r = a->r, QR = a->B * a->nk * 128;
+  char* base = (char*)a->scratch;
+  void *x = base + b.x, *qkv = base + b.qkv, *qd = base + b.qd, *op = base + b.op, *o = base + b.o, *h1 = base + b.h1,
+       *s = base + b.s, *ws = base + b.ws;
+  float* lse = (float*)(base + b.lse);
+  const int64_t ws_bytes = b.bytes - b.ws;
+  const int qkv_end[3] = {q, q + kv, q + 2 * kv}, qkv_col[3] = {0, r, 2 * r};
+  const int gu_end[2] = {F, 2 * F}, gu_col[2] = {0, r};
+  auto linear = [&](const void* in, int K, const void* w, const void* la, const void* lb, int N, int nseg, const int* end,
+                    const int* col, const void* res, int epi, void* out) {
+    return unok_gemm_nt_rows(M, N, K, in, K, w, K, la, K, (nseg ? nseg : 1) * r, lb, r, r, nseg, end, col, out,
+                             epi ? N / 2 : N, res, N, a->gate, epi, 0, ws, ws_bytes, stream);
+  };
+  if ((rc = unok_rmsnorm_fwd(UNOK_BF16, M, H, a->h, H, a->ln_in, x, H, nullptr, a->eps, stream))) return rc;
+  if ((rc = linear(x, H, a->w_qkv, a->a_qkv, a->b_qkv, q + 2 * kv, 3, qkv_end, qkv_col, nullptr, 0, qkv))) return rc;
+  if ((rc = unok_decode_prep(a->B, a->L, a->nq, a->nk, a->D, qkv, q + 2 * kv, a->q_norm, a->k_norm, a->lengths,
+                             a->inv_freq, a->eps, a->kc, a->vc, a->max_len, qd, stream)))
+    return rc;
+  if ((rc = unok_attn_fwd_split(QR, a->S, a->D, qd, a->D, a->kc, a->D, a->vc, a->D, a->ivs, op, a->D, lse, a->scale, stream)))
+    return rc;
+  if ((rc = unok_attn_split_combine(QR, a->S, a->D, op, a->D, lse, a->dst, o, a->D, stream))) return rc;
+  if ((rc = linear(o, q, a->w_o, a->a_o, a->b_o, H, 0, nullptr, nullptr, a->h, 0, h1))) return rc;
+  if ((rc = unok_rmsnorm_fwd(UNOK_BF16, M, H, h1, H, a->ln_post, x, H, nullptr, a->eps, stream))) return rc;
+  if ((rc = linear(x, H, a->w_gu, a->a_gu, a->b_gu, 2 * F, 2, gu_end, gu_col, nullptr, 1, s))) return rc;
+  return linear(s, F, a->w_d, a->a_d, a->b_d, H, 0, nullptr, nullptr, h1, 0, a->h_out);
 }

@@ -21,8 +21,11 @@ Kernels, all shared with the training step:
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
+from . import _native as N
 from . import kernels as K
 from .layers import Geometry
 
@@ -94,21 +97,24 @@ class BlockDecoder:
         if B != cache.batch:
             raise RuntimeError(f"block batch {B} does not match the cache batch {cache.batch}")
         lengths = cache.lengths
-        if check and int((lengths + L).max()) > cache.max_len:
+        if check and int(lengths.max()) + L > cache.max_len:
             raise RuntimeError("the block does not fit in the KV cache")
         rep = g.nq // g.nk
         if not prefill and rep * L > 128:
             raise NotImplementedError(f"draft blocks hold at most 128 / {rep} rows per sequence (got {L})")
         dev = ids.device
         M = B * L
-        j = torch.arange(L, device=dev)
-        pos = (lengths[:, None] + j[None, :]).reshape(-1).contiguous()            # [M] int64
         gate_rows = gate.reshape(-1).contiguous()
-        maps = self._maps(cache, lengths, B, L, prefill)
         h = K.embedding(ids.reshape(-1).contiguous().to(torch.int64), dec.embed_tokens.weight)
-        for li, layer in enumerate(dec.layers):
-            lw = layer.weights()
-            h = self._layer(h, lw, li, pos, gate_rows, cache, maps, B, L, prefill)
+        if not prefill and self._split_path(dev, cache) and self._rows_path(M, h.dtype, prefill):
+            h = self._draft_layers(h, cache, gate_rows, B, L)
+        else:
+            j = torch.arange(L, device=dev)
+            pos = (lengths[:, None] + j[None, :]).reshape(-1).contiguous()            # [M] int64
+            maps = self._maps(cache, lengths, B, L, prefill)
+            for li, layer in enumerate(dec.layers):
+                lw = layer.weights()
+                h = self._layer(h, lw, li, pos, gate_rows, cache, maps, B, L, prefill)
         x, _ = K.rmsnorm_fwd(h, dec.norm.weight, g.eps)
         V = self.base.lm_head.weight.shape[0]
         head = K.gemm_nt_rows if self._rows_path(M, x.dtype, prefill) and V % 4 == 0 else K.gemm_nt
@@ -123,6 +129,11 @@ class BlockDecoder:
         i32 = dict(device=dev, dtype=torch.int32)
         rep = g.nq // g.nk
         out = {}
+        if not prefill and self._split_path(dev, cache):
+            S = self._key_ranges(cache, B)
+            out["ivs"], out["dst"] = K.decode_maps(lengths, B, L, g.nq, g.nk, cache.max_len, S)
+            out["S"], out["QR"] = S, B * g.nk * 128
+            return out
         slot = torch.arange(128, device=dev)
         pair = torch.arange(B * g.nk, device=dev)
         valid = slot < rep * L
@@ -130,28 +141,6 @@ class BlockDecoder:
         start = pair[:, None] * cache.max_len                                           # [pairs, 1]
         lens = lengths[:, None].expand(B, g.nk).reshape(-1, 1)                          # [pairs, 1]
         seen = lens + tt[None, :] + 1                                                   # causal over cache + block
-        if not prefill and self._split_path(dev, cache):
-            # split-key layout: S key ranges per (sequence, K/V head) pair; range s of a query row
-            # holds keys [s c, (s + 1) c) of its causal prefix (c = committed length // S), the last
-            # range the rest; padding rows get empty ranges
-            pairs = B * g.nk
-            S = max(1, min(8, 256 // pairs))
-            QR = pairs * 128
-            c = lens // S
-            s_idx = torch.arange(S, device=dev)[:, None, None]                          # [S, 1, 1]
-            lo = s_idx * c[None]                                                         # [S, pairs, 1]
-            hi = torch.where(s_idx == S - 1, seen[None], torch.minimum((s_idx + 1) * c[None], seen[None]))
-            hi = torch.maximum(hi, lo)
-            lo = torch.where(valid[None, None, :], lo, 0)
-            hi = torch.where(valid[None, None, :], hi, 0)
-            ivs = torch.zeros((S * QR, 8), **i32)
-            ivs[:, 0] = (start[None] + lo).reshape(-1)
-            ivs[:, 1] = (start[None] + hi).reshape(-1)
-            # decode row (pair b nk + kv, slot r L + t) -> output row (b L + t) nq + kv rep + r
-            dst = ((pair // g.nk)[:, None] * L + tt[None, :]) * g.nq + (pair % g.nk)[:, None] * rep + (slot // L)[None, :]
-            out["dst"] = torch.where(valid[None, :], dst, -1).reshape(-1).to(**i32)
-            out["ivs"], out["S"], out["QR"] = ivs, S, QR
-            return out
         b = torch.arange(B, device=dev)[:, None, None]
         t = torch.arange(L, device=dev)[None, :, None]
         kv = torch.arange(g.nk, device=dev)[None, None, :]
@@ -175,6 +164,47 @@ class BlockDecoder:
         out["iv"] = iv
         return out
 
+    def _key_ranges(self, cache, B: int) -> int:
+        """Key ranges per (sequence, K/V head) pair: as many as give one round of attention workgroups
+        (one per pair and range, 256 CUs), at most eight."""
+        return max(1, min(8, 256 // (B * self.geo.nk)))
+
+    def _draft_layers(self, h, cache, gate_rows, B: int, L: int):
+        """All layers of a bf16 draft block, one native call each (see unok_draft_layer); the layers share
+        one scratch buffer."""
+        g, lora, dec = self.geo, self.lora, self.decoder
+        S = self._key_ranges(cache, B)
+        lengths, inv_freq = cache.lengths, dec.inv_freq
+        ivs, dst = K.decode_maps(lengths, B, L, g.nq, g.nk, cache.max_len, S)
+        a = N.DraftLayerArgs(B=B, L=L, nq=g.nq, nk=g.nk, D=g.d, H=g.H, F=g.F, r=lora.rank, S=S, max_len=cache.max_len,
+                             eps=g.eps, scale=g.d ** -0.5, lengths=N.ptr(lengths), inv_freq=N.ptr(inv_freq),
+                             gate=N.ptr(gate_rows), ivs=N.ptr(ivs), dst=N.ptr(dst))
+        nbytes = N.lib().unok_draft_layer_scratch(ctypes.byref(a))
+        if nbytes < 0:
+            N.check(-1, "unok_draft_layer_scratch")
+        scratch = torch.empty(nbytes + 256, device=h.device, dtype=torch.uint8)
+        a.scratch, a.scratch_bytes = (N.ptr(scratch) + 255) // 256 * 256, nbytes
+        if lengths.dtype != torch.int64 or not all(t.is_contiguous() for t in (*cache.k, *cache.v)):
+            raise RuntimeError("draft blocks need int64 lengths and contiguous caches")
+        other, stream = torch.empty_like(h), N.stream()
+        for li, layer in enumerate(dec.layers):
+            lw = layer.weights()
+            a.ln_in, a.ln_post, a.q_norm, a.k_norm = N.ptr(lw.ln_in), N.ptr(lw.ln_post), N.ptr(lw.q_norm), N.ptr(lw.k_norm)
+            if any(w.dtype != h.dtype or w.numel() != g.H for w in (lw.ln_in, lw.ln_post)):
+                raise RuntimeError("rmsnorm: weight must match the hidden size and dtype")
+            for part, w in (("qkv", lw.w_qkv), ("o", lw.w_o), ("gu", lw.w_gu), ("d", lw.w_d)):
+                if w.dtype != h.dtype or not w.is_contiguous():
+                    raise RuntimeError(f"draft blocks need contiguous bf16 weights (layer {li} {part})")
+                setattr(a, "w_" + part, N.ptr(w))
+                la, lb = lora.group_ptrs(li, part)
+                setattr(a, "a_" + part, la)
+                setattr(a, "b_" + part, lb)
+            a.kc, a.vc = N.ptr(cache.k[li]), N.ptr(cache.v[li])
+            a.h, a.h_out = N.ptr(h), N.ptr(other)
+            N.call("unok_draft_layer", ctypes.byref(a), stream)
+            h, other = other, h
+        return h
+
     def _split_path(self, dev, cache) -> bool:
         """bf16 draft blocks run the attention as prep + split-key attention + combine."""
         return cache.k[0].dtype == torch.bfloat16 and self.geo.d in (64, 128)
@@ -191,14 +221,10 @@ class BlockDecoder:
         r = lora.rank
         q_end, k_end = g.q, g.q + g.kv
         M = h0.shape[0]
-        few = self._rows_path(M, h0.dtype, prefill)
         qkv_segments = [(q_end, 0), (k_end, r), (k_end + g.kv, 2 * r)]
 
         def linear(x, w, part, segments=None, residual=None, swiglu=False):
             """Gated LoRA linear: x w^T + (m (.) x A^T)[:, seg] (s B)^T (+ residual)."""
-            if few:
-                return K.gemm_nt_rows(x, w, lora_a=lora.a_c(li, part), lora_b=lora.sb_c(li, part),
-                                      segments=segments, residual=residual, gate=gate_rows, swiglu=swiglu)
             h = K.gemm_nt(x, lora.a_c(li, part), gate=gate_rows)
             y = K.gemm_nt(x, w, a2=h, b2=lora.sb_c(li, part), segments=segments, residual=residual)
             return K.swiglu_fwd(y, y.shape[1] // 2) if swiglu else y
@@ -238,7 +264,6 @@ class BlockDecoder:
         g, r = self.geo, self.lora.rank
         h1 = linear(o, lw.w_o, "o", residual=h0)
         x2, _ = K.rmsnorm_fwd(h1, lw.ln_post, g.eps)
-        # few-row path: the reduction of the gate/up product applies the SwiGLU ([gate | up] is never stored)
         s = linear(x2, lw.w_gu, "gu", [(g.F, 0), (2 * g.F, r)], swiglu=True)
         return linear(s, lw.w_d, "d", residual=h1)
 

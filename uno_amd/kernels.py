@@ -549,6 +549,18 @@ def decode_prep(qkv, wq, wk, lengths, inv_freq, eps: float, kc, vc, qd, B: int, 
     return qd
 
 
+def decode_maps(lengths, B: int, L: int, nq: int, nk: int, max_len: int, S: int):
+    """Key intervals [S*QR, 8] and output rows [QR] (QR = 128 B nk) of a draft block's split-key attention
+    at the committed lengths."""
+    if lengths.dtype != torch.int64 or lengths.numel() != B or not lengths.is_contiguous():
+        raise RuntimeError("decode_maps: contiguous int64 lengths [B] required")
+    QR = B * nk * 128
+    ivs = torch.empty((S * QR, 8), device=lengths.device, dtype=torch.int32)
+    dst = torch.empty(QR, device=lengths.device, dtype=torch.int32)
+    N.call("unok_decode_maps", B, L, nq, nk, max_len, S, N.ptr(lengths), N.ptr(ivs), N.ptr(dst), N.stream())
+    return ivs, dst
+
+
 def attn_bwd_qknorm(q, k1, v1, iv, o, lse, do, Hq, Hkv, D, k2, v2, pre, rstd, wq, wk, pos, cos_tab, sin_tab, dqkv,
                     scale=None):
     """Noisy-stream backward with the q/k RMSNorm + RoPE backward in the dQ / dK epilogues (bf16): writes
