@@ -987,6 +987,99 @@ __global__ __launch_bounds__(256) void attn_dq_f32_kernel(const AttnArgs p, int 
   for (int t = 0; t < 2; ++t) if (lane + 64 * t < D) o[lane + 64 * t] = acc[t] * p.scale;
 }
 
+// fp32 forward and dQ for head dims 64 and 128 with 16-byte aligned rows: one wave per (row, head), its
+// 64 lanes taking 64 keys at a time. Each lane forms whole dot products of its key (q is in the
+// wave's registers, one readlane per element), one max and one sum across the wave serve 64 keys,
+// and the accumulation then runs over the keys with lane = output column. The form above pays the
+// cross-lane sum for every key: 2 x 256 tokens, 4 heads of 64: forward 183 -> 28 us, dQ 170 -> 41 us.
+__device__ __forceinline__ float lane_f32(float v, int lane) {
+  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane));
+}
+
+template <int D>
+__device__ __forceinline__ float dot_row(const float* row, const float (&q)[D / 64]) {
+  f32x4_t v[D / 4];
+#pragma unroll
+  for (int c = 0; c < D / 4; ++c) v[c] = *(const f32x4_t*)(row + c * 4);
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < D / 4; ++c)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[e] = fmaf(lane_f32(q[c / 16], (c * 4 + e) & 63), v[c][e], s[e]);
+  return (s[0] + s[1]) + (s[2] + s[3]);
+}
+
+// acc[t] += sum over the first n lanes' w of w x rows[k][lane + 64 t]
+template <int D>
+__device__ __forceinline__ void add_rows(const float* rows, int64_t ld, float w, int n, float (&acc)[D / 64]) {
+  const int lane = threadIdx.x & 63;
+  int k = 0;
+  for (; k + 8 <= n; k += 8) {
+    float v[8][D / 64];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int t = 0; t < D / 64; ++t) v[u][t] = rows[(int64_t)(k + u) * ld + lane + 64 * t];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int t = 0; t < D / 64; ++t) acc[t] = fmaf(lane_f32(w, k + u), v[u][t], acc[t]);
+  }
+  for (; k < n; ++k)
+#pragma unroll
+    for (int t = 0; t < D / 64; ++t) acc[t] = fmaf(lane_f32(w, k), rows[(int64_t)k * ld + lane + 64 * t], acc[t]);
+}
+
+template <int D, bool DQ>
+__global__ __launch_bounds__(256) void attn_f32_rows_kernel(const AttnArgs p) {
+  constexpr int NT = D / 64;
+  const int lane = threadIdx.x & 63;
+  // the wave's item, in a scalar register: every row address below is uniform or lane-linear
+  const int64_t item = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (item >= (int64_t)p.Mq * p.Hq) return;
+  const int qrow = (int)(item / p.Hq), h = (int)(item % p.Hq);
+  const int kvh = h / (p.Hq / p.Hkv);
+  const int4 iv = *(const int4*)(p.iv + (int64_t)qrow * 8);
+  float q[NT], g[NT], acc[NT];
+  const float* qr = (const float*)p.Q + (int64_t)qrow * p.ldq + h * D;
+  const float* gr = DQ ? (const float*)p.dO + (int64_t)qrow * p.lddo + h * D : qr;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) { q[t] = qr[lane + 64 * t]; g[t] = gr[lane + 64 * t]; acc[t] = 0.f; }
+  const float lse = DQ ? p.LSE[item] : 0.f, ds = DQ ? p.Dsum[item] : 0.f;
+  float m = -INFINITY, l = 0.f;
+  for (int src = 0; src < 2; ++src) {
+    if (!(src ? p.K2 : p.K1)) continue;
+    const int64_t ldk = src ? p.ldk2 : p.ldk1, ldv = src ? p.ldv2 : p.ldv1;
+    const float* K = (const float*)(src ? p.K2 : p.K1) + kvh * D;
+    const float* V = (const float*)(src ? p.V2 : p.V1) + kvh * D;
+    const int lo = __builtin_amdgcn_readfirstlane(src ? iv.z : iv.x), hi = __builtin_amdgcn_readfirstlane(src ? iv.w : iv.y);
+    for (int k0 = lo; k0 < hi; k0 += 64) {
+      const int n = min(64, hi - k0);
+      const bool on = lane < n;
+      const int64_t key = k0 + min(lane, n - 1);
+      const float s = dot_row<D>(K + key * ldk, q) * p.scale_log2;
+      if constexpr (DQ) {
+        const float dp = dot_row<D>(V + key * ldv, g);
+        const float w = on ? exp2f(s - lse) * (dp - ds) : 0.f;
+        add_rows<D>(K + (int64_t)k0 * ldk, ldk, w, n, acc);
+      } else {
+        const float mn = fmaxf(m, wave_max(on ? s : -INFINITY));
+        const float a = exp2f(m - mn), e = on ? exp2f(s - mn) : 0.f;
+        l = l * a + wave_sum(e);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[t] *= a;
+        add_rows<D>(V + (int64_t)k0 * ldv, ldv, e, n, acc);
+        m = mn;
+      }
+    }
+  }
+  float* o = DQ ? (float*)p.dQ + (int64_t)qrow * p.lddq + h * D : (float*)p.O + (int64_t)qrow * p.ldo + h * D;
+  const float f = DQ ? p.scale : l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) o[lane + 64 * t] = acc[t] * f;
+  if (!DQ && lane == 0) p.LSE[item] = l > 0.f ? m + log2f(l) : -INFINITY;
+}
+
 __global__ __launch_bounds__(256) void attn_dkv_f32_kernel(const AttnArgs p, int D) {
   const int lane = threadIdx.x & 63;
   const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -1036,6 +1129,12 @@ static int check_geom(int dtype, int D, int Hq, int Hkv) {
 
 static bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
+// Operands of attn_f32_rows_kernel: its keys' rows are read 16 bytes at a time.
+static bool f32_rows_ok(int D, const AttnArgs& a) {
+  return (D == 64 || D == 128) && al16(a.K1) && al16(a.V1) && a.ldk1 % 4 == 0 && a.ldv1 % 4 == 0 &&
+         (!a.K2 || (al16(a.K2) && al16(a.V2) && a.ldk2 % 4 == 0 && a.ldv2 % 4 == 0));
+}
+
 // Forward: 32 queries per wave, 128 per workgroup, two workgroups per CU.
 template <int D>
 static void launch_fwd(int Mq, int Hq, hipStream_t st, const AttnArgs& a) {
@@ -1077,7 +1176,10 @@ UNOK_EXPORT int unok_attn_fwd(int dtype, int Mq, int Hq, int Hkv, int D, const v
   a.Mq = Mq; a.Hq = Hq; a.Hkv = Hkv; a.scale = scale; a.scale_log2 = scale * 1.4426950408889634f;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == UNOK_F32) {
-    hipLaunchKernelGGL(attn_fwd_f32_kernel, dim3((unsigned)(((int64_t)Mq * Hq + 3) / 4)), dim3(256), 0, st, a, D);
+    const unsigned nb = (unsigned)(((int64_t)Mq * Hq + 3) / 4);
+    if (f32_rows_ok(D, a) && D == 64) hipLaunchKernelGGL((attn_f32_rows_kernel<64, false>), dim3(nb), dim3(256), 0, st, a);
+    else if (f32_rows_ok(D, a)) hipLaunchKernelGGL((attn_f32_rows_kernel<128, false>), dim3(nb), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(attn_fwd_f32_kernel, dim3(nb), dim3(256), 0, st, a, D);
   } else {
     UNOK_REQUIRE(dtype == UNOK_BF16, UNOK_EINVAL, "attention: bad dtype %d", dtype);
     UNOK_REQUIRE(al16(Q) && al16(K1) && al16(V1) && ldq % 8 == 0 && ldk1 % 8 == 0 && ldv1 % 8 == 0 && ldo % 8 == 0 &&
@@ -1148,7 +1250,9 @@ UNOK_EXPORT int unok_attn_bwd(int dtype, int grad_dtype, int Mq, int Mk2, int Hq
   const bool want_kv = dK != nullptr && dV != nullptr && K2 != nullptr && Mk2 > 0;
   if (want_kv) UNOK_REQUIRE(ivk != nullptr, UNOK_EINVAL, "attn_bwd: key-side interval table required for dK/dV");
   if (dtype == UNOK_F32) {
-    hipLaunchKernelGGL(attn_dq_f32_kernel, dim3(items), dim3(256), 0, st, a, D);
+    if (f32_rows_ok(D, a) && D == 64) hipLaunchKernelGGL((attn_f32_rows_kernel<64, true>), dim3(items), dim3(256), 0, st, a);
+    else if (f32_rows_ok(D, a)) hipLaunchKernelGGL((attn_f32_rows_kernel<128, true>), dim3(items), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(attn_dq_f32_kernel, dim3(items), dim3(256), 0, st, a, D);
     rc = unok::check_launch("attn_dq_f32");
     if (rc || !want_kv) return rc;
     hipLaunchKernelGGL(attn_dkv_f32_kernel, dim3((unsigned)(((int64_t)Mk2 * Hkv + 3) / 4)), dim3(256), 0, st, a, D);

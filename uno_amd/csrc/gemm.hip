@@ -426,64 +426,107 @@ __device__ __forceinline__ void store4(float* dst, const float* res, const float
 }
 
 // ---------------------------------------------------------------------------------------
-// fp32 NT kernel (fp32 parity mode): 64x64 tiles, 16-deep K slices, 4x4 outputs per thread.
+// fp32 NT kernel (fp32 parity mode): 32x32 outputs per workgroup, its NW waves taking the 16-deep K
+// chunks in turn. Lane l holds rows l % 16 and k = 4 (l / 16) + 0..3 of a chunk, one 16-byte load per
+// operand fragment straight from global memory, which four 16x16x4 MFMAs consume (full fp32
+// products and sums; both operands use the same k order); four chunks are loaded while the four
+// before are multiplied. The waves' sums meet in LDS and are added in wave order.
+// Bound by latency at the parity sizes (hundreds of rows, K 256 and 768): a 64x64 tile with one
+// 16-deep slice per barrier took 35 to 130 us per product there, this one 4 to 9 us.
+// VEC: K, K2, row strides and segment columns are multiples of 4 and operands 16-byte aligned.
 // ---------------------------------------------------------------------------------------
-template <typename OutT>
-__global__ __launch_bounds__(256) void gemm_nt_f32_kernel(const GemmNT p) {
-  __shared__ float As[16][65], Bs[16][65];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const float* A = (const float*)p.A;
-  const float* B = (const float*)p.B;
-  const float* A2 = nullptr;
-  if (p.A2 != nullptr && p.K2 > 0) A2 = (const float*)p.A2 + seg_col_of(p, n0);
-  const float* B2 = (const float*)p.B2;
-  float acc[4][4] = {};
-  for (int part = 0; part < 2; ++part) {
-    const float* a = part ? A2 : A;
-    const float* b = part ? B2 : B;
-    if (a == nullptr) continue;
-    const int64_t la = part ? p.lda2 : p.lda, lb = part ? p.ldb2 : p.ldb;
-    const int K = part ? p.K2 : p.K;
-    for (int k0 = 0; k0 < K; k0 += 16) {
+constexpr int F32_T = 32;
+
+template <typename OutT, bool VEC, int NW>
+__global__ __launch_bounds__(NW * 64) void gemm_nt_f32_kernel(const GemmNT p) {
+  constexpr int T = F32_T, G = 4, LD = T + 4;
+  __shared__ __attribute__((aligned(16))) float red[NW][T * LD];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, lr = lane & 15, lg = lane >> 4;
+  const int n0 = blockIdx.x * T;
+  const int64_t mt = (int64_t)blockIdx.z * gridDim.y + blockIdx.y;
+  if (mt * T >= p.M) return;
+  const int m0 = (int)mt * T;
+  const bool ext = p.A2 != nullptr && p.K2 > 0;
+  const int n1 = (p.K + 15) / 16, n = n1 + (ext ? (p.K2 + 15) / 16 : 0);
+  const float* A2 = ext ? (const float*)p.A2 + seg_col_of(p, n0) : nullptr;
+  int64_t ra[2], rb[2];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int e = tid + 256 * q, r = e >> 4, k = e & 15;
-        const int gm = m0 + r, gn = n0 + r, gk = k0 + k;
-        As[k][r] = (gm < p.M && gk < K) ? a[(int64_t)gm * la + gk] : 0.f;
-        Bs[k][r] = (gn < p.N && gk < K) ? b[(int64_t)gn * lb + gk] : 0.f;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        float av[4], bv[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) av[i] = As[k][ty + 16 * i];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) bv[j] = Bs[k][tx + 16 * j];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
-      }
-      __syncthreads();
-    }
+  for (int i = 0; i < 2; ++i) {
+    ra[i] = min(m0 + i * 16 + lr, p.M - 1);
+    rb[i] = min(n0 + i * 16 + lr, p.N - 1);
   }
+  auto fetch = [&](const float* row, int k, int kmax) {
+    f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (VEC) {
+      if (k < kmax) v = *(const f32x4_t*)(row + k);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (k + e < kmax) v[e] = row[k + e];
+    }
+    return v;
+  };
+  // chunk c of this wave's walk (past the end: zeros)
+  auto load = [&](int c, f32x4_t (&a)[2], f32x4_t (&b)[2]) {
+    const bool main = c < n1;
+    const float* pa = main ? (const float*)p.A : A2;
+    const float* pb = (const float*)(main ? p.B : p.B2);
+    const int64_t la = main ? p.lda : p.lda2, lb = main ? p.ldb : p.ldb2;
+    const int kmax = c >= n ? 0 : main ? p.K : p.K2, k = (main ? c : c - n1) * 16 + lg * 4;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      a[i] = fetch(pa + ra[i] * la, k, kmax);
+      b[i] = fetch(pb + rb[i] * lb, k, kmax);
+    }
+  };
+  f32x4_t acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  f32x4_t a[2][G][2], b[2][G][2];
+  const int ngroup = (n + G * NW - 1) / (G * NW);
+  auto load_group = [&](int g, f32x4_t (&ga)[G][2], f32x4_t (&gb)[G][2]) {
+#pragma unroll
+    for (int q = 0; q < G; ++q) load((g * G + q) * NW + wid, ga[q], gb[q]);
+  };
+  auto multiply = [&](const f32x4_t (&ga)[G][2], const f32x4_t (&gb)[G][2]) {
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(gb[q][j][e], ga[q][i][e], acc[i][j], 0, 0, 0);
+  };
+  load_group(0, a[0], b[0]);
+  for (int g = 0; g < ngroup; g += 2) {
+    if (g + 1 < ngroup) load_group(g + 1, a[1], b[1]);
+    multiply(a[0], b[0]);
+    if (g + 1 >= ngroup) break;
+    if (g + 2 < ngroup) load_group(g + 2, a[0], b[0]);
+    multiply(a[1], b[1]);
+  }
+  // lane l holds C[row 16 i + l % 16][cols 16 j + 4 (l / 16) + 0..3]
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) *(f32x4_t*)&red[wid][(i * 16 + lr) * LD + j * 16 + lg * 4] = acc[i][j];
+  __syncthreads();
   OutT* C = (OutT*)p.C;
   const OutT* R = (const OutT*)p.R;
+  for (int t = threadIdx.x; t < T * T; t += NW * 64) {
+    const int row = m0 + t / T, col = n0 + t % T;
+    if (row >= p.M || col >= p.N) continue;
+    float v = 0.f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = m0 + ty + 16 * i;
-    if (row >= p.M) continue;
+    for (int w = 0; w < NW; ++w) v += red[w][(t / T) * LD + t % T];
     const bool on = (p.gate == nullptr) || (p.gate[row] != 0);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int col = n0 + tx + 16 * j;
-      if (col >= p.N) continue;
-      float v = on ? acc[i][j] * p.alpha : 0.f;
-      if (R) v += ld_f(R + (int64_t)row * p.ldr + col);
-      Elem<OutT>::store(C + (int64_t)row * p.ldc + col, v);
-    }
+    v = on ? v * p.alpha : 0.f;
+    if (R) v += ld_f(R + (int64_t)row * p.ldr + col);
+    Elem<OutT>::store(C + (int64_t)row * p.ldc + col, v);
   }
 }
 
@@ -586,49 +629,67 @@ __global__ __launch_bounds__(256) void gemm_tn_bf16_kernel(const GemmTN p) {
     }
 }
 
+// fp32: 64 columns of the wider operand X (XP: A, else B) by 16 of the other, S; the four waves take
+// the split's rows four at a time in turn. Lane l loads X columns 4 (l % 16) + 0..3 and S column l % 16
+// of row l / 16 (VEC: one 16-byte load), so MFMA e multiplies X columns 4 i + e; eight steps are
+// loaded ahead of the multiplies. The waves' sums meet in LDS and are added in wave order. Bound by
+// latency at the parity sizes (512 rows): 48 us per product on 64x64 tiles with a barrier per 16 rows,
+// 5 us here.
+template <bool VEC, bool XP>
 __global__ __launch_bounds__(256) void gemm_tn_f32_kernel(const GemmTN p) {
-  __shared__ float As[16][65], Bs[16][65];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int nQ = (p.Q + 63) / 64;
-  const int p0 = (blockIdx.x / nQ) * 64, q0 = (blockIdx.x % nQ) * 64;
-  const int mbeg = blockIdx.y * p.rows_per_split;
-  const int mend = min(p.Mrows, mbeg + p.rows_per_split);
-  const float* A = (const float*)p.A;
-  const float* B = (const float*)p.B;
-  float acc[4][4] = {};
-  for (int mk = mbeg; mk < mend; mk += 16) {
+  constexpr int G = 8, LD = 17;
+  __shared__ float red[4][64 * LD];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, lr = lane & 15, lg = lane >> 4;
+  const int NX = XP ? p.P : p.Q, NS = XP ? p.Q : p.P;
+  const float* X = (const float*)(XP ? p.A : p.B);
+  const float* S = (const float*)(XP ? p.B : p.A);
+  const int64_t ldx = XP ? p.lda : p.ldb, lds = XP ? p.ldb : p.lda;
+  const int nS = (NS + 15) / 16;
+  const int x0 = (int)(blockIdx.x / nS) * 64, s0 = (int)(blockIdx.x % nS) * 16;
+  const int mbeg = blockIdx.y * p.rows_per_split, mend = min(p.Mrows, mbeg + p.rows_per_split);
+  const int xc = x0 + lr * 4, sc = min(s0 + lr, NS - 1);
+  f32x4_t acc[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int e = tid + 256 * q, k = e >> 6, c = e & 63;
-      const int gm = mk + k;
-      As[k][c] = (gm < mend && p0 + c < p.P) ? A[(int64_t)gm * p.lda + p0 + c] : 0.f;
-      Bs[k][c] = (gm < mend && q0 + c < p.Q) ? B[(int64_t)gm * p.ldb + q0 + c] : 0.f;
+  for (int e = 0; e < 4; ++e) acc[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int mk = mbeg; mk < mend; mk += 16 * G) {
+    f32x4_t x[G];
+    float v[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int m = mk + (g * 4 + wid) * 4 + lg;
+      x[g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      v[g] = 0.f;
+      if (m < mend) {
+        const float* xr = X + (int64_t)m * ldx;
+        v[g] = S[(int64_t)m * lds + sc];
+        if constexpr (VEC) {
+          x[g] = *(const f32x4_t*)(xr + min(xc, NX - 4));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[g][e] = xr[min(xc + e, NX - 1)];
+        }
+      }
     }
-    __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      float av[4], bv[4];
+    for (int g = 0; g < G; ++g)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) av[i] = As[k][ty + 16 * i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bv[j] = Bs[k][tx + 16 * j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
-    }
-    __syncthreads();
+      for (int e = 0; e < 4; ++e) acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[g][e], v[g], acc[e], 0, 0, 0);
   }
+  // acc[e][q] of lane l: X column 16 (l / 16) + 4 q + e, S column l % 16
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) red[wid][(lg * 16 + q * 4 + e) * LD + lr] = acc[e][q];
+  __syncthreads();
   float* W = p.WS + (int64_t)blockIdx.y * p.P * p.Q;
+  for (int t = threadIdx.x; t < 64 * 16; t += 256) {
+    const int xi = XP ? t / 16 : t % 64, si = XP ? t % 16 : t / 64;
+    if (x0 + xi >= NX || s0 + si >= NS) continue;
+    float sum = 0.f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = p0 + ty + 16 * i;
-    if (row >= p.P) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int col = q0 + tx + 16 * j;
-      if (col < p.Q) W[(int64_t)row * p.Q + col] = acc[i][j] * p.alpha;
-    }
+    for (int w = 0; w < 4; ++w) sum += red[w][xi * LD + si];
+    const int64_t row = XP ? x0 + xi : s0 + si, col = XP ? s0 + si : x0 + xi;
+    W[row * p.Q + col] = sum * p.alpha;
   }
 }
 
@@ -1838,6 +1899,22 @@ UNOK_EXPORT int unok_lmhead_ce_grad(int R, int V, int K, const void* H, int64_t 
   return unok::check_launch("lmhead_ce_grad");
 }
 
+// fp32 products: eight waves share the K walk of a tile where it is long (230 rows, 4096 -> 256: 581 us
+// on 64x64 tiles, 40 us here; its 64 tiles leave most CUs idle), four else.
+template <typename OutT, bool VEC>
+static void launch_nt_f32_t(const GemmNT& p, hipStream_t st) {
+  const unsigned nM = (unsigned)((p.M + F32_T - 1) / F32_T), my = nM < 32768 ? nM : 32768;
+  const dim3 grid((unsigned)((p.N + F32_T - 1) / F32_T), my, (nM + my - 1) / my);
+  if (p.K >= 1024) hipLaunchKernelGGL((gemm_nt_f32_kernel<OutT, VEC, 8>), grid, dim3(512), 0, st, p);
+  else hipLaunchKernelGGL((gemm_nt_f32_kernel<OutT, VEC, 4>), grid, dim3(256), 0, st, p);
+}
+
+template <typename OutT>
+static void launch_nt_f32(const GemmNT& p, bool vec, hipStream_t st) {
+  if (vec) launch_nt_f32_t<OutT, true>(p, st);
+  else launch_nt_f32_t<OutT, false>(p, st);
+}
+
 static int gemm_nt_any(int in_dtype, int out_dtype, int M, int N, int K,
                        const void* A, int64_t lda, const void* B, int64_t ldb,
                        const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
@@ -1865,11 +1942,12 @@ static int gemm_nt_any(int in_dtype, int out_dtype, int M, int N, int K,
     // The fp32 kernel uses 64-wide N tiles; segment boundaries must align to them.
     for (int i = 0; p.A2 && i + 1 < p.nseg; ++i)
       UNOK_REQUIRE(p.seg_end[i] % 64 == 0, UNOK_EINVAL, "gemm_nt(f32): segment end %d not a multiple of 64", p.seg_end[i]);
-    dim3 grid((N + 63) / 64, (M + 63) / 64);
-    if (out_dtype == UNOK_BF16)
-      hipLaunchKernelGGL((gemm_nt_f32_kernel<bf16_t>), grid, dim3(256), 0, st, p);
-    else
-      hipLaunchKernelGGL((gemm_nt_f32_kernel<float>), grid, dim3(256), 0, st, p);
+    const bool vec = K % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && aligned16(A) && aligned16(B) &&
+                     (!p.A2 || (K2 % 4 == 0 && lda2 % 4 == 0 && ldb2 % 4 == 0 && aligned16(A2) && aligned16(B2) &&
+                                p.seg_col[0] % 4 == 0 && p.seg_col[1] % 4 == 0 && p.seg_col[2] % 4 == 0 &&
+                                p.seg_col[3] % 4 == 0));
+    if (out_dtype == UNOK_BF16) launch_nt_f32<bf16_t>(p, vec, st);
+    else launch_nt_f32<float>(p, vec, st);
     return unok::check_launch("gemm_nt_f32");
   }
   // bf16 MFMA path: 16-byte vector loads need K-contiguous rows with 8-element granularity.
@@ -2326,8 +2404,18 @@ UNOK_EXPORT int unok_gemm_tn(int in_dtype, int Mrows, int P, int Q, const void* 
   const int nz = Mrows > 0 ? (Mrows + rps - 1) / rps : 1;
   GemmTN p{A, lda, B, ldb, (float*)workspace, Mrows, P, Q, rps, alpha};
   if (in_dtype == UNOK_F32) {
-    dim3 grid(((P + 63) / 64) * ((Q + 63) / 64), nz);
-    hipLaunchKernelGGL(gemm_tn_f32_kernel, grid, dim3(256), 0, st, p);
+    const bool xp = P >= Q;
+    const int NX = xp ? P : Q, NS = xp ? Q : P;
+    const int64_t ldx = xp ? lda : ldb;
+    const bool vec = NX % 4 == 0 && ldx % 4 == 0 && aligned16(xp ? A : B);
+    const dim3 grid((unsigned)((NX + 63) / 64) * (unsigned)((NS + 15) / 16), nz);
+    if (xp) {
+      if (vec) hipLaunchKernelGGL((gemm_tn_f32_kernel<true, true>), grid, dim3(256), 0, st, p);
+      else hipLaunchKernelGGL((gemm_tn_f32_kernel<false, true>), grid, dim3(256), 0, st, p);
+    } else {
+      if (vec) hipLaunchKernelGGL((gemm_tn_f32_kernel<true, false>), grid, dim3(256), 0, st, p);
+      else hipLaunchKernelGGL((gemm_tn_f32_kernel<false, false>), grid, dim3(256), 0, st, p);
+    }
   } else {
     UNOK_REQUIRE(in_dtype == UNOK_BF16, UNOK_EINVAL, "gemm_tn: bad dtype %d", in_dtype);
     UNOK_REQUIRE(P % 8 == 0 && Q % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned16(A) && aligned16(B),
