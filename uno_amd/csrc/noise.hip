@@ -143,9 +143,9 @@ __global__ __launch_bounds__(1024) void bd_compact_kernel(const uint8_t* __restr
                                                           const float* __restrict__ tfull,
                                                           const int64_t* __restrict__ pos, int64_t n,
                                                           float* __restrict__ p_mask, int32_t* __restrict__ count) {
-  __shared__ int32_t part[1024];
-  __shared__ int64_t pmax[1024];
-  const int tid = threadIdx.x;
+  __shared__ int32_t part[16];
+  __shared__ int64_t pmax[16];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int64_t chunk = (n + 1023) / 1024;
   const int64_t c0 = min(n, tid * chunk), c1 = min(n, c0 + chunk);
   int32_t cnt = 0;
@@ -153,18 +153,32 @@ __global__ __launch_bounds__(1024) void bd_compact_kernel(const uint8_t* __restr
   for (int64_t i = c0; i < c1; ++i) cnt += noised[i] ? 1 : 0;
   if (pos)
     for (int64_t i = c0; i < c1; ++i) mx = max(mx, pos[i]);
-  part[tid] = cnt;
-  pmax[tid] = mx;
+  // counts before this thread: a scan within the wave, then over the 16 waves (one thread walking
+  // 1024 counts took 30 of the kernel's 37 us)
+  int32_t incl = cnt;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t v = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += v;
+  }
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) mx = max(mx, (int64_t)__shfl_xor((long long)mx, d, 64));
+  if (lane == 63) part[wid] = incl;
+  if (lane == 0) pmax[wid] = mx;
   __syncthreads();
+  int32_t before = 0, total = 0;
+  int64_t m = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    if (w < wid) before += part[w];
+    total += part[w];
+    m = max(m, pmax[w]);
+  }
   if (tid == 0) {
-    int32_t run = 0;
-    int64_t m = 0;
-    for (int i = 0; i < 1024; ++i) { const int32_t v = part[i]; part[i] = run; run += v; m = max(m, pmax[i]); }
-    count[0] = run;
+    count[0] = total;
     if (pos) count[1] = (int32_t)min(m, (int64_t)0x7fffffff);
   }
-  __syncthreads();
-  int32_t o = part[tid];
+  int32_t o = before + incl - cnt;
   for (int64_t i = c0; i < c1; ++i)
     if (noised[i]) p_mask[o++] = tfull[i];
 }
