@@ -16,8 +16,8 @@ Kernels, all shared with the training step:
   the K/V head, at most 128) are laid out as the 128 query rows of one attention workgroup over
   that key range, with per-row key intervals [start, start + cached + j + 1) -- the block-diffusion
   attention kernel then reads each cache row once per pair;
-* a prefill (empty caches) is the causal forward of the prompt with the LoRA gated off, through
-  the clean-stream attention path (keys = the prompt itself).
+* a prefill (empty caches) is the clean stream's causal forward of the prompt (LoRA off, keys = the
+  prompt itself).
 """
 from __future__ import annotations
 
@@ -27,7 +27,7 @@ import torch
 
 from . import _native as N
 from . import kernels as K
-from .layers import Geometry
+from .layers import Geometry, StreamContext, clean_layer
 
 
 class BlockKVCache:
@@ -64,9 +64,7 @@ class BlockDecoder:
         [B, P, V] and commits all P rows."""
         if int(cache.lengths.max()) != 0:
             raise RuntimeError("prefill expects empty caches")
-        B, P = prompt_ids.shape
-        gate = torch.zeros((B, P), device=prompt_ids.device, dtype=torch.bool)
-        return self._forward(cache, prompt_ids, gate, commit=P, prefill=True)
+        return self._forward(cache, prompt_ids, None, commit=prompt_ids.shape[1], prefill=True)
 
     @torch.no_grad()
     def draft_block(self, cache: BlockKVCache, block_ids: torch.Tensor, lora_mask: torch.Tensor | None = None,
@@ -90,7 +88,7 @@ class BlockDecoder:
         return DraftGraph(self, cache, block_size, commit)
 
     # ---- the decoder -----------------------------------------------------------------------------
-    def _forward(self, cache: BlockKVCache, ids: torch.Tensor, gate: torch.Tensor, commit: int, prefill: bool,
+    def _forward(self, cache: BlockKVCache, ids: torch.Tensor, gate: torch.Tensor | None, commit: int, prefill: bool,
                  check: bool = True):
         g, lora, dec = self.geo, self.lora, self.decoder
         B, L = ids.shape
@@ -104,17 +102,19 @@ class BlockDecoder:
             raise NotImplementedError(f"draft blocks hold at most 128 / {rep} rows per sequence (got {L})")
         dev = ids.device
         M = B * L
-        gate_rows = gate.reshape(-1).contiguous()
         h = K.embedding(ids.reshape(-1).contiguous().to(torch.int64), dec.embed_tokens.weight)
-        if not prefill and self._split_path(dev, cache) and self._rows_path(M, h.dtype, prefill):
-            h = self._draft_layers(h, cache, gate_rows, B, L)
+        if prefill:
+            h = self._prefill_layers(h, cache, B, L)
+        elif self._split_path(dev, cache) and self._rows_path(M, h.dtype, prefill):
+            h = self._draft_layers(h, cache, gate.reshape(-1).contiguous(), B, L)
         else:
+            gate_rows = gate.reshape(-1).contiguous()
             j = torch.arange(L, device=dev)
             pos = (lengths[:, None] + j[None, :]).reshape(-1).contiguous()            # [M] int64
-            maps = self._maps(cache, lengths, B, L, prefill)
+            maps = self._maps(cache, lengths, B, L)
             for li, layer in enumerate(dec.layers):
                 lw = layer.weights()
-                h = self._layer(h, lw, li, pos, gate_rows, cache, maps, B, L, prefill)
+                h = self._layer(h, lw, li, pos, gate_rows, cache, maps, B, L)
         x, _ = K.rmsnorm_fwd(h, dec.norm.weight, g.eps)
         V = self.base.lm_head.weight.shape[0]
         head = K.gemm_nt_rows if self._rows_path(M, x.dtype, prefill) and V % 4 == 0 else K.gemm_nt
@@ -122,14 +122,35 @@ class BlockDecoder:
         cache.lengths += commit
         return logits.view(B, L, -1)
 
-    def _maps(self, cache, lengths, B, L, prefill):
+    def _prefill_layers(self, h, cache, B: int, P: int):
+        """All layers over B prompts of P tokens into empty caches: the clean stream's layer (no LoRA rows,
+        so no adapter products), its K and V copied into the cache rows (b, head, t)."""
+        g, dec, dev = self.geo, self.decoder, h.device
+        t = torch.arange(P, device=dev)
+        b = torch.arange(B, device=dev)
+        iv = torch.zeros((B, P, 8), device=dev, dtype=torch.int32)
+        iv[..., 0] = b[:, None] * P
+        iv[..., 1] = b[:, None] * P + t + 1
+        kv = torch.arange(g.nk, device=dev)
+        store = ((b[:, None, None] * g.nk + kv) * cache.max_len + t[:, None]).reshape(-1).to(torch.int32)
+        sc = StreamContext(t.repeat(B), dec.inv_freq, None, iv.view(B * P, 8), [], [])
+        if h.dtype == torch.bfloat16 and g.d == 128:
+            sc.rope_cos, sc.rope_sin = K.rope_table(P, dec.inv_freq)
+        rows = B * P * g.nk
+        for li, layer in enumerate(dec.layers):
+            h, k, v = clean_layer(h, layer.weights(), g, sc)
+            K.rows_copy(k.reshape(rows, g.d), cache.k[li].view(-1, g.d), rows, dmap=store)
+            K.rows_copy(v.reshape(rows, g.d), cache.v[li].view(-1, g.d), rows, dmap=store)
+        return h
+
+    def _maps(self, cache, lengths, B, L):
         """Row maps of the cache store and of the decode query layout, and the key intervals."""
         g = self.geo
         dev = lengths.device
         i32 = dict(device=dev, dtype=torch.int32)
         rep = g.nq // g.nk
         out = {}
-        if not prefill and self._split_path(dev, cache):
+        if self._split_path(dev, cache):
             S = self._key_ranges(cache, B)
             out["ivs"], out["dst"] = K.decode_maps(lengths, B, L, g.nq, g.nk, cache.max_len, S)
             out["S"], out["QR"] = S, B * g.nk * 128
@@ -146,13 +167,6 @@ class BlockDecoder:
         kv = torch.arange(g.nk, device=dev)[None, None, :]
         # cache store: key row (b, t, head) of the block -> cache row (b, head, lengths_b + t)
         out["store"] = ((b * g.nk + kv) * cache.max_len + lengths[:, None, None] + t).reshape(-1).to(**i32)
-        if prefill:
-            starts = (torch.arange(B, device=dev) * L)[:, None]
-            iv = torch.zeros((B * L, 8), **i32)
-            iv[:, 0] = starts.expand(B, L).reshape(-1)
-            iv[:, 1] = (starts + torch.arange(1, L + 1, device=dev)[None, :]).reshape(-1)
-            out["iv"] = iv
-            return out
         # decode layout: query (b, t, head h = kv * rep + r) -> row (b * nk + kv) * 128 + r * L + t
         r = torch.arange(rep, device=dev)
         qrow = ((b * g.nk + kv)[..., None] * 128 + r[None, None, None, :] * L + t[..., None])   # [B, L, nk, rep]
@@ -216,7 +230,7 @@ class BlockDecoder:
         return (not prefill and dtype == torch.bfloat16 and M <= 512 and r % 8 == 0 and 3 * r <= 512
                 and all(k % 128 == 0 for k in (g.H, g.q, g.F)))
 
-    def _layer(self, h0, lw, li, pos, gate_rows, cache, maps, B, L, prefill):
+    def _layer(self, h0, lw, li, pos, gate_rows, cache, maps, B, L):
         g, lora = self.geo, self.lora
         r = lora.rank
         q_end, k_end = g.q, g.q + g.kv
@@ -233,7 +247,7 @@ class BlockDecoder:
         qkv = linear(x1, lw.w_qkv, "qkv", qkv_segments)
         ck = cache.k[li].view(-1, g.d)
         cv = cache.v[li].view(-1, g.d)
-        if not prefill and "ivs" in maps:
+        if "ivs" in maps:
             # q/k norm + RoPE, cache store and query layout in one kernel; split-key attention; merge
             S, QR = maps["S"], maps["QR"]
             qd = torch.empty((QR, g.d), device=qkv.device, dtype=qkv.dtype)
@@ -248,15 +262,12 @@ class BlockDecoder:
         # the block's K/V into the cache rows (b, head, cached + t)
         K.rows_copy(k.reshape(M * g.nk, g.d), ck, M * g.nk, dmap=maps["store"])
         K.rows_copy(v.contiguous().view(M * g.nk, g.d), cv, M * g.nk, dmap=maps["store"])
-        if prefill:
-            o, _ = K.attn_fwd(q, k, v, maps["iv"], g.nq, g.nk, g.d)
-        else:
-            rows = maps["iv"].shape[0]
-            qd = torch.zeros((rows, g.d), device=q.device, dtype=q.dtype)
-            K.rows_copy(q.reshape(M * g.nq, g.d), qd, M * g.nq, dmap=maps["qrow"])
-            od, _ = K.attn_fwd(qd, ck, cv, maps["iv"], 1, 1, g.d)
-            o = torch.empty((M, g.q), device=q.device, dtype=q.dtype)
-            K.rows_copy(od, o.view(M * g.nq, g.d), M * g.nq, smap=maps["qrow"])
+        rows = maps["iv"].shape[0]
+        qd = torch.zeros((rows, g.d), device=q.device, dtype=q.dtype)
+        K.rows_copy(q.reshape(M * g.nq, g.d), qd, M * g.nq, dmap=maps["qrow"])
+        od, _ = K.attn_fwd(qd, ck, cv, maps["iv"], 1, 1, g.d)
+        o = torch.empty((M, g.q), device=q.device, dtype=q.dtype)
+        K.rows_copy(od, o.view(M * g.nq, g.d), M * g.nq, smap=maps["qrow"])
         return self._mlp(o, h0, lw, li, linear)
 
     def _mlp(self, o, h0, lw, li, linear):
