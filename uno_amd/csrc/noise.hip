@@ -50,40 +50,52 @@ struct BdArgs {
   int64_t* noisy_ids; int64_t* clean_ids;                      // [B*L] token ids per stream row
 };
 
-// One workgroup per batch row. Segment starts/ends come from a chunked scan. REGION_ONLY writes
-// just the [noisy | clean] region mask (the layout step that precedes noising).
+// Workgroups (row, part): every one scans its whole row for segment starts, in 1024 chunks, and then
+// writes 1024 tokens of it, one per thread, looking up its segment from the chunk's carries and a walk
+// within the chunk. Bound by latency: one workgroup writing a whole row took 99 us for 8192 tokens
+// and 42 us for 4 x 4096, most of it token after token in one thread, and the carries' serial scan
+// 15 us. REGION_ONLY writes just the [noisy | clean] region mask (the layout step that precedes
+// noising).
 template <bool REGION_ONLY>
 __global__ __launch_bounds__(1024) void bd_prepare_kernel(const BdArgs a) {
   __shared__ int carry_start[1024];
   __shared__ int carry_end[1024];
-  const int b = blockIdx.x, L = a.L, tid = threadIdx.x;
+  __shared__ int wave_start[16], wave_end[16];
+  const int b = blockIdx.x, L = a.L, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int chunk = (L + 1023) / 1024;
-  const int c0 = min(L, tid * chunk), c1 = min(L, c0 + chunk);
   const int64_t* pos = a.pos + (int64_t)b * L;
-  int last_start = -1, first_start = INT_MAX;
-  for (int t = c0; t < c1; ++t) {
-    const bool st = (t == 0) || (pos[t - 1] >= pos[t]);
-    if (st) { last_start = t; if (first_start == INT_MAX) first_start = t; }
-  }
-  carry_start[tid] = last_start;
-  carry_end[tid] = first_start;
-  __syncthreads();
-  if (tid == 0) {
-    int run = -1;
-    for (int i = 0; i < 1024; ++i) { const int v = carry_start[i]; carry_start[i] = run; if (v > run) run = v; }
-    int runm = L;
-    for (int i = 1023; i >= 0; --i) { const int v = carry_end[i]; carry_end[i] = runm; if (v < runm) runm = v; }
+  {
+    const int c0 = min(L, tid * chunk), c1 = min(L, c0 + chunk);
+    int last = -1, first = L;
+    for (int t = c0; t < c1; ++t) {
+      const bool st = (t == 0) || (pos[t - 1] >= pos[t]);
+      if (st) { last = t; first = min(first, t); }
+    }
+    // last start up to the chunk (running maximum) and first start from the chunk on (running minimum
+    // from the end), within the wave and then over the waves
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int u = __shfl_up(last, d, 64), v = __shfl_down(first, d, 64);
+      if (lane >= d) last = max(last, u);
+      if (lane + d < 64) first = min(first, v);
+    }
+    if (lane == 63) wave_start[wid] = last;
+    if (lane == 0) wave_end[wid] = first;
+    const int before = __shfl_up(last, 1, 64), after = __shfl_down(first, 1, 64);
+    __syncthreads();
+    int s = lane > 0 ? before : -1, e = lane < 63 ? after : L;
+    for (int w = 0; w < wid; ++w) s = max(s, wave_start[w]);
+    for (int w = wid + 1; w < 16; ++w) e = min(e, wave_end[w]);
+    carry_start[tid] = s;
+    carry_end[tid] = e;
   }
   __syncthreads();
   // carry_start[i]: last segment start before chunk i; carry_end[i]: first start after chunk i.
-  // Within a chunk (L/1024 tokens) the next start is found by a short forward walk.
-  int seg_s = carry_start[tid];
-  const int next_start = carry_end[tid];
-  for (int t = c0; t < c1; ++t) {
-    const bool st = (t == 0) || (pos[t - 1] >= pos[t]);
-    if (st) seg_s = t;
-    // segment end: first start > t
-    int e = next_start;
+  for (int64_t tt = (int64_t)blockIdx.y * 1024 + tid; tt < L; tt += (int64_t)gridDim.y * 1024) {
+    const int t = (int)tt, ch = t / chunk, c0 = ch * chunk, c1 = min(L, c0 + chunk);
+    int seg_s = carry_start[ch], e = carry_end[ch];
+    for (int u = t; u >= c0; --u)
+      if (u == 0 || pos[u - 1] >= pos[u]) { seg_s = u; break; }
     for (int u = t + 1; u < c1; ++u)
       if (pos[u - 1] >= pos[u]) { e = u; break; }
     const int64_t base2 = (int64_t)b * 2 * L;
@@ -183,6 +195,12 @@ __global__ __launch_bounds__(1024) void bd_compact_kernel(const uint8_t* __restr
     if (noised[i]) p_mask[o++] = tfull[i];
 }
 
+// Parts of a row: 1024 tokens each (64 parts at most; the tokens of longer rows are strided over them).
+static unsigned bd_parts(int L) {
+  const int n = (L + 1023) / 1024;
+  return (unsigned)(n < 64 ? n : 64);
+}
+
 UNOK_EXPORT int unok_bd_prepare(int B, int L, const int64_t* ids, const int64_t* pos, const uint8_t* prompt,
                                 int block_size, int mask_id, int noise_mask_mode, int intra_causal, uint64_t key,
                                 int64_t* concat_ids, int64_t* concat_pos, uint8_t* region, uint8_t* noised,
@@ -196,7 +214,7 @@ UNOK_EXPORT int unok_bd_prepare(int B, int L, const int64_t* ids, const int64_t*
   BdArgs a{ids, pos, prompt, B, L, block_size, mask_id, noise_mask_mode, intra_causal, key,
            concat_ids, concat_pos, region, noised, tfull, noisy_src, clean_src, noisy_iv, clean_iv, noisy_ids,
            clean_ids};
-  hipLaunchKernelGGL(bd_prepare_kernel<false>, dim3(B), dim3(1024), 0, (hipStream_t)stream, a);
+  hipLaunchKernelGGL(bd_prepare_kernel<false>, dim3(B, bd_parts(L)), dim3(1024), 0, (hipStream_t)stream, a);
   return unok::check_launch("bd_prepare");
 }
 
@@ -206,7 +224,7 @@ UNOK_EXPORT int unok_bd_region(int B, int L, const int64_t* pos, uint8_t* region
   UNOK_REQUIRE((int64_t)B * 2 * L < INT32_MAX, UNOK_EINVAL, "bd_region: batch too large");
   BdArgs a{};
   a.pos = pos; a.B = B; a.L = L; a.bs = 1; a.region = region;
-  hipLaunchKernelGGL(bd_prepare_kernel<true>, dim3(B), dim3(1024), 0, (hipStream_t)stream, a);
+  hipLaunchKernelGGL(bd_prepare_kernel<true>, dim3(B, bd_parts(L)), dim3(1024), 0, (hipStream_t)stream, a);
   return unok::check_launch("bd_region");
 }
 
