@@ -443,9 +443,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_f32_kernel(const GemmNT p) {
   __shared__ __attribute__((aligned(16))) float red[NW][T * LD];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, lr = lane & 15, lg = lane >> 4;
   const int n0 = blockIdx.x * T;
-  const int64_t mt = (int64_t)blockIdx.z * gridDim.y + blockIdx.y;
-  if (mt * T >= p.M) return;
-  const int m0 = (int)mt * T;
+  const int m0 = blockIdx.y * T;
   const bool ext = p.A2 != nullptr && p.K2 > 0;
   const int n1 = (p.K + 15) / 16, n = n1 + (ext ? (p.K2 + 15) / 16 : 0);
   const float* A2 = ext ? (const float*)p.A2 + seg_col_of(p, n0) : nullptr;
@@ -484,6 +482,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_f32_kernel(const GemmNT p) {
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // each group's 64 products are summed on their own and then added: a chain through the whole K walk
+  // loses more than the sums of the 64x64 kernel did (1.2e-6 relative at K = 4096)
   f32x4_t a[2][G][2], b[2][G][2];
   const int ngroup = (n + G * NW - 1) / (G * NW);
   auto load_group = [&](int g, f32x4_t (&ga)[G][2], f32x4_t (&gb)[G][2]) {
@@ -491,6 +491,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_f32_kernel(const GemmNT p) {
     for (int q = 0; q < G; ++q) load((g * G + q) * NW + wid, ga[q], gb[q]);
   };
   auto multiply = [&](const f32x4_t (&ga)[G][2], const f32x4_t (&gb)[G][2]) {
+    f32x4_t part[2][2];
 #pragma unroll
     for (int q = 0; q < G; ++q)
 #pragma unroll
@@ -499,7 +500,12 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_f32_kernel(const GemmNT p) {
         for (int i = 0; i < 2; ++i)
 #pragma unroll
           for (int j = 0; j < 2; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(gb[q][j][e], ga[q][i][e], acc[i][j], 0, 0, 0);
+            part[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                gb[q][j][e], ga[q][i][e], q || e ? part[i][j] : f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] += part[i][j];
   };
   load_group(0, a[0], b[0]);
   for (int g = 0; g < ngroup; g += 2) {
@@ -527,6 +533,68 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_f32_kernel(const GemmNT p) {
     v = on ? v * p.alpha : 0.f;
     if (R) v += ld_f(R + (int64_t)row * p.ldr + col);
     Elem<OutT>::store(C + (int64_t)row * p.ldc + col, v);
+  }
+}
+
+// fp32 NT kernel for products of many tiles: 64x64 tiles, 16-deep K slices, 4x4 outputs per thread, each
+// summed over ascending k in one chain, as a sequential fp32 product is (which it matches to 1e-6 at
+// K = 4096, where the kernel above lies closer to the exact sum than to that).
+template <typename OutT>
+__global__ __launch_bounds__(256) void gemm_nt_f32_tile64_kernel(const GemmNT p) {
+  __shared__ float As[16][65], Bs[16][65];
+  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
+  const float* A = (const float*)p.A;
+  const float* B = (const float*)p.B;
+  const float* A2 = nullptr;
+  if (p.A2 != nullptr && p.K2 > 0) A2 = (const float*)p.A2 + seg_col_of(p, n0);
+  const float* B2 = (const float*)p.B2;
+  float acc[4][4] = {};
+  for (int part = 0; part < 2; ++part) {
+    const float* a = part ? A2 : A;
+    const float* b = part ? B2 : B;
+    if (a == nullptr) continue;
+    const int64_t la = part ? p.lda2 : p.lda, lb = part ? p.ldb2 : p.ldb;
+    const int K = part ? p.K2 : p.K;
+    for (int k0 = 0; k0 < K; k0 += 16) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int e = tid + 256 * q, r = e >> 4, k = e & 15;
+        const int gm = m0 + r, gn = n0 + r, gk = k0 + k;
+        As[k][r] = (gm < p.M && gk < K) ? a[(int64_t)gm * la + gk] : 0.f;
+        Bs[k][r] = (gn < p.N && gk < K) ? b[(int64_t)gn * lb + gk] : 0.f;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        float av[4], bv[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) av[i] = As[k][ty + 16 * i];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bv[j] = Bs[k][tx + 16 * j];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
+      }
+      __syncthreads();
+    }
+  }
+  OutT* C = (OutT*)p.C;
+  const OutT* R = (const OutT*)p.R;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = m0 + ty + 16 * i;
+    if (row >= p.M) continue;
+    const bool on = (p.gate == nullptr) || (p.gate[row] != 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int col = n0 + tx + 16 * j;
+      if (col >= p.N) continue;
+      float v = on ? acc[i][j] * p.alpha : 0.f;
+      if (R) v += ld_f(R + (int64_t)row * p.ldr + col);
+      Elem<OutT>::store(C + (int64_t)row * p.ldc + col, v);
+    }
   }
 }
 
@@ -670,10 +738,14 @@ __global__ __launch_bounds__(256) void gemm_tn_f32_kernel(const GemmTN p) {
         }
       }
     }
+    f32x4_t part[4];   // summed on their own, as the NT kernel's groups
 #pragma unroll
     for (int g = 0; g < G; ++g)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[g][e], v[g], acc[e], 0, 0, 0);
+      for (int e = 0; e < 4; ++e)
+        part[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[g][e], v[g], g ? part[e] : f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] += part[e];
   }
   // acc[e][q] of lane l: X column 16 (l / 16) + 4 q + e, S column l % 16
 #pragma unroll
@@ -1900,11 +1972,18 @@ UNOK_EXPORT int unok_lmhead_ce_grad(int R, int V, int K, const void* H, int64_t 
 }
 
 // fp32 products: eight waves share the K walk of a tile where it is long (230 rows, 4096 -> 256: 581 us
-// on 64x64 tiles, 40 us here; its 64 tiles leave most CUs idle), four else.
+// on 64x64 tiles, 40 us here; its 64 tiles leave most CUs idle), four else. From eight 64x64 tiles per CU
+// on the latency that this divides is covered by other workgroups, and the 64x64 kernel keeps the
+// sums' order.
 template <typename OutT, bool VEC>
 static void launch_nt_f32_t(const GemmNT& p, hipStream_t st) {
-  const unsigned nM = (unsigned)((p.M + F32_T - 1) / F32_T), my = nM < 32768 ? nM : 32768;
-  const dim3 grid((unsigned)((p.N + F32_T - 1) / F32_T), my, (nM + my - 1) / my);
+  const int64_t big = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64);
+  if (big >= 2048) {
+    const dim3 grid64((p.N + 63) / 64, (p.M + 63) / 64);
+    hipLaunchKernelGGL((gemm_nt_f32_tile64_kernel<OutT>), grid64, dim3(256), 0, st, p);
+    return;
+  }
+  const dim3 grid((p.N + F32_T - 1) / F32_T, (p.M + F32_T - 1) / F32_T);   // below 8192 tiles: M < 2^17
   if (p.K >= 1024) hipLaunchKernelGGL((gemm_nt_f32_kernel<OutT, VEC, 8>), grid, dim3(512), 0, st, p);
   else hipLaunchKernelGGL((gemm_nt_f32_kernel<OutT, VEC, 4>), grid, dim3(256), 0, st, p);
 }
