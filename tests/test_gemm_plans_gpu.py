@@ -166,3 +166,51 @@ def test_qkv_rope_on_any_row_count(dev, M, nq, nk, norm, lora):
     for i, (a, b) in enumerate(zip(got, ref)):
         if i != 3 or norm:      # rstd is written with a norm only
             assert torch.equal(a, b[:M]), i
+
+
+@pytest.mark.parametrize("M,Nn,Kd", [(1, 256, 64), (192, 256, 128), (193, 300, 192), (575, 516, 448)])
+@pytest.mark.parametrize("ranges", [1, 2])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_192_row_tiles(dev, M, Nn, Kd, ranges, out_dtype):
+    """192x256 tiles (plan 6) at row and column remainders, with residual and row gate, bit for bit the
+    256x256 tiles' result in one range (the same K order per output)."""
+    if ranges > Kd // 64:
+        pytest.skip("fewer K tiles than ranges")
+    print(f"[192] {M}x{Nn}x{Kd} ranges {ranges} {out_dtype}", flush=True)
+    torch.manual_seed(M + Nn)
+    a, b = torch.randn(M, Kd, device=dev).bfloat16(), torch.randn(Nn, Kd, device=dev).bfloat16()
+    res = torch.randn(M, Nn, device=dev).to(out_dtype)
+    gate = torch.rand(M, device=dev) > 0.3
+    outs = []
+    for tile in (6, 1):
+        out = torch.empty(M, Nn, device=dev, dtype=out_dtype)
+        _call(tile + 16 * ranges, a, b, None, None, [(Nn, 0)], out, res, gate, 0.5, ranges)
+        outs.append(out)
+    ref = 0.5 * (a.float() @ b.float().T) * gate[:, None] + res.float()
+    assert _rel(outs[0], ref) < (1e-5 if out_dtype == torch.float32 else 4e-3)
+    assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("M", [720, 777])
+def test_192_row_tiles_fused_epilogues(dev, M):
+    """The fused products at a row count for which 192-row tiles are the cheapest, against the separate
+    kernels: SwiGLU and its backward bit for bit, q|k|v with norm and RoPE to one bf16 rounding."""
+    torch.manual_seed(M)
+    H, F, nq, nk = 1024, 12288, 32, 8
+    x = torch.randn(M, H, device=dev).bfloat16()
+    w = (torch.randn(2 * F, H, device=dev) * 0.05).bfloat16()
+    gu = torch.empty(M, 2 * F, device=dev, dtype=torch.bfloat16)
+    s = K.gemm_nt_swiglu(x, K.interleave_gate_up(w, F), gu=gu, any_rows=True)
+    assert torch.equal(gu, K.gemm_nt(x, w)) and torch.equal(s, K.swiglu_fwd(gu, F))
+    assert torch.equal(s, K.gemm_nt_swiglu(x, K.interleave_gate_up(w, F), any_rows=True))
+    wt = (torch.randn(F, H, device=dev) * 0.05).bfloat16()
+    assert torch.equal(K.gemm_nt_swiglu_bwd(x, wt, None, None, gu, any_rows=True), K.swiglu_bwd(K.gemm_nt(x, wt), gu, F))
+    wq, wk = (1 + 0.1 * torch.randn(2, 128, device=dev)).bfloat16()
+    wqkv = (torch.randn(128 * (nq + 2 * nk), H, device=dev) * 0.05).bfloat16()
+    inv = 1.0 / (1e6 ** (torch.arange(0, 128, 2, device=dev).float() / 128))
+    pos = torch.randint(0, 500, (M,), device=dev)
+    q, k, v, _, _ = K.gemm_nt_qkv_rope(x, wqkv, nq, nk, wq, wk, pos, *K.rope_table(500, inv), 1e-6, any_rows=True)
+    q2, k2, v2, _ = K.qknorm_rope_fwd(K.gemm_nt(x, wqkv, out_dtype=torch.float32), nq, nk, 128, wq, wk, pos, inv, 1e-6,
+                                      out_dtype=torch.bfloat16, with_v=True)
+    for got, want in ((q, q2), (k, k2), (v, v2)):
+        assert _rel(got, want) < 1e-3

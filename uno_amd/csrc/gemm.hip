@@ -861,6 +861,8 @@ static bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
 template <typename OutT, int EPI = 0, int BM = 256, int BN = 256>
 __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p) {
   constexpr int BK = 64, NW = 4, WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
+  constexpr int HR = WM % 64 == 0 ? 64 : 48;    // rows an fp32 epilogue stages per wave at a time
+  static_assert(WM % HR == 0, "row tile");
   constexpr int CPR = BK / 8, RPI = 64 / CPR;
   constexpr int AI = BM / (RPI * NW), BI = BN / (RPI * NW);   // loads per wave and tile of A and of B
   static_assert(EPI == 0 || EPI == 6 || WN == 128, "the fused epilogues take 128 columns per wave");
@@ -1416,25 +1418,25 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
       }
     }
     asm volatile("s_barrier" ::: "memory");   // every wave's fragment reads have completed
-    float* q = (float*)smem + wid * 64 * 128;
+    float* q = (float*)smem + wid * HR * 128;
     auto body = [&](auto chk) {
     constexpr bool CHK = decltype(chk)::value;
 #pragma unroll
-    for (int h = 0; h < WM / 64; ++h) {
+    for (int h = 0; h < WM / HR; ++h) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < HR / 16; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
           const int r = i * 16 + lr;
           f32x4_t v;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = acc[4 * h + i][j][e] * p.alpha;
+          for (int e = 0; e < 4; ++e) v[e] = acc[HR / 16 * h + i][j][e] * p.alpha;
           *(f32x4_t*)&q[r * 128 + (((4 * j + lk) ^ (r & 15)) << 2)] = v;
         }
       __builtin_amdgcn_s_waitcnt(0xC07F);
       __builtin_amdgcn_wave_barrier();
 #pragma unroll 2
-      for (int it = 0; it < 8; ++it) {
+      for (int it = 0; it < HR / 8; ++it) {
         const int r = it * 8 + rsub;
         float x[16];
 #pragma unroll
@@ -1444,7 +1446,7 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
 #pragma unroll
           for (int e = 0; e < 4; ++e) x[4 * c + e] = v[e];
         }
-        const int64_t row = rowb + 64 * h + it * 8;
+        const int64_t row = rowb + HR * h + it * 8;
         if (CHK && row >= p.M) break;   // a row's eight lanes leave together; its later rows are past M too
         float out[16];
         if (isv) {
@@ -1513,35 +1515,35 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
   if constexpr (EPI == 0 && std::is_same<OutT, bf16_t>::value) {
     if (interior && (p.ldc & 7) == 0 && (!R || (p.ldr & 7) == 0)) {
       // Interior tile with bf16 output: each wave stages its WM x WN fp32 quadrant (alpha
-      // applied) through a private part of the idle LDS stages, 64 rows at a time, and stores by
+      // applied) through a private part of the idle LDS stages, HR rows at a time, and stores by
       // rows: WN / 8 lanes per row, 8 columns (16 bytes) each, the residual read the same way. 16-byte
       // chunk c of staged row r sits at slot c ^ (r & 15). The residual rows of both halves are
       // loaded first, into the registers the K loop's fragments held, so their latency passes
       // once, behind the staging, instead of once per group of rows.
-      constexpr int LPR = WN / 8, RS = 64 / LPR, NIT = 64 / RS;
+      constexpr int LPR = WN / 8, RS = 64 / LPR, NIT = HR / RS;
       const int rsub = lane / LPR, c16 = lane % LPR;
       const int64_t rowb = m0 + wm * WM + rsub;
       const int col = n0 + wn * WN + 8 * c16;
-      uint4 rw[WM / 64][NIT];
+      uint4 rw[WM / HR][NIT];
       if (R) {
 #pragma unroll
-        for (int h = 0; h < WM / 64; ++h)
+        for (int h = 0; h < WM / HR; ++h)
 #pragma unroll
           for (int it = 0; it < NIT; ++it)
-            rw[h][it] = *(const uint4*)((const bf16_t*)R + (rowb + 64 * h + it * RS) * p.ldr + col);
+            rw[h][it] = *(const uint4*)((const bf16_t*)R + (rowb + HR * h + it * RS) * p.ldr + col);
       }
       asm volatile("s_barrier" ::: "memory");   // every wave's fragment reads have completed
-      float* q = (float*)smem + wid * 64 * WN;
+      float* q = (float*)smem + wid * HR * WN;
 #pragma unroll
-      for (int h = 0; h < WM / 64; ++h) {
+      for (int h = 0; h < WM / HR; ++h) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < HR / 16; ++i)
 #pragma unroll
           for (int j = 0; j < TN; ++j) {
             const int r = i * 16 + lr;
             f32x4_t v;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = acc[4 * h + i][j][e] * p.alpha;
+            for (int e = 0; e < 4; ++e) v[e] = acc[HR / 16 * h + i][j][e] * p.alpha;
             *(f32x4_t*)&q[r * WN + (((4 * j + lk) ^ (r & 15)) << 2)] = v;
           }
         __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -1551,7 +1553,7 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
           const int r = it * RS + rsub;
           const f32x4_t v0 = *(const f32x4_t*)&q[r * WN + (((2 * c16) ^ (r & 15)) << 2)];
           const f32x4_t v1 = *(const f32x4_t*)&q[r * WN + (((2 * c16 + 1) ^ (r & 15)) << 2)];
-          const int64_t row = rowb + 64 * h + it * RS;
+          const int64_t row = rowb + HR * h + it * RS;
           float a[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
           if (R) {
             const uint32_t* rp = (const uint32_t*)&rw[h][it];
@@ -1675,15 +1677,20 @@ __global__ __launch_bounds__(256) void nt_splitk_reduce_kernel(const GemmNT p, c
 // of the 256 CUs a partial round of tiles covers; fewer workgroups share the L2 and the power
 // budget, so each runs faster):
 //   256x256   one workgroup per CU: 1.41 n + 8 per full round, (0.95 + 0.46 f) n + 8 for the rest
+//   192x256   one per CU:           1.09 n + 9,                (0.81 + 0.28 f) n + 9, plus 3%: it has to
+//             beat 256x256 by more than the model's error (3000 x 24576 x 4096: 474 against 467)
 //   128x256   one per CU:           0.97 n + 6,                (0.77 + 0.20 f) n + 6
 //   128x128   one per CU 0.62 n + 5, two per CU (1.01 n + 4) per 512 tiles, not in lockstep
 //   ranges    a second kernel: 4 us and the fp32 partials written and read once at 6 TB/s
 // and never below the operands' bytes at 4.5 TB/s. It reproduces 2048 x 4096 x 4096 at 83 / 63 / 65
 // us for the three tiles, 4096 x 4096 x 4096 at 100 / 125 / 126, 777 x 4096 x 12288 at 208 / 177 /
 // 139 in one range and 92 in four 256x256 ranges, 1801 x 2048 x 151936 at 2459 in one range and 887
-// in four, and 128 x 4096 x 4096 at 38 in one range of 128x128 tiles and 18 in eight.
+// in four, 777 x 24576 x 4096 at 177 / 153 / 198 for 256, 192 and 128 rows (a quarter of the 256-row tiles'
+// work there is padding), 3072 x 4096 x 8192 at 161 / 150 / 204 (192, 256 and 384 tiles on 256 CUs), and
+// 128 x 4096 x 4096 at 38 in one range of 128x128 tiles and 18 in eight.
 // ---------------------------------------------------------------------------------------
-enum NtTile { NT_REG = 0, NT_256 = 1, NT_128_256 = 2, NT_128 = 3, NT_SKINNY = 4, NT_LARGE64 = 5 };
+enum NtTile { NT_REG = 0, NT_256 = 1, NT_128_256 = 2, NT_128 = 3, NT_SKINNY = 4, NT_LARGE64 = 5,
+              NT_192_256 = 6 };
 struct NtPlan { int tile, splits; };
 
 static bool nt_segs_ok(const GemmNT& p, int bn) {
@@ -1693,7 +1700,7 @@ static bool nt_segs_ok(const GemmNT& p, int bn) {
 }
 
 static double nt_cost(int tile, int64_t M, int64_t N, int nk1, int nk2, int s) {
-  const int64_t bm = tile == NT_256 ? 256 : 128, bn = tile == NT_128 ? 128 : 256;
+  const int64_t bm = tile == NT_256 ? 256 : tile == NT_192_256 ? 192 : 128, bn = tile == NT_128 ? 128 : 256;
   const int64_t wg = (M + bm - 1) / bm * ((N + bn - 1) / bn) * s;
   const double n = (nk1 + s - 1) / s + nk2;
   double t;
@@ -1701,9 +1708,13 @@ static double nt_cost(int tile, int64_t M, int64_t N, int nk1, int nk2, int s) {
     t = 0.62 * n + 5;
     if (wg > 256) t = fmax(t, (double)wg / 512 * (1.01 * n + 4) + 5);
   } else {
+    struct { double round, part0, part1, fixed; } c = {0.97, 0.77, 0.20, 6};
+    if (tile == NT_256) c = {1.41, 0.95, 0.46, 8};
+    else if (tile == NT_192_256) c = {1.09, 0.81, 0.28, 9};
     const double full = (double)(wg / 256), f = (double)(wg % 256) / 256;
-    t = tile == NT_256 ? full * (1.41 * n + 8) : full * (0.97 * n + 6);
-    if (f > 0) t += tile == NT_256 ? (0.95 + 0.46 * f) * n + 8 : (0.77 + 0.20 * f) * n + 6;
+    t = full * (c.round * n + c.fixed);
+    if (f > 0) t += (c.part0 + c.part1 * f) * n + c.fixed;
+    if (tile == NT_192_256) t *= 1.03;
   }
   t = fmax(t, (double)(M + N) * (nk1 + nk2) * 128 / 4.5e6);
   if (s > 1) t += 4 + (double)M * N * (8.0 * s + 2) / 6e6;
@@ -1712,10 +1723,15 @@ static double nt_cost(int tile, int64_t M, int64_t N, int nk1, int nk2, int s) {
 
 static int nt_ext_tiles(const GemmNT& p) { return p.A2 ? (p.K2 + 63) / 64 : 0; }
 
-// Row tile of a product whose epilogue needs 256-wide tiles and whole sums.
-static bool nt_rows128(const GemmNT& p) {
+// Launches a product whose epilogue needs 256-wide tiles and whole sums on the cheapest row tile.
+template <int EPI>
+static void launch_nt_fused(const GemmNT& p, hipStream_t st) {
   const int nk1 = p.K / 64, nk2 = nt_ext_tiles(p);
-  return nt_cost(NT_128_256, p.M, p.N, nk1, nk2, 1) < nt_cost(NT_256, p.M, p.N, nk1, nk2, 1);
+  const double t256 = nt_cost(NT_256, p.M, p.N, nk1, nk2, 1), t192 = nt_cost(NT_192_256, p.M, p.N, nk1, nk2, 1),
+               t128 = nt_cost(NT_128_256, p.M, p.N, nk1, nk2, 1);
+  if (t256 <= t192 && t256 <= t128) launch_nt_w4m16<bf16_t, EPI>(p, st);
+  else if (t192 <= t128) launch_nt_w4m16<bf16_t, EPI, 192>(p, st);
+  else launch_nt_w4m16<bf16_t, EPI, 128>(p, st);
 }
 
 static NtPlan nt_plan(const GemmNT& p, bool may_split) {
@@ -1748,7 +1764,8 @@ static NtPlan nt_plan(const GemmNT& p, bool may_split) {
   const bool wide = p.N > 128 && nt_segs_ok(p, 256);
   NtPlan best = {NT_128, 1};
   double best_t = 1e30;
-  for (int tile = wide ? NT_256 : NT_128; tile <= NT_128; ++tile) {
+  for (int tile : {NT_256, NT_192_256, NT_128_256, NT_128}) {
+    if (!wide && tile != NT_128) continue;
     for (int s = 1; s <= (may_split ? 16 : 1) && nk1 / s >= 4; ++s) {
       const double t = nt_cost(tile, p.M, p.N, nk1, nk2, s);
       if (t < best_t) { best_t = t; best = {tile, s}; }
@@ -1787,8 +1804,7 @@ static int swiglu_fwd_product(int M, int N, int K, const void* A, int64_t lda, c
   p.M = M; p.N = N; p.K = K; p.K2 = ext ? K2 : 0; p.alpha = 1.f; p.nseg = 1;
   for (int i = 0; i < 4; ++i) { p.seg_end[i] = N; p.seg_col[i] = 0; }
   UNOK_REQUIRE(buffer_ranges_ok(p), UNOK_EINVAL, "gemm_nt_swiglu: operands exceed 32-bit buffer offsets");
-  if (nt_rows128(p)) launch_nt_w4m16<bf16_t, 1, 128>(p, (hipStream_t)stream);
-  else launch_nt_w4m16<bf16_t, 1>(p, (hipStream_t)stream);
+  launch_nt_fused<1>(p, (hipStream_t)stream);
   return unok::check_launch("gemm_nt_swiglu");
 }
 
@@ -1851,8 +1867,7 @@ static int qkv_rope_product(int M, int K, int nq, int nk, const void* A, int64_t
   p.qk_wq = wq; p.qk_wk = wk; p.qk_pos = pos; p.qk_cos = cos_tab; p.qk_sin = sin_tab; p.qk_P = P;
   p.qk_nq = nq; p.qk_nk = nk; p.qk_eps = eps;
   UNOK_REQUIRE(buffer_ranges_ok(p), UNOK_EINVAL, "gemm_nt_qkv_rope: operands exceed 32-bit buffer offsets");
-  if (nt_rows128(p)) launch_nt_w4m16<bf16_t, 5, 128>(p, (hipStream_t)stream);
-  else launch_nt_w4m16<bf16_t, 5>(p, (hipStream_t)stream);
+  launch_nt_fused<5>(p, (hipStream_t)stream);
   return unok::check_launch("gemm_nt_qkv_rope");
 }
 
@@ -1897,8 +1912,7 @@ static int swiglu_bwd_product(int M, int F, int K, const void* A, int64_t lda, c
   p.M = M; p.N = F; p.K = K; p.K2 = p.A2 ? K2 : 0; p.alpha = 1.f; p.nseg = 1;
   for (int i = 0; i < 4; ++i) { p.seg_end[i] = F; p.seg_col[i] = 0; }
   UNOK_REQUIRE(buffer_ranges_ok(p), UNOK_EINVAL, "gemm_nt_swiglu_bwd: operands exceed 32-bit buffer offsets");
-  if (nt_rows128(p)) launch_nt_w4m16<bf16_t, 2, 128>(p, (hipStream_t)stream);
-  else launch_nt_w4m16<bf16_t, 2>(p, (hipStream_t)stream);
+  launch_nt_fused<2>(p, (hipStream_t)stream);
   return unok::check_launch("gemm_nt_swiglu_bwd");
 }
 
@@ -2043,7 +2057,7 @@ static int gemm_nt_any(int in_dtype, int out_dtype, int M, int N, int K,
   NtPlan pl = nt_plan(p, ws != nullptr);
   if (plan > 0) {
     const int tile = plan & 15, n = plan >> 4;
-    const bool tiles = tile >= NT_256 && tile <= NT_128 && K > 0 && K % 64 == 0 && (!p.A2 || K2 % 32 == 0) &&
+    const bool tiles = ((tile >= NT_256 && tile <= NT_128) || tile == NT_192_256) && K > 0 && K % 64 == 0 && (!p.A2 || K2 % 32 == 0) &&
                        nt_segs_ok(p, tile == NT_128 ? 128 : 256) && buffer_ranges_ok(p);
     const bool skinny = tile == NT_SKINNY && N <= 192 && !p.A2 && K > 0 && K % 64 == 0;
     UNOK_REQUIRE((tiles || skinny) && n >= 1 && n <= K / 64 && (n == 1 || (ws && out_vec4_ok(p) && (int64_t)M * N < (1ll << 32))),
@@ -2059,6 +2073,7 @@ static int gemm_nt_any(int in_dtype, int out_dtype, int M, int N, int K,
     q.C = ws; q.ldc = N; q.R = nullptr; q.gate = nullptr; q.alpha = 1.f;
     if (pl.tile == NT_SKINNY) launch_nt_skinny(q, UNOK_F32, st);
     else if (pl.tile == NT_256) launch_nt_w4m16<float, 6, 256, 256>(q, st);
+    else if (pl.tile == NT_192_256) launch_nt_w4m16<float, 6, 192, 256>(q, st);
     else if (pl.tile == NT_128_256) launch_nt_w4m16<float, 6, 128, 256>(q, st);
     else launch_nt_w4m16<float, 6, 128, 128>(q, st);
     const int rc = unok::check_launch("gemm_nt_splits");
@@ -2072,6 +2087,9 @@ static int gemm_nt_any(int in_dtype, int out_dtype, int M, int N, int K,
   switch (pl.tile) {
     case NT_SKINNY: launch_nt_skinny(p, out_dtype, st); break;
     case NT_256: if (f32) launch_nt_w4m16<float>(p, st); else launch_nt_w4m16<bf16_t>(p, st); break;
+    case NT_192_256:
+      if (f32) launch_nt_w4m16<float, 0, 192, 256>(p, st); else launch_nt_w4m16<bf16_t, 0, 192, 256>(p, st);
+      break;
     case NT_128_256:
       if (f32) launch_nt_w4m16<float, 0, 128, 256>(p, st); else launch_nt_w4m16<bf16_t, 0, 128, 256>(p, st);
       break;
