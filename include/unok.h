@@ -70,10 +70,11 @@ int unok_gemm_nt_ws(int in_dtype, int out_dtype, int M, int N, int K,
 int unok_gemm_nt_swiglu(int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
                         const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
                         void* C, int64_t ldc, void* gu, int64_t ldgu, void* stream);
-/* The same for any number of rows. */
+/* The same for any number of rows. plain_rows != 0: B holds its N/2 gate rows and then its N/2 up rows,
+ * as a fused projection stores them (B2 stays interleaved). */
 int unok_gemm_nt_swiglu_any(int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
                         const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
-                        void* C, int64_t ldc, void* gu, int64_t ldgu, void* stream);
+                        void* C, int64_t ldc, void* gu, int64_t ldgu, int plain_rows, void* stream);
 
 /* dgu[M, 2F] = SwiGLU backward of dS = A[M,K] B[F,K]^T + A2[M,K2] B2[F,K2]^T against
  * gu[M, 2F] = [gate | up] (dS is never stored); bf16, rounded exactly as unok_gemm_nt followed by

@@ -214,3 +214,22 @@ def test_192_row_tiles_fused_epilogues(dev, M):
                                       out_dtype=torch.bfloat16, with_v=True)
     for got, want in ((q, q2), (k, k2), (v, v2)):
         assert _rel(got, want) < 1e-3
+
+
+@pytest.mark.parametrize("M,F,Kd,r", [(5, 256, 128, 0), (300, 1536, 512, 32), (777, 12288, 1024, 0), (2100, 5632, 320, 64)])
+def test_swiglu_product_on_the_fused_projection_rows(dev, M, F, Kd, r):
+    """The SwiGLU product reading [gate; up] weight rows as they are stored: bit for bit the one over
+    interleaved rows, with and without an extension and the stored [gate | up]."""
+    torch.manual_seed(M + F)
+    bf = torch.bfloat16
+    x, w = (torch.randn(M, Kd, device=dev) * 0.5).to(bf), (torch.randn(2 * F, Kd, device=dev) * 0.1).to(bf)
+    kw = {}
+    if r:
+        kw = dict(a2=(torch.randn(M, 2 * r, device=dev) * 0.5).to(bf),
+                  b2_interleaved=(torch.randn(2 * F, 2 * r, device=dev) * 0.1).to(bf))
+    gus = [torch.empty(M, 2 * F, device=dev, dtype=bf) for _ in range(2)]
+    wi = K.interleave_gate_up(w, F)
+    ref = K.gemm_nt_swiglu(x, wi, gu=gus[0], any_rows=True, **kw)
+    got = K.gemm_nt_swiglu(x, w, gu=gus[1], any_rows=True, plain_rows=True, **kw)
+    assert torch.equal(got, ref) and torch.equal(*gus)
+    assert torch.equal(K.gemm_nt_swiglu(x, w, any_rows=True, plain_rows=True, **kw), ref)

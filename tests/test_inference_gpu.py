@@ -142,3 +142,35 @@ def test_draft_graph_replays_match_eager(dev, dtype):
     # longest committed length is now 41: one more block of 16 would need 57 > 56 rows
     with pytest.raises(RuntimeError, match="does not fit"):
         dg.replay(blk)
+
+
+@pytest.mark.parametrize("write", ["load_state_dict", "data"])
+def test_prefill_follows_in_place_weight_updates(dev, write):
+    """A prefill after base weights were written in place (load_state_dict, a write through .data), with
+    nothing rebuilt by the caller: bit for bit the prefill of a model that was loaded with them."""
+    s = SPECS["gqa4_d128"]
+    cfg = Cfg(s["vocab_size"], s["hidden_size"], s["intermediate_size"], s["num_hidden_layers"],
+              s["num_attention_heads"], s["num_key_value_heads"], s["head_dim"], lora_rank=s["rank"],
+              lora_alpha=s["alpha"])
+    ucfg = UnoQwen3Config(vocab_size=cfg.vocab_size, hidden_size=cfg.hidden_size,
+                          intermediate_size=cfg.intermediate_size, num_hidden_layers=cfg.num_hidden_layers,
+                          num_attention_heads=cfg.num_attention_heads, num_key_value_heads=cfg.num_key_value_heads,
+                          head_dim=cfg.head_dim, block_size=16)
+    models = []
+    for seed in (0, 5):
+        model = UnoQwen3ForCausalLM(ucfg, device=dev, dtype=torch.bfloat16)
+        model.load_weights(init_params(cfg, seed=seed))
+        models.append(model)
+    old, new = models
+    if write == "load_state_dict":
+        old.load_state_dict(new.state_dict())
+    else:
+        for p, q in zip(old.parameters(), new.parameters()):
+            p.data.copy_(q.data)
+    ids = torch.randint(0, cfg.vocab_size - 1, (2, 150), generator=torch.Generator().manual_seed(3)).to(dev)
+    logits = []
+    for model in models:
+        lm, _ = create_lora_model(model, LoraSettings("all", s["rank"], s["alpha"], 0.0))
+        dec = BlockDecoder(lm)
+        logits.append(dec.prefill(dec.new_cache(2, 256), ids))
+    assert torch.equal(*logits)

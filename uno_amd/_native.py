@@ -95,8 +95,9 @@ SIGNATURES: dict[str, tuple] = {
     "unok_transpose_jobs": (_i, [_i, _p, _i, _i64, _p, _p, _p]),
 }
 
-for _name in ("unok_gemm_nt_swiglu", "unok_gemm_nt_swiglu_bwd", "unok_gemm_nt_qkv_rope"):
+for _name in ("unok_gemm_nt_swiglu_bwd", "unok_gemm_nt_qkv_rope"):
     SIGNATURES[_name + "_any"] = SIGNATURES[_name]
+SIGNATURES["unok_gemm_nt_swiglu_any"] = (_i, [*SIGNATURES["unok_gemm_nt_swiglu"][1][:-1], _i, _p])
 
 _lock = threading.Lock()
 _lib = None

@@ -31,6 +31,7 @@ struct GemmNT {
   const void* R; int64_t ldr;
   const uint8_t* gate;
   void* C2; int64_t ldc2;          // second output of the SwiGLU forward epilogue (gate | up), or null
+  int gu_rows;                     // SwiGLU forward: F with B = [gate; up] of F rows each (0: B's rows interleaved)
   int group;                       // row tiles per tile group of the direct-to-LDS tile kernel (0: 8)
   int splits;                      // K ranges (0 or 1: none): the product writes fp32 partials [splits][M][N] to C
   int M, N, K, K2;
@@ -902,10 +903,16 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
   const int mrows = min(p.M - m0, BM), nrows = min(p.N - n0, BN);
   __amdgpu_buffer_rsrc_t ra = make_rsrc((const bf16_t*)p.A + (int64_t)m0 * p.lda,
                                         (uint32_t)(((int64_t)(mrows - 1) * p.lda + p.K) * 2));
-  __amdgpu_buffer_rsrc_t rb = make_rsrc((const bf16_t*)p.B + (int64_t)n0 * p.ldb,
-                                        (uint32_t)(((int64_t)(nrows - 1) * p.ldb + p.K) * 2));
+  // The SwiGLU forward epilogue reads gate and up features in alternating blocks of 64 columns. With
+  // gu_rows, B holds them as [gate; up] and the loads take the rows from there (the tile's 128 gate
+  // rows from n0 / 2 on and their up rows gu_rows further), so no rearranged copy of the weight exists
+  // that could fall behind it; the LDS tile and the products are the same.
+  const bool split_gu = EPI == 1 && p.gu_rows > 0;
+  const int b_first = split_gu ? n0 / 2 : n0, b_span = split_gu ? p.gu_rows + BN / 2 : nrows;
+  __amdgpu_buffer_rsrc_t rb = make_rsrc((const bf16_t*)p.B + (int64_t)b_first * p.ldb,
+                                        (uint32_t)(((int64_t)(b_span - 1) * p.ldb + p.K) * 2));
   uint32_t a_vo[AI], b_vo[BI];
-  auto set_offsets = [&](int64_t lda, int64_t ldb) {
+  auto set_offsets = [&](int64_t lda, int64_t ldb, bool gu) {
 #pragma unroll
     for (int i = 0; i < AI; ++i) {
       const int r = (i * NW + wid) * RPI + lrowi;
@@ -914,10 +921,11 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
 #pragma unroll
     for (int i = 0; i < BI; ++i) {
       const int r = (i * NW + wid) * RPI + lrowi;
-      b_vo[i] = (uint32_t)(((int64_t)min(r, nrows - 1) * ldb + (slot ^ dma_swz<BK>(r)) * 8) * 2);
+      const int br = gu ? (r >> 7) * 64 + (r & 63) + ((r >> 6) & 1) * p.gu_rows : min(r, nrows - 1);
+      b_vo[i] = (uint32_t)(((int64_t)br * ldb + (slot ^ dma_swz<BK>(r)) * 8) * 2);
     }
   };
-  set_offsets(p.lda, p.ldb);
+  set_offsets(p.lda, p.ldb, split_gu);
   int kbase = 0;
   // Sets up the operand pair of tile t (the LoRA pair from tile nk1 on; tiles are set up in
   // order, and every range starts before tile nk1) and returns its k byte offset.
@@ -926,7 +934,7 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
       ra = make_rsrc((const bf16_t*)p.A2 + seg_col_of(p, n0) + (int64_t)m0 * p.lda2,
                      (uint32_t)(((int64_t)(mrows - 1) * p.lda2 + p.K2) * 2));
       rb = make_rsrc((const bf16_t*)p.B2 + (int64_t)n0 * p.ldb2, (uint32_t)(((int64_t)(nrows - 1) * p.ldb2 + p.K2) * 2));
-      set_offsets(p.lda2, p.ldb2);
+      set_offsets(p.lda2, p.ldb2, false);
       kbase = nk1;
     }
     return (uint32_t)(t - kbase) * BK * 2;
@@ -1786,7 +1794,8 @@ static NtPlan nt_plan(const GemmNT& p, bool may_split) {
 // unfused product followed by unok_swiglu_fwd. M and N multiples of 256, K of 64.
 static int swiglu_fwd_product(int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
                                     const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
-                                    void* C, int64_t ldc, void* gu, int64_t ldgu, void* stream, int row_step) {
+                                    void* C, int64_t ldc, void* gu, int64_t ldgu, void* stream, int row_step,
+                                    bool plain_rows) {
   UNOK_REQUIRE(M >= 0 && N >= 0 && K >= 0 && K2 >= 0, UNOK_EINVAL, "gemm_nt_swiglu: negative size M=%d N=%d K=%d",
                M, N, K);
   if (M == 0 || N == 0) return 0;
@@ -1803,7 +1812,9 @@ static int swiglu_fwd_product(int M, int N, int K, const void* A, int64_t lda, c
   p.C = C; p.ldc = ldc; p.C2 = gu; p.ldc2 = ldgu;
   p.M = M; p.N = N; p.K = K; p.K2 = ext ? K2 : 0; p.alpha = 1.f; p.nseg = 1;
   for (int i = 0; i < 4; ++i) { p.seg_end[i] = N; p.seg_col[i] = 0; }
-  UNOK_REQUIRE(buffer_ranges_ok(p), UNOK_EINVAL, "gemm_nt_swiglu: operands exceed 32-bit buffer offsets");
+  if (plain_rows) p.gu_rows = N / 2;
+  UNOK_REQUIRE(buffer_ranges_ok(p) && ((int64_t)(p.gu_rows + 127) * p.ldb + p.K) * 2 <= 0xFFFFFFFFll, UNOK_EINVAL,
+               "gemm_nt_swiglu: operands exceed 32-bit buffer offsets");
   launch_nt_fused<1>(p, (hipStream_t)stream);
   return unok::check_launch("gemm_nt_swiglu");
 }
@@ -1811,14 +1822,17 @@ static int swiglu_fwd_product(int M, int N, int K, const void* A, int64_t lda, c
 UNOK_EXPORT int unok_gemm_nt_swiglu(int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
                                     const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
                                     void* C, int64_t ldc, void* gu, int64_t ldgu, void* stream) {
-  return swiglu_fwd_product(M, N, K, A, lda, B, ldb, A2, lda2, B2, ldb2, K2, C, ldc, gu, ldgu, stream, 256);
+  return swiglu_fwd_product(M, N, K, A, lda, B, ldb, A2, lda2, B2, ldb2, K2, C, ldc, gu, ldgu, stream, 256, false);
 }
 
-// unok_gemm_nt_swiglu for any number of rows.
+// unok_gemm_nt_swiglu for any number of rows; with plain_rows, B holds the N / 2 gate rows and then the
+// N / 2 up rows (B2 stays interleaved).
 UNOK_EXPORT int unok_gemm_nt_swiglu_any(int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
                                         const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
-                                        void* C, int64_t ldc, void* gu, int64_t ldgu, void* stream) {
-  return swiglu_fwd_product(M, N, K, A, lda, B, ldb, A2, lda2, B2, ldb2, K2, C, ldc, gu, ldgu, stream, 1);
+                                        void* C, int64_t ldc, void* gu, int64_t ldgu, int plain_rows,
+                                        void* stream) {
+  return swiglu_fwd_product(M, N, K, A, lda, B, ldb, A2, lda2, B2, ldb2, K2, C, ldc, gu, ldgu, stream, 1,
+                            plain_rows != 0);
 }
 
 // q|k|v projection with the q/k RMSNorm and RoPE in its epilogue (bf16, head dim 128): the product

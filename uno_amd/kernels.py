@@ -365,10 +365,14 @@ def gemm_nt_qkv_rope(x, w_qkv, nq, nk, wq, wk, pos, cos_tab, sin_tab, eps, *, a2
 
 def gemm_nt_swiglu(a: torch.Tensor, b_interleaved: torch.Tensor, *, a2: torch.Tensor | None = None,
                    b2_interleaved: torch.Tensor | None = None, gu: torch.Tensor | None = None,
-                   out: torch.Tensor | None = None, any_rows: bool = False) -> torch.Tensor:
+                   out: torch.Tensor | None = None, any_rows: bool = False, plain_rows: bool = False) -> torch.Tensor:
     """silu(gate) * up of a @ b.T (+ a2 @ b2.T) for gate/up weight rows interleaved in blocks of 64
     (``interleave_gate_up``; b2 likewise); bf16, M and the row count of b multiples of 256, K and
-    K2 = b2.shape[1] of 32 (with ``any_rows`` any M). With ``gu`` ([M, rows]), also stores the product as [gate | up]."""
+    K2 = b2.shape[1] of 32 (with ``any_rows`` any M). ``plain_rows`` (with ``any_rows``): b is [gate; up] as the
+    fused projection stores it (b2 stays interleaved). With ``gu`` ([M, rows]), also stores the product as
+    [gate | up]."""
+    if plain_rows and not any_rows:
+        raise RuntimeError("gemm_nt_swiglu: plain_rows goes with any_rows")
     _rowmajor(a, "a")
     _rowmajor(b_interleaved, "b")
     M, K = a.shape
@@ -394,10 +398,10 @@ def gemm_nt_swiglu(a: torch.Tensor, b_interleaved: torch.Tensor, *, a2: torch.Te
         ev0.record()
     else:
         rec = None
-    N.call("unok_gemm_nt_swiglu_any" if any_rows else "unok_gemm_nt_swiglu", M, rows, K, N.ptr(a), _ld(a), N.ptr(b_interleaved), _ld(b_interleaved),
-           N.ptr(a2), _ld(a2) if a2 is not None else 0, N.ptr(b2_interleaved),
-           _ld(b2_interleaved) if b2_interleaved is not None else 0, K2,
-           N.ptr(out), _ld(out), N.ptr(gu), _ld(gu) if gu is not None else 0, N.stream())
+    N.call("unok_gemm_nt_swiglu_any" if any_rows else "unok_gemm_nt_swiglu", M, rows, K, N.ptr(a), _ld(a),
+           N.ptr(b_interleaved), _ld(b_interleaved), N.ptr(a2), _ld(a2) if a2 is not None else 0,
+           N.ptr(b2_interleaved), _ld(b2_interleaved) if b2_interleaved is not None else 0, K2, N.ptr(out), _ld(out),
+           N.ptr(gu), _ld(gu) if gu is not None else 0, *((int(plain_rows),) if any_rows else ()), N.stream())
     if rec is not None:
         ev1.record()
         rec.records.append((ev0, ev1, 2.0 * M * rows * (K + K2), (M, rows, K, K2)))
@@ -439,8 +443,10 @@ def gemm_nt_swiglu_bwd(a: torch.Tensor, b: torch.Tensor, a2: torch.Tensor | None
 
 
 def swiglu_fused_ok(M: int, F: int, K: int, any_rows: bool = False) -> bool:
-    """Shapes the fused gate/up + SwiGLU product accepts."""
-    return (any_rows or M % 256 == 0) and (2 * F) % 256 == 0 and K % 64 == 0 and K > 0
+    """Shapes the fused gate/up + SwiGLU product accepts (F K: a tile's gate and up rows lie within the
+    32-bit byte offsets of one buffer)."""
+    return ((any_rows or M % 256 == 0) and (2 * F) % 256 == 0 and K % 64 == 0 and K > 0
+            and (F + 128) * K * 2 <= 0xFFFFFFFF)
 
 
 def interleave_gate_up(w_gu: torch.Tensor, F: int) -> torch.Tensor:

@@ -40,7 +40,6 @@ class LayerWeights:
     ln_post: torch.Tensor
     q_norm: torch.Tensor | None
     k_norm: torch.Tensor | None
-    w_gu_i: torch.Tensor | None = None   # [2F, H], gate/up rows interleaved in blocks of 64
 
 
 @dataclass
@@ -112,8 +111,8 @@ def clean_layer(h: torch.Tensor, lw: LayerWeights, g: Geometry, sc: StreamContex
     o, _ = K.attn_fwd(q, k, v, sc.iv_clean, g.nq, g.nk, g.d)
     h1 = K.gemm_nt(o, lw.w_o, residual=h)
     x2, _ = K.rmsnorm_fwd(h1, lw.ln_post, g.eps)
-    if lw.w_gu_i is not None and x2.dtype == torch.bfloat16 and K.swiglu_fused_ok(M, g.F, g.H, any_rows=True):
-        s = K.gemm_nt_swiglu(x2, lw.w_gu_i, any_rows=True)      # gate/up product with SwiGLU in its epilogue
+    if x2.dtype == torch.bfloat16 and K.swiglu_fused_ok(M, g.F, g.H, any_rows=True):
+        s = K.gemm_nt_swiglu(x2, lw.w_gu, any_rows=True, plain_rows=True)   # SwiGLU in the product's epilogue
     else:
         s = K.swiglu_fwd(K.gemm_nt(x2, lw.w_gu), g.F)
     h2 = K.gemm_nt(s, lw.w_d, residual=h1)
@@ -145,13 +144,12 @@ def noisy_layer_forward(h0, lw: LayerWeights, lora, li: int, g: Geometry, sc: St
     h1 = K.gemm_nt(o, lw.w_o, a2=h_o, b2=lora.sb_c(li, "o") if on("o") else None, residual=h0)
     x2, rstd2 = K.rmsnorm_fwd(h1, lw.ln_post, g.eps)
     h_gu = K.gemm_nt(x2, lora.a_c(li, "gu")) if on("gu") else None
-    fused = (lw.w_gu_i is not None and x2.dtype == torch.bfloat16
-             and K.swiglu_fused_ok(x2.shape[0], g.F, x2.shape[1], any_rows=True))
+    fused = x2.dtype == torch.bfloat16 and K.swiglu_fused_ok(x2.shape[0], g.F, x2.shape[1], any_rows=True)
     sb_gu_i = lora.sb_gu_i(li) if fused and on("gu") else None
     if fused and (not on("gu") or (sb_gu_i is not None and (2 * r) % 32 == 0)):
         # gate/up product with its LoRA terms, SwiGLU in the epilogue; [gate | up] kept for backward
         gu = torch.empty((x2.shape[0], 2 * g.F), device=x2.device, dtype=x2.dtype)
-        s = K.gemm_nt_swiglu(x2, lw.w_gu_i, a2=h_gu, b2_interleaved=sb_gu_i, gu=gu, any_rows=True)
+        s = K.gemm_nt_swiglu(x2, lw.w_gu, a2=h_gu, b2_interleaved=sb_gu_i, gu=gu, any_rows=True, plain_rows=True)
     else:
         gu = K.gemm_nt(x2, lw.w_gu, a2=h_gu, b2=lora.sb_c(li, "gu") if on("gu") else None,
                        segments=[(g.F, 0), (2 * g.F, r)] if on("gu") else None)
