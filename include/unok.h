@@ -176,12 +176,13 @@ int unok_gemm_nt_qkv_rope(int M, int K, int nq, int nk, const void* A, int64_t l
                           int nseg, const int* seg_end, const int* seg_col, const void* wq, const void* wk,
                           const int64_t* pos, const float* cos_tab, const float* sin_tab, int P, float eps,
                           void* q_out, void* k_out, void* v_out, float* rstd, void* qk_pre, void* stream);
-/* The same for any number of rows. */
+/* The same for any number of rows; pre_f32 != 0: qk_pre in fp32. */
 int unok_gemm_nt_qkv_rope_any(int M, int K, int nq, int nk, const void* A, int64_t lda, const void* B,
                           int64_t ldb, const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
                           int nseg, const int* seg_end, const int* seg_col, const void* wq, const void* wk,
                           const int64_t* pos, const float* cos_tab, const float* sin_tab, int P, float eps,
-                          void* q_out, void* k_out, void* v_out, float* rstd, void* qk_pre, void* stream);
+                          void* q_out, void* k_out, void* v_out, float* rstd, void* qk_pre, int pre_f32,
+                          void* stream);
 
 /* out = silu(gate) * up over the fused [gate | up] projection, rounded once (modeling_qwen3.py:81-82). */
 int unok_swiglu_fwd(int dtype, int M, int F, const void* gu, int64_t ld, void* out, void* stream);
@@ -226,6 +227,14 @@ int unok_attn_bwd(int dtype, int grad_dtype, int Mq, int Mk2, int Hq, int Hkv, i
  * rstd [Mq, Hq + Hkv] their 1/rms, cos_tab / sin_tab [P, D/2] the angles (unok_rope_table) at
  * each row's position; wq / wk null: RoPE only. Dsum [Mq, Hq] fp32 is caller scratch. */
 int unok_attn_bwd_qknorm(int Mq, int Hq, int Hkv, int D, const void* Q, int64_t ldq, const void* K1,
+                         int64_t ldk1, const void* V1, int64_t ldv1, const void* K2, int64_t ldk2,
+                         const void* V2, int64_t ldv2, const int32_t* iv, const void* O, int64_t ldo,
+                         const float* LSE, const void* dO, int64_t lddo, float* Dsum, const void* pre,
+                         int64_t ldpre, const float* rstd, const void* wq, const void* wk,
+                         const int64_t* pos, const float* cos_tab, const float* sin_tab, int P,
+                         void* dqkv, int64_t lddqkv, float scale, void* stream);
+/* The same with pre in fp32. */
+int unok_attn_bwd_qknorm_f32(int Mq, int Hq, int Hkv, int D, const void* Q, int64_t ldq, const void* K1,
                          int64_t ldk1, const void* V1, int64_t ldv1, const void* K2, int64_t ldk2,
                          const void* V2, int64_t ldv2, const int32_t* iv, const void* O, int64_t ldo,
                          const float* LSE, const void* dO, int64_t lddo, float* Dsum, const void* pre,

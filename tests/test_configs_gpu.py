@@ -263,3 +263,18 @@ def test_packing_collator_rows_fp32_step(dev):
     worst = max(((mine[k].cpu() - v.grad).norm() / v.grad.norm().clamp_min(1e-30)).item() for k, v in leaves.items())
     print(f"   loss rel {lrel:.2e}; worst grad rel L2 {worst:.2e}", flush=True)
     assert lrel < 1e-5 and worst < 2e-4
+
+
+# --- row counts that are no multiple of a tile ----------------------------------------------------
+
+RAGGED = dict(RANK32, intermediate_size=1536, B=3, L=263, prompt=31)
+RAGGED_PACKED = dict(RAGGED, B=1, L=1021)
+RAGGED_SEGMENTS = [401, 97, 330, 193]
+
+
+@pytest.mark.parametrize("spec,segments", [(RAGGED, None), (RAGGED_PACKED, RAGGED_SEGMENTS)])
+def test_ragged_rows_bf16_step(dev, spec, segments):
+    """789 and 1021 rows: every fused product of the layer on a row count between tiles, with its
+    backward."""
+    print(f"[configs] ragged rows {spec['B']}x{spec['L']}, bf16", flush=True)
+    _bf16_one_step(dev, spec, CE, 8, segments=segments)

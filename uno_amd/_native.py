@@ -95,9 +95,10 @@ SIGNATURES: dict[str, tuple] = {
     "unok_transpose_jobs": (_i, [_i, _p, _i, _i64, _p, _p, _p]),
 }
 
-for _name in ("unok_gemm_nt_swiglu_bwd", "unok_gemm_nt_qkv_rope"):
-    SIGNATURES[_name + "_any"] = SIGNATURES[_name]
-SIGNATURES["unok_gemm_nt_swiglu_any"] = (_i, [*SIGNATURES["unok_gemm_nt_swiglu"][1][:-1], _i, _p])
+SIGNATURES["unok_gemm_nt_swiglu_bwd_any"] = SIGNATURES["unok_gemm_nt_swiglu_bwd"]
+SIGNATURES["unok_attn_bwd_qknorm_f32"] = SIGNATURES["unok_attn_bwd_qknorm"]
+for _name in ("unok_gemm_nt_swiglu", "unok_gemm_nt_qkv_rope"):          # an option before the stream
+    SIGNATURES[_name + "_any"] = (_i, [*SIGNATURES[_name][1][:-1], _i, _p])
 
 _lock = threading.Lock()
 _lib = None

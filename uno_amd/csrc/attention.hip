@@ -43,11 +43,11 @@ struct AttnArgs {
   // bf16 kernels with qkn_out set: instead of dQ / dK, the gradient of the q/k projection before
   // the q/k RMSNorm and RoPE (their backward applied to the fp32 dQ / dK accumulators), written into
   // the q / k column blocks of qkn_out [Mq, (Hq + 2 Hkv) D]; the q/k head columns of qkn_pre
-  // [Mq, (Hq + Hkv) D] are the pre-norm values (bf16), qkn_rstd [Mq, Hq + Hkv] their 1/rms, and
+  // [Mq, (Hq + Hkv) D] are the pre-norm values (bf16, or fp32 with qkn_pre_f32), qkn_rstd [Mq, Hq + Hkv] their 1/rms, and
   // qkn_cos / qkn_sin [qkn_P, D/2] the angles at each row's position qkn_pos. No norm when qkn_wq is
   // null (RoPE only).
   bf16_t* qkn_out; int64_t ld_qkn_out;
-  const bf16_t* qkn_pre; int64_t ld_qkn_pre;
+  const void* qkn_pre; int64_t ld_qkn_pre; int qkn_pre_f32;
   const float* qkn_rstd;
   const bf16_t* qkn_wq; const bf16_t* qkn_wk;
   const int64_t* qkn_pos;
@@ -65,12 +65,15 @@ __device__ __forceinline__ bf16x8_t ld_bf16x8(const bf16_t* p) { return *(const 
 // scale), so a dim's RoPE partner c +- D/2 is block t ^ (NDT/2) of the same lane and the other half
 // of the row sits in lane ^ 32. Writes r (g - xhat mean(g xhat)) with g = w * RoPE^-1(dy) (or
 // RoPE^-1(dy) without the norm) as bf16 at dst[c]; pre / rs: the row's pre-norm head and 1/rms;
-// cs / sn: the row's angle-table rows. Lanes with valid false take part in the shuffle only.
-template <int D>
+// cs / sn: the row's angle-table rows. Lanes with valid false take part in the shuffle only. An fp32
+// head (PreT float) is loaded where it is used: held from the start, its 64 registers would not fit
+// beside the rest (dQ, dK and dV of 7680 rows, 16/8 heads of 128: 168 us with bf16 heads, 175 with fp32).
+template <int D, typename PreT>
 __device__ __forceinline__ void qknorm_rope_bwd_acc(const f32x16_t (&acc)[D / 32], float scale, int g, bool valid,
-                                                    const bf16_t* pre, float rs, const bf16_t* wn, const float* cs,
+                                                    const PreT* pre, float rs, const bf16_t* wn, const float* cs,
                                                     const float* sn, bf16_t* dst) {
   constexpr int NDT = D / 32, HT = NDT / 2;
+  constexpr bool F32 = std::is_same<PreT, float>::value;
   // every input load first (independent of each other), then the arithmetic
   float4 cv[HT][4], sv[HT][4];
   uint2 xw[NDT][4], ww[NDT][4];
@@ -88,7 +91,7 @@ __device__ __forceinline__ void qknorm_rope_bwd_acc(const f32x16_t (&acc)[D / 32
 #pragma unroll
       for (int j4 = 0; j4 < 4; ++j4) {
         const int c = 32 * t + 8 * j4 + 4 * g;
-        xw[t][j4] = valid ? *(const uint2*)(pre + c) : make_uint2(0, 0);
+        if (!F32) xw[t][j4] = valid ? *(const uint2*)(pre + c) : make_uint2(0, 0);
         ww[t][j4] = valid ? *(const uint2*)(wn + c) : make_uint2(0, 0);
       }
   }
@@ -114,9 +117,15 @@ __device__ __forceinline__ void qknorm_rope_bwd_acc(const f32x16_t (&acc)[D / 32
     for (int t = 0; t < NDT; ++t)
 #pragma unroll
       for (int j4 = 0; j4 < 4; ++j4) {
-        const uint2 xv = xw[t][j4], wv = ww[t][j4];
-        const float x4[4] = {__uint_as_float(xv.x << 16), __uint_as_float(xv.x & 0xffff0000u),
-                             __uint_as_float(xv.y << 16), __uint_as_float(xv.y & 0xffff0000u)};
+        const uint2 wv = ww[t][j4];
+        f32x4_t x4 = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (F32) {
+          if (valid) x4 = *(const f32x4_t*)(pre + 32 * t + 8 * j4 + 4 * g);
+        } else {
+          const uint2 xv = xw[t][j4];
+          x4 = f32x4_t{__uint_as_float(xv.x << 16), __uint_as_float(xv.x & 0xffff0000u),
+                       __uint_as_float(xv.y << 16), __uint_as_float(xv.y & 0xffff0000u)};
+        }
         const float w4[4] = {__uint_as_float(wv.x << 16), __uint_as_float(wv.x & 0xffff0000u),
                              __uint_as_float(wv.y << 16), __uint_as_float(wv.y & 0xffff0000u)};
 #pragma unroll
@@ -693,8 +702,14 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_dq_bf16_kernel(const Att
   }
   if (p.qkn_out != nullptr) {       // wave-uniform: the q/k-norm + RoPE backward on the accumulators
     const int row = qvalid ? qrow : 0;
-    qknorm_rope_bwd_acc<D>(dq, p.scale, g, qvalid, p.qkn_pre + (int64_t)row * p.ld_qkn_pre + h * D, qkn_rs, p.qkn_wq,
-                           p.qkn_cos + qkn_ar, p.qkn_sin + qkn_ar, p.qkn_out + (int64_t)row * p.ld_qkn_out + h * D);
+    const int64_t at = (int64_t)row * p.ld_qkn_pre + h * D;
+    bf16_t* dst = p.qkn_out + (int64_t)row * p.ld_qkn_out + h * D;
+    if (p.qkn_pre_f32)
+      qknorm_rope_bwd_acc<D>(dq, p.scale, g, qvalid, (const float*)p.qkn_pre + at, qkn_rs, p.qkn_wq, p.qkn_cos + qkn_ar,
+                             p.qkn_sin + qkn_ar, dst);
+    else
+      qknorm_rope_bwd_acc<D>(dq, p.scale, g, qvalid, (const bf16_t*)p.qkn_pre + at, qkn_rs, p.qkn_wq, p.qkn_cos + qkn_ar,
+                             p.qkn_sin + qkn_ar, dst);
   } else if (qvalid && p.grad_f32) {
     float* out = (float*)p.dQ + (int64_t)qrow * p.lddq + h * D;
 #pragma unroll
@@ -879,8 +894,14 @@ __global__ __launch_bounds__(256, 1) void attn_dkv_bf16_kernel(const AttnArgs p)
   }
   if (p.qkn_out != nullptr) {       // wave-uniform: the k-norm + RoPE backward on the dK accumulators
     const int row = kvalid ? krow : 0, col = (p.Hq + kvh) * D;
-    qknorm_rope_bwd_acc<D>(dk, p.scale, g, kvalid, p.qkn_pre + (int64_t)row * p.ld_qkn_pre + col, qkn_rs, p.qkn_wk,
-                           p.qkn_cos + qkn_ar, p.qkn_sin + qkn_ar, p.qkn_out + (int64_t)row * p.ld_qkn_out + col);
+    const int64_t at = (int64_t)row * p.ld_qkn_pre + col;
+    bf16_t* dst = p.qkn_out + (int64_t)row * p.ld_qkn_out + col;
+    if (p.qkn_pre_f32)
+      qknorm_rope_bwd_acc<D>(dk, p.scale, g, kvalid, (const float*)p.qkn_pre + at, qkn_rs, p.qkn_wk, p.qkn_cos + qkn_ar,
+                             p.qkn_sin + qkn_ar, dst);
+    else
+      qknorm_rope_bwd_acc<D>(dk, p.scale, g, kvalid, (const bf16_t*)p.qkn_pre + at, qkn_rs, p.qkn_wk, p.qkn_cos + qkn_ar,
+                             p.qkn_sin + qkn_ar, dst);
   }
   if (kvalid) {
     bf16_t* ov = (bf16_t*)p.dV + (int64_t)krow * p.lddv + kvh * D;
@@ -1275,15 +1296,15 @@ UNOK_EXPORT int unok_attn_bwd(int dtype, int grad_dtype, int Mq, int Mk2, int Hq
 // epilogues (bf16): instead of dQ and dK, the gradient before the norm is written into the q and k
 // column blocks of dqkv [Mq, (Hq + 2 Hkv) D] (row stride lddqkv), dV into its v block. Source-2
 // keys are the query rows themselves (Mk2 = Mq). pre [Mq, (Hq + Hkv) D] holds the pre-norm q/k
-// columns (bf16, row stride ldpre), rstd [Mq, Hq + Hkv] their 1/rms (read only with wq / wk),
-// cos_tab / sin_tab [P, D/2] the angles at each row's position pos.
-UNOK_EXPORT int unok_attn_bwd_qknorm(int Mq, int Hq, int Hkv, int D, const void* Q, int64_t ldq, const void* K1,
+// columns (bf16, or fp32 with pre_f32; row stride ldpre), rstd [Mq, Hq + Hkv] their 1/rms (read only with
+// wq / wk), cos_tab / sin_tab [P, D/2] the angles at each row's position pos.
+static int attn_bwd_qknorm_any(int Mq, int Hq, int Hkv, int D, const void* Q, int64_t ldq, const void* K1,
                                      int64_t ldk1, const void* V1, int64_t ldv1, const void* K2, int64_t ldk2,
                                      const void* V2, int64_t ldv2, const int32_t* iv, const void* O, int64_t ldo,
                                      const float* LSE, const void* dO, int64_t lddo, float* Dsum, const void* pre,
                                      int64_t ldpre, const float* rstd, const void* wq, const void* wk,
                                      const int64_t* pos, const float* cos_tab, const float* sin_tab, int P,
-                                     void* dqkv, int64_t lddqkv, float scale, void* stream) {
+                                     void* dqkv, int64_t lddqkv, float scale, void* stream, bool pre_f32) {
   if (Mq == 0) return 0;
   int rc = check_geom(UNOK_BF16, D, Hq, Hkv);
   if (rc) return rc;
@@ -1300,7 +1321,7 @@ UNOK_EXPORT int unok_attn_bwd_qknorm(int Mq, int Hq, int Hkv, int D, const void*
   a.dV = (bf16_t*)dqkv + (int64_t)(Hq + Hkv) * D; a.lddv = lddqkv;
   a.Mq = Mq; a.Mk2 = Mq; a.Hq = Hq; a.Hkv = Hkv; a.scale = scale; a.scale_log2 = scale * 1.4426950408889634f;
   a.qkn_out = (bf16_t*)dqkv; a.ld_qkn_out = lddqkv;
-  a.qkn_pre = (const bf16_t*)pre; a.ld_qkn_pre = ldpre; a.qkn_rstd = rstd;
+  a.qkn_pre = pre; a.ld_qkn_pre = ldpre; a.qkn_pre_f32 = pre_f32; a.qkn_rstd = rstd;
   a.qkn_wq = (const bf16_t*)wq; a.qkn_wk = (const bf16_t*)wk; a.qkn_pos = pos;
   a.qkn_cos = cos_tab; a.qkn_sin = sin_tab; a.qkn_P = P;
   hipStream_t st = (hipStream_t)stream;
@@ -1312,4 +1333,27 @@ UNOK_EXPORT int unok_attn_bwd_qknorm(int Mq, int Hq, int Hkv, int D, const void*
   if (D == 128) launch_dkv<128>(kblocks, st, a);
   else launch_dkv<64>(kblocks, st, a);
   return unok::check_launch("attn_dkv_bf16");
+}
+
+UNOK_EXPORT int unok_attn_bwd_qknorm(int Mq, int Hq, int Hkv, int D, const void* Q, int64_t ldq, const void* K1,
+                                     int64_t ldk1, const void* V1, int64_t ldv1, const void* K2, int64_t ldk2,
+                                     const void* V2, int64_t ldv2, const int32_t* iv, const void* O, int64_t ldo,
+                                     const float* LSE, const void* dO, int64_t lddo, float* Dsum, const void* pre,
+                                     int64_t ldpre, const float* rstd, const void* wq, const void* wk,
+                                     const int64_t* pos, const float* cos_tab, const float* sin_tab, int P,
+                                     void* dqkv, int64_t lddqkv, float scale, void* stream) {
+  return attn_bwd_qknorm_any(Mq, Hq, Hkv, D, Q, ldq, K1, ldk1, V1, ldv1, K2, ldk2, V2, ldv2, iv, O, ldo, LSE, dO, lddo, Dsum,
+                             pre, ldpre, rstd, wq, wk, pos, cos_tab, sin_tab, P, dqkv, lddqkv, scale, stream, false);
+}
+
+// unok_attn_bwd_qknorm with fp32 pre-norm columns.
+UNOK_EXPORT int unok_attn_bwd_qknorm_f32(int Mq, int Hq, int Hkv, int D, const void* Q, int64_t ldq, const void* K1,
+                                     int64_t ldk1, const void* V1, int64_t ldv1, const void* K2, int64_t ldk2,
+                                     const void* V2, int64_t ldv2, const int32_t* iv, const void* O, int64_t ldo,
+                                     const float* LSE, const void* dO, int64_t lddo, float* Dsum, const void* pre,
+                                     int64_t ldpre, const float* rstd, const void* wq, const void* wk,
+                                     const int64_t* pos, const float* cos_tab, const float* sin_tab, int P,
+                                     void* dqkv, int64_t lddqkv, float scale, void* stream) {
+  return attn_bwd_qknorm_any(Mq, Hq, Hkv, D, Q, ldq, K1, ldk1, V1, ldv1, K2, ldk2, V2, ldv2, iv, O, ldo, LSE, dO, lddo, Dsum,
+                             pre, ldpre, rstd, wq, wk, pos, cos_tab, sin_tab, P, dqkv, lddqkv, scale, stream, true);
 }

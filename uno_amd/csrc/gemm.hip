@@ -54,7 +54,7 @@ struct GemmNT {
   // heads, then nk v heads. q/k heads are normalised (when qk_wq is set), scaled by the weight and
   // rotated in fp32, then rounded once into qk_q / qk_k; v heads are rounded into qk_v.
   void* qk_q; void* qk_k; void* qk_v;
-  void* qk_pre;                    // [M, 128 (nq+nk)] bf16 q/k before the norm, or null
+  void* qk_pre; int qk_pre_f32;    // [M, 128 (nq+nk)] q/k before the norm (bf16, or fp32 with qk_pre_f32), or null
   float* qk_rstd;                  // [M, nq+nk] 1/rms per row and q/k head, or null
   const void* qk_wq; const void* qk_wk;
   const int64_t* qk_pos;           // [M] position of each row
@@ -1408,7 +1408,8 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
     if (isq) { dst = (bf16_t*)p.qk_q + (int64_t)head * 128 + c0; ldd = (int64_t)nq * 128; }
     else if (!isv) { dst = (bf16_t*)p.qk_k + (int64_t)(head - nq) * 128 + c0; ldd = (int64_t)p.qk_nk * 128; }
     else { dst = (bf16_t*)p.qk_v + (int64_t)(head - nqk) * 128 + c0; ldd = (int64_t)p.qk_nk * 128; }
-    bf16_t* pre = p.qk_pre && !isv ? (bf16_t*)p.qk_pre + (int64_t)head * 128 + c0 : nullptr;
+    const bool pre = p.qk_pre && !isv;
+    const int64_t pre0 = (int64_t)head * 128 + c0;
     const int64_t ldp = (int64_t)nqk * 128;
     const bool norm = !isv && p.qk_wq != nullptr;
     float wv[16];
@@ -1461,10 +1462,15 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
 #pragma unroll
           for (int e = 0; e < 16; ++e) out[e] = x[e];
         } else {
-          if (pre) {
+          if (pre && p.qk_pre_f32) {
+            float* dp = (float*)p.qk_pre + row * ldp + pre0;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+              *(f32x4_t*)(dp + (c < 2 ? 0 : 56) + 4 * c) = f32x4_t{x[4 * c], x[4 * c + 1], x[4 * c + 2], x[4 * c + 3]};
+          } else if (pre) {
 #pragma unroll
             for (int hh = 0; hh < 2; ++hh)
-              *(uint4*)(pre + row * ldp + 64 * hh) =
+              *(uint4*)((bf16_t*)p.qk_pre + row * ldp + pre0 + 64 * hh) =
                   make_uint4(pack2_bf16(x[8 * hh], x[8 * hh + 1]), pack2_bf16(x[8 * hh + 2], x[8 * hh + 3]),
                              pack2_bf16(x[8 * hh + 4], x[8 * hh + 5]), pack2_bf16(x[8 * hh + 6], x[8 * hh + 7]));
           }
@@ -1839,7 +1845,7 @@ UNOK_EXPORT int unok_gemm_nt_swiglu_any(int M, int N, int K, const void* A, int6
 // A[M,K] B[N,K]^T (+ the LoRA extension, up to 4 segments as in unok_gemm_nt), N = 128 (nq + 2 nk),
 // stays in fp32 until each q/k head is normalised (wq / wk, or neither), scaled by the weight and
 // rotated; q [M, 128 nq], k and v [M, 128 nk] are written contiguous in bf16, rstd [M, nq+nk] (when
-// non-null), and the q/k columns before the norm in bf16 into qk_pre [M, 128 (nq+nk)] (when
+// non-null), and the q/k columns before the norm in bf16 (pre_f32: fp32) into qk_pre [M, 128 (nq+nk)] (when
 // non-null). cos_tab / sin_tab [P, 64] hold cos / sin of fl32(p * inv_freq[j]) (unok_rope_table);
 // positions are clamped to [0, P). Same values as unok_gemm_nt into fp32 followed by
 // unok_qknorm_rope_fwd. M and N multiples of 256, K of 64, K2 of 32.
@@ -1848,7 +1854,7 @@ static int qkv_rope_product(int M, int K, int nq, int nk, const void* A, int64_t
                                       int nseg, const int* seg_end, const int* seg_col, const void* wq, const void* wk,
                                       const int64_t* pos, const float* cos_tab, const float* sin_tab, int P, float eps,
                                       void* q_out, void* k_out, void* v_out, float* rstd, void* qk_pre, void* stream,
-                                      int row_step) {
+                                      int row_step, bool pre_f32) {
   UNOK_REQUIRE(M >= 0 && K >= 0 && K2 >= 0 && nq > 0 && nk > 0 && P > 0, UNOK_EINVAL,
                "gemm_nt_qkv_rope: bad sizes M=%d K=%d nq=%d nk=%d P=%d", M, K, nq, nk, P);
   if (M == 0) return 0;
@@ -1878,6 +1884,7 @@ static int qkv_rope_product(int M, int K, int nq, int nk, const void* A, int64_t
     UNOK_REQUIRE(p.seg_end[nseg - 1] == N, UNOK_EINVAL, "gemm_nt_qkv_rope: last segment must end at N");
   }
   p.qk_q = q_out; p.qk_k = k_out; p.qk_v = v_out; p.qk_pre = qk_pre; p.qk_rstd = rstd;
+  p.qk_pre_f32 = pre_f32;
   p.qk_wq = wq; p.qk_wk = wk; p.qk_pos = pos; p.qk_cos = cos_tab; p.qk_sin = sin_tab; p.qk_P = P;
   p.qk_nq = nq; p.qk_nk = nk; p.qk_eps = eps;
   UNOK_REQUIRE(buffer_ranges_ok(p), UNOK_EINVAL, "gemm_nt_qkv_rope: operands exceed 32-bit buffer offsets");
@@ -1891,17 +1898,18 @@ UNOK_EXPORT int unok_gemm_nt_qkv_rope(int M, int K, int nq, int nk, const void* 
                                       const int64_t* pos, const float* cos_tab, const float* sin_tab, int P, float eps,
                                       void* q_out, void* k_out, void* v_out, float* rstd, void* qk_pre, void* stream) {
   return qkv_rope_product(M, K, nq, nk, A, lda, B, ldb, A2, lda2, B2, ldb2, K2, nseg, seg_end, seg_col, wq, wk, pos, cos_tab, sin_tab, P,
-                          eps, q_out, k_out, v_out, rstd, qk_pre, stream, 256);
+                          eps, q_out, k_out, v_out, rstd, qk_pre, stream, 256, false);
 }
 
-// unok_gemm_nt_qkv_rope for any number of rows.
+// unok_gemm_nt_qkv_rope for any number of rows; pre_f32 != 0: qk_pre in fp32.
 UNOK_EXPORT int unok_gemm_nt_qkv_rope_any(int M, int K, int nq, int nk, const void* A, int64_t lda, const void* B,
                                       int64_t ldb, const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
                                       int nseg, const int* seg_end, const int* seg_col, const void* wq, const void* wk,
                                       const int64_t* pos, const float* cos_tab, const float* sin_tab, int P, float eps,
-                                      void* q_out, void* k_out, void* v_out, float* rstd, void* qk_pre, void* stream) {
+                                      void* q_out, void* k_out, void* v_out, float* rstd, void* qk_pre, int pre_f32,
+                                      void* stream) {
   return qkv_rope_product(M, K, nq, nk, A, lda, B, ldb, A2, lda2, B2, ldb2, K2, nseg, seg_end, seg_col, wq, wk, pos, cos_tab, sin_tab, P,
-                          eps, q_out, k_out, v_out, rstd, qk_pre, stream, 1);
+                          eps, q_out, k_out, v_out, rstd, qk_pre, stream, 1, pre_f32 != 0);
 }
 
 // dgu[M, 2F] = SwiGLU backward of dS = A[M,K] B[F,K]^T + A2[M,K2] B2[F,K2]^T (bf16, never stored)

@@ -314,10 +314,11 @@ def qkv_rope_fused_ok(M: int, K: int, K2: int, nq: int, nk: int, d: int, dtype, 
 
 
 def gemm_nt_qkv_rope(x, w_qkv, nq, nk, wq, wk, pos, cos_tab, sin_tab, eps, *, a2=None, b2=None, segments=None,
-                     want_rstd=True, want_pre=False, any_rows=False):
+                     want_rstd=True, want_pre=False, any_rows=False, pre_dtype=torch.bfloat16):
     """q|k|v projection (+ LoRA extension) with q/k RMSNorm + RoPE in the GEMM epilogue (bf16, head dim
-    128). Returns (q, k, v, rstd or None, pre or None); ``pre`` = the pre-norm q/k columns in bf16.
-    ``any_rows`` takes any number of rows; otherwise M must be a multiple of 256."""
+    128). Returns (q, k, v, rstd or None, pre or None); ``pre`` = the pre-norm q/k columns in ``pre_dtype``
+    (bf16; with ``any_rows`` also fp32). ``any_rows`` takes any number of rows; otherwise M must be a multiple
+    of 256."""
     _rowmajor(x, "x")
     _rowmajor(w_qkv, "w_qkv")
     M, Kd = x.shape
@@ -339,12 +340,14 @@ def gemm_nt_qkv_rope(x, w_qkv, nq, nk, wq, wk, pos, cos_tab, sin_tab, eps, *, a2
         raise RuntimeError("gemm_nt_qkv_rope: shape outside the fused kernel")
     if pos.dtype != torch.int64 or pos.numel() != M:
         raise RuntimeError("gemm_nt_qkv_rope: pos must be int64 [M]")
+    if pre_dtype != torch.bfloat16 and not (any_rows and pre_dtype == torch.float32):
+        raise RuntimeError("gemm_nt_qkv_rope: pre is bf16, or fp32 with any_rows")
     e = dict(device=x.device, dtype=x.dtype)
     q = torch.empty((M, 128 * nq), **e)
     k = torch.empty((M, 128 * nk), **e)
     v = torch.empty((M, 128 * nk), **e)
     rstd = torch.empty((M, nq + nk), device=x.device, dtype=torch.float32) if want_rstd else None
-    pre = torch.empty((M, 128 * (nq + nk)), **e) if want_pre else None
+    pre = torch.empty((M, 128 * (nq + nk)), device=x.device, dtype=pre_dtype) if want_pre else None
     Nn = w_qkv.shape[0]
     rec = _recorder
     if rec is not None and rec.predicate(x.dtype, M, Nn, Kd, K2, seg_end or [Nn]):
@@ -352,10 +355,11 @@ def gemm_nt_qkv_rope(x, w_qkv, nq, nk, wq, wk, pos, cos_tab, sin_tab, eps, *, a2
         ev0.record()
     else:
         rec = None
-    N.call("unok_gemm_nt_qkv_rope_any" if any_rows else "unok_gemm_nt_qkv_rope", M, Kd, nq, nk, N.ptr(x), _ld(x), N.ptr(w_qkv), _ld(w_qkv), N.ptr(a2),
-           _ld(a2) if a2 is not None else 0, N.ptr(b2), _ld(b2) if b2 is not None else 0, K2, len(seg_end),
-           N.int_array(seg_end), N.int_array(seg_col), N.ptr(wq), N.ptr(wk), N.ptr(pos), N.ptr(cos_tab),
-           N.ptr(sin_tab), cos_tab.shape[0], float(eps), N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(rstd), N.ptr(pre),
+    N.call("unok_gemm_nt_qkv_rope_any" if any_rows else "unok_gemm_nt_qkv_rope", M, Kd, nq, nk, N.ptr(x), _ld(x),
+           N.ptr(w_qkv), _ld(w_qkv), N.ptr(a2), _ld(a2) if a2 is not None else 0, N.ptr(b2),
+           _ld(b2) if b2 is not None else 0, K2, len(seg_end), N.int_array(seg_end), N.int_array(seg_col),
+           N.ptr(wq), N.ptr(wk), N.ptr(pos), N.ptr(cos_tab), N.ptr(sin_tab), cos_tab.shape[0], float(eps), N.ptr(q),
+           N.ptr(k), N.ptr(v), N.ptr(rstd), N.ptr(pre), *((int(pre_dtype == torch.float32),) if any_rows else ()),
            N.stream())
     if rec is not None:
         ev1.record()
@@ -576,14 +580,15 @@ def attn_bwd_qknorm(q, k1, v1, iv, o, lse, do, Hq, Hkv, D, k2, v2, pre, rstd, wq
     _contig(do, "do")
     _rowmajor(pre, "pre")
     _rowmajor(dqkv, "dqkv")
-    if q.dtype != torch.bfloat16 or pre.dtype != torch.bfloat16 or dqkv.dtype != torch.bfloat16:
-        raise RuntimeError("attn_bwd_qknorm: bf16 only")
+    if q.dtype != torch.bfloat16 or pre.dtype not in (torch.bfloat16, torch.float32) or dqkv.dtype != torch.bfloat16:
+        raise RuntimeError("attn_bwd_qknorm: bf16 only (pre: bf16 or fp32)")
     if pre.shape != (Mq, (Hq + Hkv) * D) or dqkv.shape != (Mq, (Hq + 2 * Hkv) * D) or k2.shape[0] != Mq:
         raise RuntimeError("attn_bwd_qknorm: pre [Mq, (Hq+Hkv) D], dqkv [Mq, (Hq+2Hkv) D] and Mq keys required")
     if pos.dtype != torch.int64 or pos.numel() != Mq:
         raise RuntimeError("attn_bwd_qknorm: pos must be int64 [Mq]")
     dsum = torch.empty((Mq, Hq), device=q.device, dtype=torch.float32)
-    N.call("unok_attn_bwd_qknorm", Mq, Hq, Hkv, D, N.ptr(q), _ld(q), N.ptr(k1), _ld(k1), N.ptr(v1), _ld(v1),
+    N.call("unok_attn_bwd_qknorm" if pre.dtype == torch.bfloat16 else "unok_attn_bwd_qknorm_f32", Mq, Hq, Hkv, D,
+           N.ptr(q), _ld(q), N.ptr(k1), _ld(k1), N.ptr(v1), _ld(v1),
            N.ptr(k2), _ld(k2), N.ptr(v2), _ld(v2), N.ptr(iv), N.ptr(o), _ld(o), N.ptr(lse), N.ptr(do), _ld(do),
            N.ptr(dsum), N.ptr(pre), _ld(pre), N.ptr(rstd), N.ptr(wq), N.ptr(wk), N.ptr(pos), N.ptr(cos_tab),
            N.ptr(sin_tab), cos_tab.shape[0], N.ptr(dqkv), _ld(dqkv), float(scale), N.stream())

@@ -80,18 +80,27 @@ def _qkv_dtype(x: torch.Tensor):
     return torch.float32 if x.dtype == torch.bfloat16 else x.dtype
 
 
+def qk_pre_dtype(rows: int):
+    """Element type of the pre-norm q/k columns that the fused q|k|v epilogue of a bf16 step keeps for the
+    backward: bf16 for row counts of whole 256-row tiles, fp32 otherwise, as the projection output kept
+    there by the separate norm kernel is (two 1B layers of 5 x 1531 rows, forward and backward: 5.59 ms with
+    bf16 columns, 5.62 with fp32)."""
+    return torch.float32 if rows % 256 else torch.bfloat16
+
+
 def project_qk_v(x1, lw: LayerWeights, g: Geometry, sc: StreamContext, a2=None, b2=None, segments=None,
                  for_backward: bool = False):
     """q/k/v projection (with its LoRA extension), q/k norm and RoPE: (x_qk, q, k, v, rstd), where x_qk
     holds the pre-norm q/k columns first (what the q/k norm backward reads): the fp32 projection
-    output, or, when the GEMM applies the norm and RoPE in its epilogue, their bf16 copy (only with
-    ``for_backward``; None otherwise)."""
+    output, or, when the GEMM applies the norm and RoPE in its epilogue, their copy in qk_pre_dtype (only
+    with ``for_backward``; None otherwise)."""
     K2 = b2.shape[1] if b2 is not None else 0
     if sc.rope_cos is not None and K.qkv_rope_fused_ok(x1.shape[0], x1.shape[1], K2, g.nq, g.nk, g.d, x1.dtype,
                                                        any_rows=True):
         q, k, v, rstd, pre = K.gemm_nt_qkv_rope(x1, lw.w_qkv, g.nq, g.nk, lw.q_norm, lw.k_norm, sc.pos, sc.rope_cos,
                                                 sc.rope_sin, g.eps, a2=a2, b2=b2, segments=segments,
-                                                want_rstd=for_backward, want_pre=for_backward, any_rows=True)
+                                                want_rstd=for_backward, want_pre=for_backward, any_rows=True,
+                                                pre_dtype=qk_pre_dtype(x1.shape[0]))
         return pre, q, k, v, rstd
     qkv = K.gemm_nt(x1, lw.w_qkv, a2=a2, b2=b2, segments=segments, out_dtype=_qkv_dtype(x1))
     if qkv.dtype == x1.dtype:
@@ -160,15 +169,15 @@ def noisy_layer_forward(h0, lw: LayerWeights, lora, li: int, g: Geometry, sc: St
     return h2, (h0, x1, rstd1, h_qkv, qkv, q, k, v, rstd_qk, o, lse, h_o, h1, x2, rstd2, h_gu, gu, s, h_d)
 
 
-def saved_bytes_per_row(g: Geometry, rank: int, elem: int, fused_qkv: bool = True) -> int:
+def saved_bytes_per_row(g: Geometry, rank: int, elem: int, fused_qkv: bool = True, pre_elem: int | None = None) -> int:
     """Bytes of activations one noisy-stream layer keeps per token row for its backward
-    (``fused_qkv``: the q|k|v epilogue keeps bf16 pre-norm q/k; otherwise a bf16 step keeps the fp32
-    projection output)."""
+    (``fused_qkv``: the q|k|v epilogue keeps the pre-norm q/k in ``pre_elem`` bytes, ``elem`` by default;
+    otherwise a bf16 step keeps the fp32 projection output)."""
     stored = 4 * g.H + g.q + g.kv + g.q + 3 * g.F + 7 * rank
     if elem == 2 and not fused_qkv:
         qkv = (g.q + 2 * g.kv) * 4 + g.kv * elem
     else:
-        qkv = (g.q + 2 * g.kv) * elem
+        qkv = (g.q + g.kv) * (pre_elem or elem) + g.kv * elem
     return stored * elem + qkv + 4 * (2 + g.nq + g.nk + g.nq)
 
 
@@ -256,8 +265,8 @@ class NoisyLayer(torch.autograd.Function):
         # dq and dk in the q/k/v projection's precision (fp32 for a bf16 step) up to the q/k norm
         # backward, which writes the bf16 q/k gradient blocks of dqkv; dv goes straight into dqkv
         dqkv = torch.empty((M, g.q + 2 * g.kv), device=dh2.device, dtype=dh2.dtype)
-        if qkv.dtype == torch.bfloat16 and qkv.shape[1] == k_end and sc.rope_cos is not None:
-            # the fused forward kept the bf16 pre-norm q/k: the attention backward applies the q/k
+        if dh2.dtype == torch.bfloat16 and qkv.shape[1] == k_end and sc.rope_cos is not None:
+            # the fused forward kept the pre-norm q/k: the attention backward applies the q/k
             # norm + RoPE backward to its fp32 dQ / dK accumulators and writes dqkv directly
             K.attn_bwd_qknorm(q, sc.clean_k[li], sc.clean_v[li], sc.iv_noisy, o, lse, do, g.nq, g.nk, g.d, k, v,
                               qkv, rstd_qk, lw.q_norm, lw.k_norm, sc.pos, sc.rope_cos, sc.rope_sin, dqkv)

@@ -362,7 +362,8 @@ class UnoQwen3Model(nn.Module):
             if self._auto_plan is not None and self._auto_plan[0] == key:
                 self.last_recompute_plan = list(self._auto_plan[1])
                 return self.last_recompute_plan
-            per_layer = Lyr.saved_bytes_per_row(self.geo, rank, elem) * rows
+            pre_elem = Lyr.qk_pre_dtype(rows).itemsize if elem == 2 else elem
+            per_layer = Lyr.saved_bytes_per_row(self.geo, rank, elem, pre_elem=pre_elem) * rows
             input_only = self.geo.H * elem * rows
             budget = self.recompute_budget_bytes
             if budget is None:
