@@ -174,3 +174,32 @@ def test_prefill_follows_in_place_weight_updates(dev, write):
         dec = BlockDecoder(lm)
         logits.append(dec.prefill(dec.new_cache(2, 256), ids))
     assert torch.equal(*logits)
+
+
+def test_draft_block_with_strided_weights(dev):
+    """Weights whose rows are not dense run through the products one by one: the same logits, bit for bit."""
+    s = SPECS["gqa4_r32"]
+    ucfg = UnoQwen3Config(vocab_size=s["vocab_size"], hidden_size=s["hidden_size"],
+                          intermediate_size=s["intermediate_size"], num_hidden_layers=2,
+                          num_attention_heads=s["num_attention_heads"], num_key_value_heads=s["num_key_value_heads"],
+                          head_dim=s["head_dim"], block_size=16)
+    model = UnoQwen3ForCausalLM(ucfg, device=dev, dtype=torch.bfloat16)
+    model.random_init(3)
+    lm, _ = create_lora_model(model, LoraSettings("all", s["rank"], s["alpha"], 0.0))
+    dec = BlockDecoder(lm)
+    g = torch.Generator().manual_seed(7)
+    prompt = torch.randint(0, s["vocab_size"], (2, 50), generator=g).to(dev)
+    blk = torch.randint(0, s["vocab_size"], (2, 16), generator=g).to(dev)
+    logits = []
+    for strided in (False, True):
+        if strided:
+            layer = model.model.layers[1]
+            for name in ("w_d", "w_qkv"):
+                w = getattr(layer, name)
+                wide = torch.zeros(w.shape[0], w.shape[1] + 64, device=dev, dtype=w.dtype)
+                wide[:, :w.shape[1]] = w
+                setattr(layer, name, wide[:, :w.shape[1]])
+        cache = dec.new_cache(2, 128)
+        dec.prefill(cache, prompt)
+        logits.append(dec.draft_block(cache, blk))
+    assert torch.equal(*logits)

@@ -835,6 +835,12 @@ UNOK_EXPORT int64_t unok_draft_layer_scratch(const unok_draft_layer_args* a) {
 UNOK_EXPORT int unok_draft_layer(const unok_draft_layer_args* a, void* stream) {
   int rc = draft_sizes_ok(a);
   if (rc || a->B == 0 || a->L == 0) return rc;
+  for (const void* q : {a->ln_in, a->ln_post, a->w_qkv, a->a_qkv, a->b_qkv, a->w_o, a->a_o, a->b_o, a->w_gu, a->a_gu, a->b_gu,
+                        a->w_d, a->a_d, a->b_d, (const void*)a->kc, (const void*)a->vc, (const void*)a->lengths,
+                        (const void*)a->inv_freq, (const void*)a->gate, (const void*)a->ivs, (const void*)a->dst, a->h,
+                        (const void*)a->h_out})
+    UNOK_REQUIRE(q != nullptr, UNOK_EINVAL, "draft_layer: null operand");
+  UNOK_REQUIRE(a->h != a->h_out, UNOK_EINVAL, "draft_layer: h and h_out may not overlap");
   const DraftBuffers b = draft_buffers(*a);
   UNOK_REQUIRE(a->scratch != nullptr && a->scratch_bytes >= b.bytes && ((uintptr_t)a->scratch & 255) == 0, UNOK_EINVAL,
                "draft_layer: scratch of %lld bytes (256-byte aligned) required, got %lld", (long long)b.bytes,
