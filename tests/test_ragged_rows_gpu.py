@@ -81,3 +81,37 @@ def test_attention_backward_reads_fp32_pre_norm_columns(dev, D, Hq, Hkv, norm):
     diff, mag = (fused[:, :e].float() - ref[:, :e].float()).abs(), ref[:, :e].float().abs()
     assert _rel(fused[:, :e], ref[:, :e]) < 2e-3
     assert bool((diff <= mag.clamp_min(mag.max() * 2 ** -8) * 2 ** -7).all())
+
+
+def test_fused_products_refuse_mismatched_operands(dev):
+    """What the separate products refuse, the fused ones refuse too: dtypes and sizes of weights, norm
+    weights, extension operands and outputs."""
+    bf, M, H, F, nq, nk, r = torch.bfloat16, 70, 128, 256, 4, 2, 32
+    n = 128 * (nq + 2 * nk)
+    z = lambda *s, dtype=bf: torch.zeros(*s, device=dev, dtype=dtype)
+    x, wqkv, wn = z(M, H), z(n, H), z(128)
+    pos = torch.zeros(M, device=dev, dtype=torch.int64)
+    cos, sin = K.rope_table(4, torch.ones(64, device=dev))
+    qkv = lambda x=x, w=wqkv, wq=wn, **kw: K.gemm_nt_qkv_rope(x, w, nq, nk, wq, wn, pos, cos, sin, 1e-6, any_rows=True, **kw)
+    qkv()
+    ext = lambda a, b: dict(a2=a, b2=b, segments=[(128 * nq, 0), (128 * (nq + nk), r), (n, 2 * r)])
+    qkv(**ext(z(M, 3 * r), z(n, r)))
+    for bad in (lambda: qkv(w=wqkv.float()), lambda: qkv(wq=wn.float()), lambda: qkv(wq=z(64)),
+                lambda: qkv(**ext(z(M, 3 * r, dtype=torch.float32), z(n, r))),
+                lambda: qkv(**ext(z(M, 3 * r), z(n, r, dtype=torch.float32))),
+                lambda: qkv(**ext(z(M - 1, 3 * r), z(n, r))), lambda: qkv(**ext(z(M, 3 * r), z(n - 8, r)))):
+        with pytest.raises(RuntimeError, match="gemm_nt_qkv_rope"):
+            bad()
+    w, h, b2 = z(2 * F, H), z(M, 2 * r), z(2 * F, 2 * r)
+    up = lambda **kw: K.gemm_nt_swiglu(x, w, any_rows=True, plain_rows=True, **kw)
+    up(a2=h, b2_interleaved=b2)
+    for kw in (dict(a2=h.float(), b2_interleaved=b2), dict(a2=h, b2_interleaved=b2.float()), dict(out=z(M, F - 8)),
+               dict(out=z(M, F, dtype=torch.float32))):
+        with pytest.raises(RuntimeError, match="gemm_nt_swiglu"):
+            up(**kw)
+    gu, wd, h, b2 = z(M, 2 * F), z(F, H), z(M, r), z(F, r)
+    down = lambda b=wd, a2=h, b2=b2, gu=gu, **kw: K.gemm_nt_swiglu_bwd(x, b, a2, b2, gu, any_rows=True, **kw)
+    down()
+    for kw in (dict(b=wd.float()), dict(a2=h.float()), dict(b2=b2.float()), dict(gu=gu.float()), dict(dgu=z(M, F))):
+        with pytest.raises(RuntimeError, match="gemm_nt_swiglu_bwd"):
+            down(**kw)

@@ -322,14 +322,19 @@ def gemm_nt_qkv_rope(x, w_qkv, nq, nk, wq, wk, pos, cos_tab, sin_tab, eps, *, a2
     _rowmajor(x, "x")
     _rowmajor(w_qkv, "w_qkv")
     M, Kd = x.shape
-    if w_qkv.shape != (128 * (nq + 2 * nk), Kd):
-        raise RuntimeError("gemm_nt_qkv_rope: w_qkv must be [128 (nq + 2 nk), K]")
+    if w_qkv.shape != (128 * (nq + 2 * nk), Kd) or w_qkv.dtype != x.dtype:
+        raise RuntimeError("gemm_nt_qkv_rope: w_qkv must be [128 (nq + 2 nk), K] in the dtype of x")
+    for w in (wq, wk):
+        if w is not None and (w.numel() != 128 or w.dtype != x.dtype):
+            raise RuntimeError("gemm_nt_qkv_rope: norm weights must be [128] in the dtype of x")
     K2 = 0
     seg_end, seg_col = [], []
     if a2 is not None:
         _rowmajor(a2, "a2")
         _rowmajor(b2, "b2")
         K2 = b2.shape[1]
+        if a2.dtype != x.dtype or b2.dtype != x.dtype or a2.shape[0] != M or b2.shape[0] != w_qkv.shape[0]:
+            raise RuntimeError("gemm_nt_qkv_rope: a2 [M,*] and b2 [N,K2] in the dtype of x required")
         segs = list(segments) if segments else [(w_qkv.shape[0], 0)]
         for _, col in segs:
             if col + K2 > a2.shape[1]:
@@ -388,14 +393,17 @@ def gemm_nt_swiglu(a: torch.Tensor, b_interleaved: torch.Tensor, *, a2: torch.Te
         _rowmajor(a2, "a2")
         _rowmajor(b2_interleaved, "b2")
         K2 = b2_interleaved.shape[1]
-        if b2_interleaved.shape[0] != rows or a2.shape[0] != M or a2.shape[1] < K2:
-            raise RuntimeError("gemm_nt_swiglu: a2 [M,>=K2] and b2 [N,K2] required")
+        if b2_interleaved.shape[0] != rows or a2.shape[0] != M or a2.shape[1] < K2 or a2.dtype != a.dtype \
+                or b2_interleaved.dtype != a.dtype:
+            raise RuntimeError("gemm_nt_swiglu: a2 [M,>=K2] and b2 [N,K2] in the dtype of a required")
     if gu is not None:
         _rowmajor(gu, "gu")
         if tuple(gu.shape) != (M, rows) or gu.dtype != a.dtype:
             raise RuntimeError("gemm_nt_swiglu: gu must be [M, N] in the dtype of a")
     out = out if out is not None else torch.empty((M, rows // 2), device=a.device, dtype=a.dtype)
     _rowmajor(out, "out")
+    if tuple(out.shape) != (M, rows // 2) or out.dtype != a.dtype:
+        raise RuntimeError("gemm_nt_swiglu: out must be [M, N/2] in the dtype of a")
     rec = _recorder
     if rec is not None and rec.predicate(a.dtype, M, rows, K, K2, [rows]):
         ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -420,17 +428,19 @@ def gemm_nt_swiglu_bwd(a: torch.Tensor, b: torch.Tensor, a2: torch.Tensor | None
         _rowmajor(t, n)
     M, K = a.shape
     F = b.shape[0]
-    if b.shape[1] != K or tuple(gu.shape) != (M, 2 * F):
-        raise RuntimeError("gemm_nt_swiglu_bwd: a [M,K], b [F,K] and gu [M,2F] required")
+    if b.shape[1] != K or tuple(gu.shape) != (M, 2 * F) or any(t.dtype != torch.bfloat16 for t in (a, b, gu)):
+        raise RuntimeError("gemm_nt_swiglu_bwd: bf16 a [M,K], b [F,K] and gu [M,2F] required")
     K2 = 0
     if a2 is not None:
         _rowmajor(a2, "a2")
         _rowmajor(b2, "b2")
         K2 = b2.shape[1]
-        if b2.shape[0] != F or a2.shape[0] != M or a2.shape[1] < K2:
-            raise RuntimeError("gemm_nt_swiglu_bwd: a2 [M,>=K2] and b2 [F,K2] required")
+        if b2.shape[0] != F or a2.shape[0] != M or a2.shape[1] < K2 or a2.dtype != a.dtype or b2.dtype != a.dtype:
+            raise RuntimeError("gemm_nt_swiglu_bwd: bf16 a2 [M,>=K2] and b2 [F,K2] required")
     dgu = dgu if dgu is not None else torch.empty((M, 2 * F), device=a.device, dtype=a.dtype)
     _rowmajor(dgu, "dgu")
+    if tuple(dgu.shape) != (M, 2 * F) or dgu.dtype != a.dtype:
+        raise RuntimeError("gemm_nt_swiglu_bwd: dgu must be [M, 2F] in the dtype of a")
     rec = _recorder
     if rec is not None and rec.predicate(a.dtype, M, F, K, K2, [F]):
         ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
