@@ -49,8 +49,9 @@ int unok_gemm_nt(int in_dtype, int out_dtype, int M, int N, int K,
  * whose K the library splits into ranges (few rows, too few output tiles for the chip), ranges x M x N
  * floats; a second kernel adds the partials in range order, so a result does not depend on timing.
  * plan 0: the library's choice of tile and ranges, as unok_gemm_nt_plan returns it for the sizes:
- * tile + 16 * ranges with tile 1: 256x256, 2: 128x256, 3: 128x128, 4: 64 rows x all columns, 5: 256x256
- * with 64-bit addresses (0: the register-staged kernel, no ranges); otherwise that plan. */
+ * tile + 16 * ranges with tile 1: 256x256, 2: 128x256, 3: 128x128, 4: 64 rows x all columns, 6: 192x256, and
+ * for fp32 products, which have no ranges, 7: 64x64, 8: 32x32; otherwise that plan, if the tile takes the product.
+ * 0 (the register-staged kernel) and 5 (256x256 with 64-bit addresses) are choices of the library only. */
 int unok_gemm_nt_plan(int in_dtype, int M, int N, int K, int K2, int nseg, const int* seg_end);
 int unok_gemm_nt_ws(int in_dtype, int out_dtype, int M, int N, int K,
                     const void* A, int64_t lda, const void* B, int64_t ldb,

@@ -1,0 +1,41 @@
+"""The library's choice of tiles and K ranges (unok_gemm_nt_plan, a function of the sizes alone) at sizes
+on both sides of its lines, where both sides were measured."""
+import pytest
+
+from uno_amd import _native as N
+from uno_amd import kernels as K
+
+F32_64, F32_32 = 7, 8
+
+
+@pytest.fixture(autouse=True)
+def _built():
+    if not N.LIB_PATH.exists():
+        pytest.skip("libunok.so not built")
+
+
+def _f32(M, Nn, Kd, K2=0):
+    return N.lib().unok_gemm_nt_plan(N.F32, M, Nn, Kd, K2, 1 if K2 else 0, N.int_array([Nn] if K2 else []))
+
+
+# us on 64x64 / 32x32 tiles: the last figures of each line
+@pytest.mark.parametrize("M,Nn,Kd,K2,tile", [
+    (1334, 4096, 8, 0, F32_64),      # 11 / 42
+    (3837, 1536, 64, 8, F32_64),     # 33 / 62
+    (3502, 1536, 33, 32, F32_64),    # 29 / 69
+    (407, 4096, 8, 8, F32_64),       # 9 / 16
+    (4066, 1024, 256, 32, F32_64),   # 67 / 77
+    (4096, 1536, 128, 0, F32_64),    # 40 / 50
+    (4096, 1536, 256, 0, F32_32),    # 71 / 65
+    (512, 4096, 128, 0, F32_32),     # 23 / 20
+    (1024, 1536, 256, 0, F32_32),    # 40 / 20
+    (2048, 768, 4096, 0, F32_32),    # 594 / 232
+    (512, 768, 256, 8, F32_32),      # 33 / 8, the parity step's products
+    (2000, 1536, 255, 0, F32_64),    # 46 / 72 (K no multiple of 4: element loads)
+    (2000, 250, 9, 0, F32_64),       # 6.1 / 7.6
+    (300, 770, 255, 0, F32_32),      # 33 / 9
+    (2048, 256, 8, 0, F32_32),       # 6 / 6
+    (8192, 2048, 256, 0, F32_64),    # from 2048 tiles on
+])
+def test_fp32_tiles(M, Nn, Kd, K2, tile):
+    assert _f32(M, Nn, Kd, K2) == tile + 16

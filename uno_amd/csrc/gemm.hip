@@ -1704,7 +1704,7 @@ __global__ __launch_bounds__(256) void nt_splitk_reduce_kernel(const GemmNT p, c
 // 128 x 4096 x 4096 at 38 in one range of 128x128 tiles and 18 in eight.
 // ---------------------------------------------------------------------------------------
 enum NtTile { NT_REG = 0, NT_256 = 1, NT_128_256 = 2, NT_128 = 3, NT_SKINNY = 4, NT_LARGE64 = 5,
-              NT_192_256 = 6 };
+              NT_192_256 = 6, NT_F32_64 = 7, NT_F32_32 = 8 };
 struct NtPlan { int tile, splits; };
 
 static bool nt_segs_ok(const GemmNT& p, int bn) {
@@ -2007,27 +2007,45 @@ UNOK_EXPORT int unok_lmhead_ce_grad(int R, int V, int K, const void* H, int64_t 
   return unok::check_launch("lmhead_ce_grad");
 }
 
-// fp32 products: eight waves share the K walk of a tile where it is long (230 rows, 4096 -> 256: 581 us
-// on 64x64 tiles, 40 us here; its 64 tiles leave most CUs idle), four else. From eight 64x64 tiles per CU
-// on the latency that this divides is covered by other workgroups, and the 64x64 kernel keeps the
-// sums' order.
+// fp32 products: 32x32 tiles whose waves share the K walk, eight of them where it is long (230 rows, 4096
+// -> 256: 581 us on 64x64 tiles, 40 us here; its 64 tiles leave most CUs idle), four else; or 64x64 tiles
+// where a short K leaves those waves nothing to share and the outputs, which a 32x32 tile pays for four
+// times as often, are what the time goes to. The cheaper by a model of the measured times (us, with T
+// 64x64 tiles and g groups of 64 k per wave): 64x64 4 + (0.11 + T / 12000) (K + K2); 32x32 4 + (0.0265 +
+// at most 0.013 for the first group + 0.032 for each further one) T, with eight waves 4 + (0.03 + 0.068 g)
+// T, and with element loads 4 + (0.02 + 0.0003 (K + K2)) T. Measured, 64x64 / 32x32: 1334 x 4096 x 8 11 /
+// 42, 512 x 4096 x 64 13 / 19, x 128 23 / 20, x 512 77 / 44; 4096 x 1536 x 128 40 / 50, x 256 71 / 65; element
+// loads 2000 x 1536 x 255 46 / 72, 300 x 770 x 255 33 / 9. Up to 128 tiles the 32x32 ones are not behind with
+// 16-byte loads; from eight 64x64 tiles per CU on the latency that they divide is covered by other workgroups,
+// and the 64x64 kernel keeps the sums' order.
+static int nt_f32_tile(int M, int N, int K, int K2, bool vec) {
+  const int64_t big = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+  if (big >= 2048) return NT_F32_64;
+  if (big <= 128 && vec) return NT_F32_32;
+  const int nw = K >= 1024 ? 8 : 4, n = (K + 15) / 16 + (K2 + 15) / 16, g = (n + 4 * nw - 1) / (4 * nw);
+  const double t64 = 4 + (0.11 + big / 12000.) * (K + K2);
+  const double t32 = 4 + big * (!vec ? 0.02 + 0.0003 * (K + K2) :
+                                nw == 8 ? 0.03 + 0.068 * g :
+                                0.0265 + 0.0008 * (n < 16 ? n : 16) + 0.032 * (g > 1 ? g - 1 : 0));
+  return t64 < t32 ? NT_F32_64 : NT_F32_32;
+}
+
 template <typename OutT, bool VEC>
-static void launch_nt_f32_t(const GemmNT& p, hipStream_t st) {
-  const int64_t big = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64);
-  if (big >= 2048) {
+static void launch_nt_f32_t(const GemmNT& p, int tile, hipStream_t st) {
+  if (tile == NT_F32_64) {
     const dim3 grid64((p.N + 63) / 64, (p.M + 63) / 64);
     hipLaunchKernelGGL((gemm_nt_f32_tile64_kernel<OutT>), grid64, dim3(256), 0, st, p);
     return;
   }
-  const dim3 grid((p.N + F32_T - 1) / F32_T, (p.M + F32_T - 1) / F32_T);   // below 8192 tiles: M < 2^17
+  const dim3 grid((p.N + F32_T - 1) / F32_T, (p.M + F32_T - 1) / F32_T);
   if (p.K >= 1024) hipLaunchKernelGGL((gemm_nt_f32_kernel<OutT, VEC, 8>), grid, dim3(512), 0, st, p);
   else hipLaunchKernelGGL((gemm_nt_f32_kernel<OutT, VEC, 4>), grid, dim3(256), 0, st, p);
 }
 
 template <typename OutT>
-static void launch_nt_f32(const GemmNT& p, bool vec, hipStream_t st) {
-  if (vec) launch_nt_f32_t<OutT, true>(p, st);
-  else launch_nt_f32_t<OutT, false>(p, st);
+static void launch_nt_f32(const GemmNT& p, bool vec, int tile, hipStream_t st) {
+  if (vec) launch_nt_f32_t<OutT, true>(p, tile, st);
+  else launch_nt_f32_t<OutT, false>(p, tile, st);
 }
 
 static int gemm_nt_any(int in_dtype, int out_dtype, int M, int N, int K,
@@ -2061,8 +2079,11 @@ static int gemm_nt_any(int in_dtype, int out_dtype, int M, int N, int K,
                      (!p.A2 || (K2 % 4 == 0 && lda2 % 4 == 0 && ldb2 % 4 == 0 && aligned16(A2) && aligned16(B2) &&
                                 p.seg_col[0] % 4 == 0 && p.seg_col[1] % 4 == 0 && p.seg_col[2] % 4 == 0 &&
                                 p.seg_col[3] % 4 == 0));
-    if (out_dtype == UNOK_BF16) launch_nt_f32<bf16_t>(p, vec, st);
-    else launch_nt_f32<float>(p, vec, st);
+    const int tile = plan > 0 ? plan & 15 : nt_f32_tile(M, N, K, p.A2 ? K2 : 0, vec);
+    UNOK_REQUIRE((tile == NT_F32_64 || (tile == NT_F32_32 && M <= 32 * 65535)) && plan >> 4 <= 1, UNOK_EINVAL,
+                 "gemm_nt: plan %d does not take this product", plan);
+    if (out_dtype == UNOK_BF16) launch_nt_f32<bf16_t>(p, vec, tile, st);
+    else launch_nt_f32<float>(p, vec, tile, st);
     return unok::check_launch("gemm_nt_f32");
   }
   // bf16 MFMA path: 16-byte vector loads need K-contiguous rows with 8-element granularity.
@@ -2149,10 +2170,11 @@ UNOK_EXPORT int unok_gemm_nt(int in_dtype, int out_dtype, int M, int N, int K,
                      R, ldr, gate, alpha, 0, nullptr, 0, stream);
 }
 
-// The library's choice for a product with a workspace: tile + 16 * ranges (0: fp32, and sizes or
-// segments only the register-staged kernel takes). K2 = 0 without an extension.
+// The library's choice for a product with a workspace: tile + 16 * ranges (0: sizes or segments that only
+// the register-staged kernel takes). K2 = 0 without an extension.
 UNOK_EXPORT int unok_gemm_nt_plan(int in_dtype, int M, int N, int K, int K2, int nseg, const int* seg_end) {
-  if (in_dtype != UNOK_BF16 || M <= 0 || N <= 0 || K <= 0) return 0;
+  if ((in_dtype != UNOK_BF16 && in_dtype != UNOK_F32) || M <= 0 || N <= 0 || K <= 0) return 0;
+  if (in_dtype == UNOK_F32) return nt_f32_tile(M, N, K, K2 > 0 ? K2 : 0, K % 4 == 0 && (K2 <= 0 || K2 % 4 == 0)) + 16;
   GemmNT p{};
   p.M = M; p.N = N; p.K = K; p.K2 = K2; p.lda = p.ldb = K; p.lda2 = p.ldb2 = K2; p.ldc = N;
   p.nseg = 1;
