@@ -45,7 +45,10 @@ def test_nt_f32_segments(dev, r):
     assert _rel(K.gemm_nt(a, b, a2=a2, b2=b2, segments=segs), ref) < 2e-6
 
 
-@pytest.mark.parametrize("Mr,P,Q", [(512, 256, 8), (512, 8, 256), (1, 1, 1), (257, 65, 24), (700, 17, 70), (64, 100, 100)])
+@pytest.mark.parametrize("Mr,P,Q", [(512, 256, 8), (512, 8, 256), (1, 1, 1), (257, 65, 24), (700, 17, 70), (64, 100, 100),
+                                    # both sides of the line to 64x64 tiles (320 of them, 36 (rows - 10), 64 rows)
+                                    (1, 1000, 1290), (1, 1000, 1270), (33, 2040, 1700), (33, 2040, 1600), (64, 3840, 2100),
+                                    (65, 3840, 2100)])
 @pytest.mark.parametrize("offset", [0, 1])
 def test_tn_f32(dev, Mr, P, Q, offset):
     print(f"[f32 tn] {Mr} {P}x{Q} offset {offset}", flush=True)

@@ -698,6 +698,54 @@ __global__ __launch_bounds__(256) void gemm_tn_bf16_kernel(const GemmTN p) {
     }
 }
 
+// fp32 with few rows and many outputs: 64x64 tiles, 16-deep row slices, 4x4 outputs per thread (the launch
+// holds the line and both sides' times). Bound by the workgroups' fixed cost and the output's bytes.
+__global__ __launch_bounds__(256) void gemm_tn_f32_tile64_kernel(const GemmTN p) {
+  __shared__ float As[16][65], Bs[16][65];
+  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+  const int nQ = (p.Q + 63) / 64;
+  const int p0 = (blockIdx.x / nQ) * 64, q0 = (blockIdx.x % nQ) * 64;
+  const int mbeg = blockIdx.y * p.rows_per_split;
+  const int mend = min(p.Mrows, mbeg + p.rows_per_split);
+  const float* A = (const float*)p.A;
+  const float* B = (const float*)p.B;
+  float acc[4][4] = {};
+  for (int mk = mbeg; mk < mend; mk += 16) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int e = tid + 256 * q, k = e >> 6, c = e & 63;
+      const int gm = mk + k;
+      As[k][c] = (gm < mend && p0 + c < p.P) ? A[(int64_t)gm * p.lda + p0 + c] : 0.f;
+      Bs[k][c] = (gm < mend && q0 + c < p.Q) ? B[(int64_t)gm * p.ldb + q0 + c] : 0.f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      float av[4], bv[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) av[i] = As[k][ty + 16 * i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) bv[j] = Bs[k][tx + 16 * j];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
+    }
+    __syncthreads();
+  }
+  float* W = p.WS + (int64_t)blockIdx.y * p.P * p.Q;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = p0 + ty + 16 * i;
+    if (row >= p.P) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int col = q0 + tx + 16 * j;
+      if (col < p.Q) W[(int64_t)row * p.Q + col] = acc[i][j] * p.alpha;
+    }
+  }
+}
+
 // fp32: 64 columns of the wider operand X (XP: A, else B) by 16 of the other, S; the four waves take
 // the split's rows four at a time in turn. Lane l loads X columns 4 (l % 16) + 0..3 and S column l % 16
 // of row l / 16 (VEC: one 16-byte load), so MFMA e multiplies X columns 4 i + e; eight steps are
@@ -2550,7 +2598,14 @@ UNOK_EXPORT int unok_gemm_tn(int in_dtype, int Mrows, int P, int Q, const void* 
     const int64_t ldx = xp ? lda : ldb;
     const bool vec = NX % 4 == 0 && ldx % 4 == 0 && aligned16(xp ? A : B);
     const dim3 grid((unsigned)((NX + 63) / 64) * (unsigned)((NS + 15) / 16), nz);
-    if (xp) {
+    // Up to 64 rows the 64x16 tiles' four waves have a few loads each, and a workgroup's fixed cost, paid
+    // four times as often as on 64x64 tiles, decides once there are enough of them (us, 64x64 / 64x16:
+    // 16 rows 300 x 4096 10.6 / 11.8, 4096 x 6144 58 / 109; 33 rows 1000 x 2048 16 / 16, 4096 x 2048 36 / 42;
+    // 64 rows 1000 x 4096 31 / 30, 4096 x 2048 41 / 43, 4096 x 6144 95 / 114; 100 rows 4096 x 6144 129 / 118).
+    const int64_t big = (int64_t)((P + 63) / 64) * ((Q + 63) / 64);
+    if (Mrows <= 64 && big >= 320 && big >= 36ll * (Mrows - 10)) {
+      hipLaunchKernelGGL(gemm_tn_f32_tile64_kernel, dim3((unsigned)big, nz), dim3(256), 0, st, p);
+    } else if (xp) {
       if (vec) hipLaunchKernelGGL((gemm_tn_f32_kernel<true, true>), grid, dim3(256), 0, st, p);
       else hipLaunchKernelGGL((gemm_tn_f32_kernel<false, true>), grid, dim3(256), 0, st, p);
     } else {
