@@ -39,3 +39,36 @@ def _f32(M, Nn, Kd, K2=0):
 ])
 def test_fp32_tiles(M, Nn, Kd, K2, tile):
     assert _f32(M, Nn, Kd, K2) == tile + 16
+
+
+def _bf16(M, Nn, Kd, K2=0):
+    return K.nt_plan(M, Nn, Kd, K2, (Nn,) if K2 else ())
+
+
+SKINNY, REG = 4, 0
+
+
+# us in one range / in the ranges taken: the last figures of each line
+@pytest.mark.parametrize("M,Nn,Kd,tile,splits", [
+    (8192, 64, 1024, SKINNY, 1),      # 9.4 / 14.0 in four
+    (6000, 128, 1024, SKINNY, 1),     # 13.1 / 15.6 in two
+    (15955, 32, 1024, SKINNY, 1),     # 9.6 / 13.0 in two
+    (15955, 64, 2048, SKINNY, 1),     # 15.1 / 19.0 in two
+    (4096, 192, 1024, SKINNY, 1),     # 15.8 / 17.2 in two
+    (12000, 64, 12288, SKINNY, 1),    # 70 / 74 in two: the activations' bytes
+    (16384, 64, 4096, SKINNY, 1),
+    (777, 192, 128, REG, 1),          # 7.1 / 7.8 on 64-row tiles
+    (8192, 192, 128, SKINNY, 1),
+])
+def test_skinny_products_in_one_range(M, Nn, Kd, tile, splits):
+    assert _bf16(M, Nn, Kd) == (tile, splits)
+
+
+@pytest.mark.parametrize("M,Nn,Kd", [(2048, 64, 4096),     # 24 / 14
+                                     (777, 192, 12288),    # 112 / 21
+                                     (17, 32, 2048),       # 14 / 7
+                                     (6000, 64, 4096),     # 24 / 17
+                                     (8192, 128, 12288)])  # 90 / 57
+def test_skinny_products_in_ranges(M, Nn, Kd):
+    tile, splits = _bf16(M, Nn, Kd)
+    assert tile == SKINNY and splits > 1

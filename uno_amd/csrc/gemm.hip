@@ -1799,24 +1799,31 @@ static void launch_nt_fused(const GemmNT& p, hipStream_t st) {
 static NtPlan nt_plan(const GemmNT& p, bool may_split) {
   const int nk1 = p.K / 64, nk2 = nt_ext_tiles(p);
   may_split = may_split && out_vec4_ok(p) && (int64_t)p.M * p.N < (1ll << 32);
-  if (p.N <= 192 && !p.A2 && p.K % 64 == 0 && nk1 > 0) {
+  if (p.N <= 192 && !p.A2 && p.K % 64 == 0 && nk1 > (p.N > 128 && p.M < 4096 ? 2 : 0)) {
     // Skinny products (LoRA x A^T and dY B, N = r .. 3r): every activation row is read from HBM
-    // once, by 64-row tiles that span all N columns. (N = 256 and 384 run faster on the tiles below.)
-    // Few rows take K ranges, one round of workgroups (two per CU for N <= 64), at least four K tiles
-    // and at most 8 MB of partials: 2048 x 64 x 4096 22.7 -> 11.5 us, 777 x 192 x 12288 107 -> 21 us.
+    // once, by 64-row tiles that span all N columns. (N = 256 and 384 run faster on the tiles below; 192
+    // columns with fewer than 4096 rows and two K tiles or less on the register-staged kernel, 7.1 / 7.8 us
+    // at 777 x 192 x 128.)
+    // Few rows take K ranges where these pay: up to 16, of at least four K tiles, in one round of
+    // workgroups (two per CU for N <= 64), by the measured times (us, with c = columns / 64, n = K tiles of
+    // a range): (2.7 + 1.33 c) + (0.195 + 0.12 c) n, not below the activations' bytes at 5.2 TB/s; ranges
+    // add 2.5 and the partials written and read once at 2.5 TB/s. Measured, one range / best: 2048 x 64 x
+    // 4096 24 / 14, 777 x 192 x 12288 112 / 21, 4096 x 64 x 2048 14 / 12 in four; but 8192 x 64 x 1024 9 / 14 and
+    // 15955 x 64 x 2048 15 / 19 in two or four.
     const int64_t wg = (p.M + 63) / 64;
-    int64_t s = 1;
-    if (may_split && wg < 256) {
-      s = (p.N <= 64 ? 512 : 256) / wg;
-      s = s < nk1 / 4 ? s : nk1 / 4;
-      s = s < 16 ? s : 16;
-      const int64_t cap = (8ll << 20) / ((int64_t)p.M * p.N * 4);
-      s = s < cap ? s : cap;
-      if (s < 1 || nk1 < 16) s = 1;
+    int best = 1;
+    if (may_split) {
+      const double c = (p.N + 63) / 64, c0 = 2.7 + 1.33 * c, c1 = 0.195 + 0.12 * c;
+      const double hbm = (double)(p.M + p.N) * p.K * 2 / 5.2e6;
+      double best_t = fmax(c0 + c1 * nk1, hbm);
+      for (int s = 2; s <= 16 && s <= nk1 / 4 && wg * s <= (p.N <= 64 ? 512 : 256); ++s) {
+        const double t = fmax(c0 + c1 * ((nk1 + s - 1) / s), hbm) + 2.5 + (double)p.M * p.N * (8.0 * s + 2) / 2.5e6;
+        if (t < best_t) { best_t = t; best = s; }
+      }
     }
-    return {NT_SKINNY, (int)s};
+    return {NT_SKINNY, best};
   }
-  if (p.K % 64 || nk1 == 0 || (p.A2 && p.K2 % 32) || !nt_segs_ok(p, 128)) return {NT_REG, 1};
+  if (p.K % 64 || nk1 == 0 || (p.A2 && p.K2 % 32) || !nt_segs_ok(p, 128) || (p.N <= 192 && !p.A2)) return {NT_REG, 1};
   if (!buffer_ranges_ok(p)) {
     // operands beyond 32-bit buffer offsets: the kernel with 64-bit addresses
     const int64_t big = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256);
