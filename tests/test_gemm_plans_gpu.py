@@ -233,3 +233,14 @@ def test_swiglu_product_on_the_fused_projection_rows(dev, M, F, Kd, r):
     got = K.gemm_nt_swiglu(x, w, gu=gus[1], any_rows=True, plain_rows=True, **kw)
     assert torch.equal(got, ref) and torch.equal(*gus)
     assert torch.equal(K.gemm_nt_swiglu(x, w, any_rows=True, plain_rows=True, **kw), ref)
+
+
+@pytest.mark.parametrize("M,Nn,Kd", [(300, 4096, 12288), (485, 4096, 12288), (777, 6144, 1024), (1196, 2048, 11008)])
+@pytest.mark.parametrize("K2", [32, 128])
+def test_zero_extension_changes_no_bit(dev, M, Nn, Kd, K2):
+    """As above for the library's own choice: a product with an adapter of zeros is the plain product."""
+    torch.manual_seed(M + K2)
+    a, b = torch.randn(M, Kd, device=dev).bfloat16(), torch.randn(Nn, Kd, device=dev).bfloat16()
+    h, bl = torch.randn(M, K2, device=dev).bfloat16(), torch.zeros(Nn, K2, device=dev).bfloat16()
+    plain = K.gemm_nt(a, b, out_dtype=torch.float32)
+    assert torch.equal(plain, K.gemm_nt(a, b, a2=h, b2=bl, out_dtype=torch.float32))

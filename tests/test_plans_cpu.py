@@ -72,3 +72,11 @@ def test_skinny_products_in_one_range(M, Nn, Kd, tile, splits):
 def test_skinny_products_in_ranges(M, Nn, Kd):
     tile, splits = _bf16(M, Nn, Kd)
     assert tile == SKINNY and splits > 1
+
+
+@pytest.mark.parametrize("M,Nn,Kd", [(300, 4096, 12288), (485, 4096, 12288), (1196, 2048, 11008), (777, 4096, 4096),
+                                     (64, 4096, 4096), (5, 512, 192), (3000, 24576, 4096)])
+@pytest.mark.parametrize("K2", [32, 64, 128, 384])
+def test_an_extension_leaves_the_ranges(M, Nn, Kd, K2):
+    """The same K ranges with and without an extension, so that one of zeros changes no bit."""
+    assert _bf16(M, Nn, Kd, K2)[1] == _bf16(M, Nn, Kd)[1]

@@ -940,7 +940,8 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_w4m16_kernel(const GemmNT p)
   // and its second 32-wide k-step then runs on zeroed fragments.
   const int nk_all = nk1 + (ext ? (p.K2 + BK - 1) / BK : 0);
   // this range's K tiles [kt0, nk): the main tiles are divided among the ranges and the extension
-  // belongs to the last one, so an extension of zeros leaves every sum as it was
+  // belongs to the last one, so an extension of zeros leaves every sum as it was (nt_plan counts the
+  // ranges without it)
   const int kt0 = EPI == 6 ? (int)((int64_t)split * nk1 / p.splits) : 0;
   const int nk = EPI == 6 && split + 1 < p.splits ? (int)((int64_t)(split + 1) * nk1 / p.splits) : nk_all;
   const bool half_last = ext && nk == nk_all && (p.K2 % BK) != 0;
@@ -1831,19 +1832,21 @@ static NtPlan nt_plan(const GemmNT& p, bool may_split) {
     return {large ? NT_LARGE64 : NT_REG, 1};
   }
   const bool wide = p.N > 128 && nt_segs_ok(p, 256);
+  // The count of ranges comes from the product without its extension, and the tile for that count from the
+  // whole: the tiles add an output's products in one order, so a product sums alike with and without one.
   NtPlan best = {NT_128, 1};
-  double best_t = 1e30;
-  for (int tile : {NT_256, NT_192_256, NT_128_256, NT_128}) {
-    if (!wide && tile != NT_128) continue;
-    for (int s = 1; s <= (may_split ? 16 : 1) && nk1 / s >= 4; ++s) {
-      const double t = nt_cost(tile, p.M, p.N, nk1, nk2, s);
-      if (t < best_t) { best_t = t; best = {tile, s}; }
+  auto choose = [&](int s0, int s1, int k2) {
+    double best_t = 1e30;
+    for (int tile : {NT_256, NT_192_256, NT_128_256, NT_128}) {
+      if (!wide && tile != NT_128) continue;
+      for (int s = s0; s <= s1 && (s == 1 || nk1 / s >= 4); ++s) {
+        const double t = nt_cost(tile, p.M, p.N, nk1, k2, s);
+        if (t < best_t) { best_t = t; best = {tile, s}; }
+      }
     }
-    if (nk1 < 4) {
-      const double t = nt_cost(tile, p.M, p.N, nk1, nk2, 1);
-      if (t < best_t) { best_t = t; best = {tile, 1}; }
-    }
-  }
+  };
+  choose(1, may_split ? 16 : 1, 0);
+  if (nk2) choose(best.splits, best.splits, nk2);
   return best;
 }
 
