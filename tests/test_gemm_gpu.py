@@ -72,7 +72,7 @@ def test_gemm_nt_lora_segments_gate_residual(dev, dtype):
 def test_gemm_nt_direct_to_lds_path(dev, M, N, Kd):
     """Shapes large enough (>= 512 tiles of 256x256, K a multiple of 64) for the direct-to-LDS
     kernel, including ragged M/N edges, with fp32 output."""
-    assert K.nt_uses_256_tiles(M, N, [N])
+    assert K.nt_uses_256_tiles(M, N, [N], Kd)
     torch.manual_seed(M + N)
     a = torch.randn(M, Kd, device=dev).bfloat16()
     b = torch.randn(N, Kd, device=dev).bfloat16()
@@ -105,7 +105,7 @@ def test_gemm_nt_direct_to_lds_lora_residual(dev):
     torch.manual_seed(2)
     M, Kd, r = 8192, 1024, 64
     ends = [4096, 5120, 6144]
-    assert K.nt_uses_256_tiles(M, ends[-1], ends)
+    assert K.nt_uses_256_tiles(M, ends[-1], ends, Kd, r)
     a = torch.randn(M, Kd, device=dev).bfloat16()
     w = torch.randn(ends[-1], Kd, device=dev).bfloat16() * 0.05
     h = torch.randn(M, 3 * r, device=dev).bfloat16()
@@ -280,7 +280,7 @@ def test_gemm_nt_lora_rank_not_multiple_of_64(dev, r):
     torch.manual_seed(r)
     M, N, Kd = 4096, 6144, 512
     ends = [4096, 5120, 6144]
-    assert K.nt_uses_256_tiles(M, N, ends)
+    assert K.nt_uses_256_tiles(M, N, ends, Kd, r)
     a = torch.randn(M, Kd, device=dev).bfloat16()
     w = (torch.randn(N, Kd, device=dev) * 0.1).bfloat16()
     h = torch.randn(M, 3 * r, device=dev).bfloat16()

@@ -48,10 +48,10 @@ def nt_plan(M: int, N_: int, K: int, K2: int = 0, seg_end: tuple = ()) -> tuple[
     return code & 15, max(1, code >> 4)
 
 
-def nt_uses_256_tiles(M: int, N: int, seg_end, K: int = 0) -> bool:
-    """Whether unok_gemm_nt runs a bf16 product on the 256x256 MFMA kernel."""
-    segs = tuple(seg_end)
-    return nt_plan(M, N, K or 4096, 64 if len(segs) > 1 else 0, segs if len(segs) > 1 else ())[0] == 1
+def nt_uses_256_tiles(M: int, N: int, seg_end, K: int, K2: int = 0) -> bool:
+    """Whether gemm_nt runs a bf16 product (with an extension of K2 columns) on the 256x256 MFMA kernel in
+    one range of K."""
+    return nt_plan(M, N, K, K2, tuple(seg_end) if K2 else ()) == (1, 1)
 
 
 def _rowmajor(t: torch.Tensor, name: str) -> None:
