@@ -53,6 +53,8 @@ int unok_gemm_nt(int in_dtype, int out_dtype, int M, int N, int K,
  * for fp32 products, which have no ranges, 7: 64x64, 8: 32x32; otherwise that plan, if the tile takes the product.
  * 0 (the register-staged kernel) and 5 (256x256 with 64-bit addresses) are choices of the library only. */
 int unok_gemm_nt_plan(int in_dtype, int M, int N, int K, int K2, int nseg, const int* seg_end);
+/* The tile on which unok_gemm_nt_swiglu, _swiglu_bwd and _qkv_rope run a product of M x N (N % 256 == 0). */
+int unok_gemm_nt_fused_tile(int M, int N, int K, int K2);
 int unok_gemm_nt_ws(int in_dtype, int out_dtype, int M, int N, int K,
                     const void* A, int64_t lda, const void* B, int64_t ldb,
                     const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,

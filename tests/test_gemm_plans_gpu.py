@@ -1,4 +1,4 @@
-"""The tiles and K ranges unok_gemm_nt_ws chooses between (256x256, 128x256, 128x128, 64 rows x all
+"""The tiles and K ranges unok_gemm_nt_ws chooses between (256x256, 192x256, 128x256, 128x128, 64 rows x all
 columns; one or several ranges) against fp32 torch products of the same operands, at tile edges and
 remainders, with strided operands, LoRA segments, row gate, residual and both output types.
 
@@ -30,7 +30,7 @@ def _call(plan, a, b, a2, b2, segs, out, res, gate, alpha, ranges):
 
 
 @pytest.mark.parametrize("M,Nn,Kd", [(1, 256, 64), (127, 256, 320), (129, 520, 256), (257, 1028, 448), (640, 512, 1024)])
-@pytest.mark.parametrize("tile", [1, 2, 3])
+@pytest.mark.parametrize("tile", [1, 2, 3, 6])
 @pytest.mark.parametrize("ranges", [1, 3])
 def test_tiles_and_ranges(dev, M, Nn, Kd, tile, ranges):
     if ranges > Kd // 64:
@@ -51,7 +51,8 @@ def test_tiles_and_ranges(dev, M, Nn, Kd, tile, ranges):
         assert _rel(out, a.float() @ b.float().T + r.float()) < tol, dt
 
 
-@pytest.mark.parametrize("tile,ends", [(1, [256, 512, 768]), (2, [512, 768, 1024]), (3, [128, 384, 512])])
+@pytest.mark.parametrize("tile,ends", [(1, [256, 512, 768]), (2, [512, 768, 1024]), (3, [128, 384, 512]),
+                                       (6, [256, 512, 768])])
 @pytest.mark.parametrize("K2", [32, 64, 96])
 @pytest.mark.parametrize("ranges", [1, 2, 5])
 def test_extension_segments(dev, tile, ends, K2, ranges):
@@ -116,8 +117,9 @@ def test_plan_rejects_what_a_tile_does_not_take(dev):
 @pytest.mark.parametrize("M", [1, 100, 129, 300, 511, 2100])
 @pytest.mark.parametrize("F,Kd,r", [(256, 128, 32), (1536, 512, 64)])
 def test_fused_epilogues_on_any_row_count(dev, M, F, Kd, r):
-    """The SwiGLU products on row counts between tiles: bit for bit the first M rows of the product over
-    rows padded to a multiple of 256, and no row past M written."""
+    """The SwiGLU products on row counts between tiles (128-row tiles at these sizes): bit for bit the first
+    M rows of the product over rows padded to a multiple of 256, and no row past M written."""
+    assert {N.lib().unok_gemm_nt_fused_tile(m, n, Kd, 0) for m in (M, (M + 255) // 256 * 256) for n in (F, 2 * F)} == {2}
     torch.manual_seed(M + F)
     P = (M + 255) // 256 * 256
     bf = torch.bfloat16
@@ -193,8 +195,11 @@ def test_192_row_tiles(dev, M, Nn, Kd, ranges, out_dtype):
 
 @pytest.mark.parametrize("M", [720, 777])
 def test_192_row_tiles_fused_epilogues(dev, M):
-    """The fused products at a row count for which 192-row tiles are the cheapest, against the separate
-    kernels: SwiGLU and its backward bit for bit, q|k|v with norm and RoPE to one bf16 rounding."""
+    """The fused products at a row count for which 192-row tiles are the cheapest (the q|k|v product's are
+    at others: test_fused_epilogues_by_tile), against the separate kernels: SwiGLU and its backward bit for
+    bit, q|k|v with norm and RoPE to one bf16 rounding."""
+    tile = N.lib().unok_gemm_nt_fused_tile
+    assert tile(M, 24576, 1024, 0) == 6 and tile(M, 12288, 1024, 0) == 6 and tile(M, 6144, 1024, 0) == 2
     torch.manual_seed(M)
     H, F, nq, nk = 1024, 12288, 32, 8
     x = torch.randn(M, H, device=dev).bfloat16()
@@ -244,3 +249,100 @@ def test_zero_extension_changes_no_bit(dev, M, Nn, Kd, K2):
     h, bl = torch.randn(M, K2, device=dev).bfloat16(), torch.zeros(Nn, K2, device=dev).bfloat16()
     plain = K.gemm_nt(a, b, out_dtype=torch.float32)
     assert torch.equal(plain, K.gemm_nt(a, b, a2=h, b2=bl, out_dtype=torch.float32))
+
+
+def _unsplit(a, b, a2=None, b2=None, segs=(), out_dtype=torch.bfloat16):
+    """gemm_nt in one range of K (the entry point without a workspace)."""
+    out = torch.empty(a.shape[0], b.shape[0], device=a.device, dtype=out_dtype)
+    N.call("unok_gemm_nt", N.BF16, N.dtype_code(out_dtype), a.shape[0], b.shape[0], a.shape[1], N.ptr(a), a.stride(0),
+           N.ptr(b), b.stride(0), N.ptr(a2), a2.stride(0) if a2 is not None else 0, N.ptr(b2),
+           b2.stride(0) if b2 is not None else 0, b2.shape[1] if b2 is not None else 0, len(segs),
+           N.int_array([s[0] for s in segs]), N.int_array([s[1] for s in segs]), N.ptr(out), out.stride(0), None, 0, None, 1.0,
+           N.stream())
+    return out
+
+
+def _tile(M, n, Kd, K2):
+    return N.lib().unok_gemm_nt_fused_tile(M, n, Kd, K2)
+
+
+# tile chosen, rows (ragged and whole), hidden width, FFN width
+@pytest.mark.parametrize("tile,M,H,F", [(1, 400, 1024, 12288), (1, 7655, 2048, 5632), (6, 300, 1024, 12288),
+                                        (6, 384, 1024, 12288), (2, 150, 1024, 12288)])
+@pytest.mark.parametrize("r", [0, 16, 32])
+def test_swiglu_epilogue_by_tile(dev, tile, M, H, F, r):
+    """SwiGLU in the epilogue of 256-, 192- and 128-row tiles with a last tile that is not full, with and
+    without the LoRA extension (2 r columns) and the stored [gate | up]: bit for bit the plain product
+    followed by the SwiGLU kernel, and no row past M written."""
+    assert _tile(M, 2 * F, H, 2 * r) == tile
+    torch.manual_seed(M + r)
+    bf = torch.bfloat16
+    x, w = (torch.randn(M, H, device=dev) * 0.5).to(bf), (torch.randn(2 * F, H, device=dev) * 0.05).to(bf)
+    kw, ext = {}, ()
+    if r:
+        h, sb = (torch.randn(M, 2 * r, device=dev) * 0.5).to(bf), (torch.randn(2 * F, r, device=dev) * 0.1).to(bf)
+        b2 = torch.zeros(F // 64, 2, 64, 2 * r, device=dev, dtype=bf)
+        b2[:, 0, :, :r], b2[:, 1, :, r:] = sb[:F].view(-1, 64, r), sb[F:].view(-1, 64, r)
+        kw = dict(a2=h, b2_interleaved=b2.view(2 * F, 2 * r))
+        pad = torch.zeros(2 * F, 2 * r, device=dev, dtype=bf)      # the same extension over plain rows, same K order
+        pad[:F, :r], pad[F:, r:] = sb[:F], sb[F:]
+        ext = (h, pad, [(2 * F, 0)])
+    want = _unsplit(x, w, *ext)
+    s = K.swiglu_fwd(want, F)
+    for store in (False, True):
+        out, gu = torch.full((M + 300, F), 7.0, device=dev, dtype=bf), torch.full((M + 300, 2 * F), 7.0, device=dev, dtype=bf)
+        K.gemm_nt_swiglu(x, w, out=out[:M], gu=gu[:M] if store else None, any_rows=True, plain_rows=True, **kw)
+        assert torch.equal(out[:M], s) and bool((out[M:] == 7).all())
+        if store:
+            assert torch.equal(gu[:M], want) and bool((gu[M:] == 7).all())
+
+
+@pytest.mark.parametrize("tile,M,H,F", [(1, 1000, 1024, 12288), (1, 7655, 2048, 5632), (6, 700, 1024, 12288),
+                                        (6, 768, 1024, 12288), (2, 300, 1024, 12288)])
+@pytest.mark.parametrize("r", [0, 32])
+def test_swiglu_backward_epilogue_by_tile(dev, tile, M, H, F, r):
+    """The SwiGLU backward likewise."""
+    assert _tile(M, F, H, r) == tile
+    torch.manual_seed(M + r)
+    bf = torch.bfloat16
+    dy, wt = (torch.randn(M, H, device=dev) * 0.5).to(bf), (torch.randn(F, H, device=dev) * 0.05).to(bf)
+    gu = (torch.randn(M, 2 * F, device=dev) * 2).to(bf)
+    a2, b2 = ((torch.randn(M, r, device=dev) * 0.5).to(bf), (torch.randn(F, r, device=dev) * 0.1).to(bf)) if r else (None, None)
+    want = K.swiglu_bwd(_unsplit(dy, wt, a2, b2, [(F, 0)] if r else ()), gu, F)
+    dgu = torch.full((M + 300, 2 * F), 7.0, device=dev, dtype=bf)
+    K.gemm_nt_swiglu_bwd(dy, wt, a2, b2, gu, dgu=dgu[:M], any_rows=True)
+    assert torch.equal(dgu[:M], want) and bool((dgu[M:] == 7).all())
+
+
+@pytest.mark.parametrize("tile,M,H", [(1, 2000, 1024), (6, 1301, 1024), (6, 1344, 1024), (2, 700, 1024)])
+@pytest.mark.parametrize("r", [0, 32, 64])
+@pytest.mark.parametrize("pre_f32", [0, 1])
+def test_qkv_rope_epilogue_by_tile(dev, tile, M, H, r, pre_f32):
+    """q|k|v with norm and RoPE on 256-, 192- (in two 48-row passes) and 128-row tiles, with and without the
+    LoRA extension: v and the kept pre-norm columns bit for bit the plain fp32 product's rounding, q and k
+    within one bf16 rounding of the separate norm kernel, no row past M written."""
+    nq, nk, d, bf = 32, 8, 128, torch.bfloat16
+    n, e = d * (nq + 2 * nk), d * (nq + nk)
+    assert _tile(M, n, H, r) == tile
+    torch.manual_seed(M + r)
+    x, w = torch.randn(M, H, device=dev).to(bf), (torch.randn(n, H, device=dev) * 0.05).to(bf)
+    h, b2, segs = None, None, []
+    if r:
+        h, b2 = torch.randn(M, 3 * r, device=dev).to(bf), (torch.randn(n, r, device=dev) * 0.05).to(bf)
+        segs = [(d * nq, 0), (e, r), (n, 2 * r)]
+    wq, wk = (1 + 0.1 * torch.randn(2, d, device=dev)).to(bf)
+    inv = 1.0 / (1e6 ** (torch.arange(0, d, 2, device=dev).float() / d))
+    pos, (cos, sin) = torch.randint(0, 500, (M,), device=dev), K.rope_table(500, inv)
+    P = M + 300
+    full = lambda c, dt=bf: torch.full((P, c), 7.0, device=dev, dtype=dt)  # noqa: E731
+    q, k, v, rstd = full(d * nq), full(d * nk), full(d * nk), full(nq + nk, torch.float32)
+    pre = full(e, torch.float32 if pre_f32 else bf)
+    N.call("unok_gemm_nt_qkv_rope_any", M, H, nq, nk, N.ptr(x), H, N.ptr(w), H, N.ptr(h), 3 * r, N.ptr(b2), r, r, len(segs),
+           N.int_array([s[0] for s in segs]), N.int_array([s[1] for s in segs]), N.ptr(wq), N.ptr(wk), N.ptr(pos), N.ptr(cos),
+           N.ptr(sin), 500, 1e-6, N.ptr(q), N.ptr(k), N.ptr(v), N.ptr(rstd), N.ptr(pre), pre_f32, N.stream())
+    y = _unsplit(x, w, h, b2, segs, torch.float32)
+    q2, k2, v2, rstd2 = K.qknorm_rope_fwd(y, nq, nk, d, wq, wk, pos, inv, 1e-6, out_dtype=bf, with_v=True)
+    assert torch.equal(v[:M], v2) and torch.equal(pre[:M], y[:, :e].to(pre.dtype))
+    assert _rel(q[:M], q2) < 1e-3 and _rel(k[:M], k2) < 1e-3 and _rel(rstd[:M], rstd2.view(M, -1)) < 1e-5
+    for t in (q, k, v, rstd, pre):
+        assert bool((t[M:] == 7).all())

@@ -38,6 +38,7 @@ SIGNATURES: dict[str, tuple] = {
     "unok_gemm_nt": (_i, [_i, _i, _i, _i, _i, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _i,
                           _i, _ip, _ip, _p, _i64, _p, _i64, _p, _f, _p]),
     "unok_gemm_nt_plan": (_i, [_i, _i, _i, _i, _i, _i, _ip]),
+    "unok_gemm_nt_fused_tile": (_i, [_i, _i, _i, _i]),
     "unok_gemm_nt_ws": (_i, [_i, _i, _i, _i, _i, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _i,
                              _i, _ip, _ip, _p, _i64, _p, _i64, _p, _f, _i, _p, _i64, _p]),
     "unok_gemm_nt_swiglu": (_i, [_i, _i, _i, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _i, _p, _i64, _p, _i64, _p]),

@@ -1786,14 +1786,18 @@ static double nt_cost(int tile, int64_t M, int64_t N, int nk1, int nk2, int s) {
 
 static int nt_ext_tiles(const GemmNT& p) { return p.A2 ? (p.K2 + 63) / 64 : 0; }
 
-// Launches a product whose epilogue needs 256-wide tiles and whole sums on the cheapest row tile.
+// The row tile of a product whose epilogue needs 256-wide tiles and whole sums: the cheapest.
+static int nt_fused_tile(int64_t M, int64_t N, int nk1, int nk2) {
+  const double t256 = nt_cost(NT_256, M, N, nk1, nk2, 1), t192 = nt_cost(NT_192_256, M, N, nk1, nk2, 1),
+               t128 = nt_cost(NT_128_256, M, N, nk1, nk2, 1);
+  return t256 <= t192 && t256 <= t128 ? NT_256 : t192 <= t128 ? NT_192_256 : NT_128_256;
+}
+
 template <int EPI>
 static void launch_nt_fused(const GemmNT& p, hipStream_t st) {
-  const int nk1 = p.K / 64, nk2 = nt_ext_tiles(p);
-  const double t256 = nt_cost(NT_256, p.M, p.N, nk1, nk2, 1), t192 = nt_cost(NT_192_256, p.M, p.N, nk1, nk2, 1),
-               t128 = nt_cost(NT_128_256, p.M, p.N, nk1, nk2, 1);
-  if (t256 <= t192 && t256 <= t128) launch_nt_w4m16<bf16_t, EPI>(p, st);
-  else if (t192 <= t128) launch_nt_w4m16<bf16_t, EPI, 192>(p, st);
+  const int tile = nt_fused_tile(p.M, p.N, p.K / 64, nt_ext_tiles(p));
+  if (tile == NT_256) launch_nt_w4m16<bf16_t, EPI>(p, st);
+  else if (tile == NT_192_256) launch_nt_w4m16<bf16_t, EPI, 192>(p, st);
   else launch_nt_w4m16<bf16_t, EPI, 128>(p, st);
 }
 
@@ -2244,6 +2248,13 @@ UNOK_EXPORT int unok_gemm_nt_plan(int in_dtype, int M, int N, int K, int K2, int
   }
   const NtPlan pl = nt_plan(p, true);
   return pl.tile == NT_REG ? 0 : pl.tile + 16 * pl.splits;
+}
+
+// The tile (as unok_gemm_nt_plan's) on which the products with a fused epilogue run: N the product's
+// columns, K2 = 0 without an extension.
+UNOK_EXPORT int unok_gemm_nt_fused_tile(int M, int N, int K, int K2) {
+  if (M <= 0 || N <= 0 || K <= 0 || N % 256 || K % 64 || K2 < 0) return 0;
+  return nt_fused_tile(M, N, K / 64, (K2 + 63) / 64);
 }
 
 // unok_gemm_nt with a workspace of ws_bytes for the partial sums of a product whose K is split.
