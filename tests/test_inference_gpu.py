@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from oracle.model import Cfg, decoder, init_lora, init_params
+from uno_amd import kernels as K
 from uno_amd.inference import BlockDecoder
 from uno_amd.model import UnoQwen3Config, UnoQwen3ForCausalLM
 from uno_amd.training.config import LoraSettings
@@ -203,3 +204,29 @@ def test_draft_block_with_strided_weights(dev):
         dec.prefill(cache, prompt)
         logits.append(dec.draft_block(cache, blk))
     assert torch.equal(*logits)
+
+
+@pytest.mark.parametrize("B,P", [(1, 777), (3, 211)])
+def test_prefill_at_prompt_lengths(dev, B, P):
+    """Prefills of several hundred tokens, for which the products take the tiles and K ranges of real
+    prompts (the down product runs in K ranges), against the oracle; then a draft block over the cache."""
+    cfg = Cfg(4096, 1024, 4096, 2, 8, 2, 128, lora_rank=32, lora_alpha=64)
+    assert K.nt_plan(B * P, 1024, 4096)[1] > 1
+    params = {k: v.bfloat16().float() for k, v in init_params(cfg, seed=0).items()}
+    lora = init_lora(cfg, seed=1)
+    model = UnoQwen3ForCausalLM(UnoQwen3Config(vocab_size=4096, hidden_size=1024, intermediate_size=4096,
+                                               num_hidden_layers=2, num_attention_heads=8, num_key_value_heads=2,
+                                               head_dim=128, block_size=16), device=dev, dtype=torch.bfloat16)
+    model.load_weights(params)
+    lm, _ = create_lora_model(model, LoraSettings("all", 32, 64, 0.0))
+    lm.load_lora(lora)
+    dec = BlockDecoder(lm)
+    g = torch.Generator().manual_seed(P)
+    ids, blk = torch.randint(0, 4095, (B, P), generator=g), torch.randint(0, 4095, (B, 16), generator=g)
+    cache = dec.new_cache(B, P + 16)
+    got = torch.cat([dec.prefill(cache, ids.to(dev)), dec.draft_block(cache, blk.to(dev))], 1)
+    for b in range(B):
+        gate = torch.zeros(1, P + 16)
+        gate[0, P + 1:] = 1.0
+        ref = _oracle_logits(params, lora, cfg, torch.cat([ids[b], blk[b]])[None], gate)
+        assert _rel(got[b, :P], ref[:P]) < 2e-2 and _rel(got[b, P:], ref[P:]) < 2e-2
