@@ -1859,7 +1859,8 @@ static NtPlan nt_plan(const GemmNT& p, bool may_split) {
 // seg_end/seg_col: `nseg` (<= 4) extension segments over N (ignored when A2 is null).
 // C[M, N/2] = silu(G) * U for the gate/up product A[M,K] B[N,K]^T with 64-row interleaved B (rows
 // 128 b + [0, 64) gate, 128 b + [64, 128) up of features 64 b + [0, 64)), bf16, rounded as the
-// unfused product followed by unok_swiglu_fwd. M and N multiples of 256, K of 64.
+// unfused product followed by unok_swiglu_fwd. M a multiple of row_step, N of 256, K of 64. With plain_rows,
+// B holds the gate rows and then the up rows.
 static int swiglu_fwd_product(int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
                                     const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
                                     void* C, int64_t ldc, void* gu, int64_t ldgu, void* stream, int row_step,
@@ -1910,7 +1911,7 @@ UNOK_EXPORT int unok_gemm_nt_swiglu_any(int M, int N, int K, const void* A, int6
 // non-null), and the q/k columns before the norm in bf16 (pre_f32: fp32) into qk_pre [M, 128 (nq+nk)] (when
 // non-null). cos_tab / sin_tab [P, 64] hold cos / sin of fl32(p * inv_freq[j]) (unok_rope_table);
 // positions are clamped to [0, P). Same values as unok_gemm_nt into fp32 followed by
-// unok_qknorm_rope_fwd. M and N multiples of 256, K of 64, K2 of 32.
+// unok_qknorm_rope_fwd. M a multiple of row_step, N of 256, K of 64, K2 of 32.
 static int qkv_rope_product(int M, int K, int nq, int nk, const void* A, int64_t lda, const void* B,
                                       int64_t ldb, const void* A2, int64_t lda2, const void* B2, int64_t ldb2, int K2,
                                       int nseg, const int* seg_end, const int* seg_col, const void* wq, const void* wk,
@@ -1976,7 +1977,7 @@ UNOK_EXPORT int unok_gemm_nt_qkv_rope_any(int M, int K, int nq, int nk, const vo
 
 // dgu[M, 2F] = SwiGLU backward of dS = A[M,K] B[F,K]^T + A2[M,K2] B2[F,K2]^T (bf16, never stored)
 // against gu[M, 2F] = [gate | up]; rounded exactly as unok_gemm_nt followed by unok_swiglu_bwd.
-// M and F multiples of 256, K of 64, K2 of 32.
+// M a multiple of row_step, F of 256, K of 64, K2 of 32.
 static int swiglu_bwd_product(int M, int F, int K, const void* A, int64_t lda, const void* B,
                                         int64_t ldb, const void* A2, int64_t lda2, const void* B2, int64_t ldb2,
                                         int K2, const void* gu, int64_t ldgu, void* dgu, int64_t lddgu,

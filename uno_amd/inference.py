@@ -8,9 +8,12 @@ the block (nano_vllm_uno/layers/attention.py:628-668, BLOCK_DECODE: the block's 
 the cache first, then flash attention with causal=True over the cached lengths). After the draft
 the noise K/V are discarded: only the committed rows (the seed) advance the cache.
 
-Kernels, all shared with the training step:
-* the gated LoRA is the GEMM's K-extension: h = m (.) (x A^T) by the skinny GEMM with its row gate,
-  then y = x W^T + h (s B)^T (+ residual) in the 256x256 / register-staged MFMA GEMMs;
+Kernels:
+* the gated LoRA linears of a bf16 draft block are the few-row products (unok_gemm_nt_rows), which stream
+  each weight once past the block's rows: the LoRA A rows are extra product columns, and the reduction
+  forms h = m (.) (x A^T) and adds h (s B)^T (+ residual, or SwiGLU); a layer is one native call
+  (unok_draft_layer). Other dtypes, and more than 512 rows, run the training step's GEMMs with the LoRA
+  as their K-extension;
 * the cache is head-major, [layers][B, Hkv, max_len, D] for K and V, so one (sequence, K/V head)
   pair's keys are contiguous rows; the block's queries of that pair (L rows x the q-heads sharing
   the K/V head, at most 128) are laid out as the 128 query rows of one attention workgroup over
@@ -315,8 +318,8 @@ class BlockDecoder:
 class DraftGraph:
     """A draft block of fixed shape [B, L] over one cache, captured as a single HIP graph.
 
-    The decoder issues about twenty kernels per layer; launched one by one from Python, a block of a
-    36-layer model costs more host time than device time. Replaying the captured graph is one host
+    The decoder runs 13 kernels per layer; issued from Python, even as one call per layer, a block of few
+    rows can cost more host time than device time. Replaying the captured graph is one host
     call per block. Everything that depends on the committed lengths (the positions, the cache
     store rows, the decode query layout and the key intervals) is computed on the device from
     ``cache.lengths`` inside the graph, so each replay drafts at the current lengths and then
