@@ -242,6 +242,24 @@ def test_rows_tiles_and_short_ranges(dev, M, N, Kd, r, splits):
     assert _rel(plain, _ref(a, w)) < 4e-3
 
 
+@pytest.mark.parametrize("M", [17, 32])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_rows_wide_weight_at_few_rows(dev, M, splits):
+    """17 to 32 rows over a weight of more than 2^27 elements (an LM head's): the 128-column tile, writing C
+    itself and through K ranges."""
+    N, Kd = 33000, 4096
+    torch.manual_seed(M + splits)
+    a = torch.randn(M, Kd, device=dev).bfloat16()
+    w = (torch.randn(N, Kd, device=dev) * 0.05).bfloat16()
+    res = torch.randn(M, N, device=dev).bfloat16()
+    assert _rel(K.gemm_nt_rows(a, w, splits=splits), _ref(a, w)) < 4e-3
+    la, lb = (torch.randn(16, Kd, device=dev) * 0.05).bfloat16(), (torch.randn(N, 8, device=dev) * 0.05).bfloat16()
+    segs = [(16000, 8), (N, 0)]
+    gate = torch.rand(M, device=dev) > 0.3
+    out = K.gemm_nt_rows(a, w, lora_a=la, lora_b=lb, segments=segs, residual=res, gate=gate, splits=splits)
+    assert _rel(out, _ref(a, w, la, lb, segs, res, gate)) < 4e-3
+
+
 @pytest.mark.parametrize("B,L,nq,nk,max_len,S", [(1, 1, 4, 4, 33, 1), (3, 5, 16, 8, 70, 8), (2, 32, 4, 1, 4096, 3)])
 def test_decode_maps(dev, B, L, nq, nk, max_len, S):
     """Every key of a query's causal prefix lies in exactly one range, ranges follow each other, padding

@@ -16,7 +16,9 @@ def _rel(a, b):
     return ((a.double() - b).norm() / b.norm().clamp_min(1e-300)).item()
 
 
-@pytest.mark.parametrize("M,N,Kd", [(1, 1, 1), (33, 8, 16), (512, 256, 256), (31, 65, 37), (230, 256, 4096), (64, 96, 1028)])
+@pytest.mark.parametrize("M,N,Kd", [(1, 1, 1), (33, 8, 16), (512, 256, 256), (31, 65, 37), (230, 256, 4096), (64, 96, 1028),
+                                    # 64x64 tiles for a short K over many outputs; 32x32 ones from K = 256 there
+                                    (700, 2100, 8), (1001, 1300, 33), (1001, 1300, 256)])
 @pytest.mark.parametrize("offset", [0, 1])
 def test_nt_f32(dev, M, N, Kd, offset):
     """offset 1: operands that start 4 bytes past 16-byte alignment (element loads)."""
